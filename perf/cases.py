@@ -1,0 +1,367 @@
+"""Performance cases: the calls a program built on egg_sync makes, over the sizes it makes them at.
+
+The kinds, and what each stands for:
+
+  dropin    algorithms.EGG_SynC(D, eps) on a host tensor: the reference's own call, as its
+            experiment harness makes it (n from a few hundred to 128k, few dimensions).
+            The smallest sizes are bound by launches and host work.
+  solve     solver.solve on device data, 2 or 3 dimensions: dense grids, up to the
+            benchmark's n = 1,000,000, d = 3, eps = 0.02.
+  highd     solver.solve from 5 to 20 dimensions: sparse grids, where most cells hold one
+            point (the benchmark's d = 8 form; the widths of the real data sets).
+  batch     solver.solve_batch: several data sets of uneven size, each with several eps.
+  pass      solver.iteration: one pass of the loop with its per-point counts and flags.
+  features  learned.features: grid build and cell summaries only, bound by memory traffic.
+  sync      algorithms.SynC: the r_c stop rule and the SynC labels.
+  brute     solver.simple_solve: brute-force SynC, every point against all points.
+  train     one optimiser step of the jump network on a batch of trajectory samples.
+  infer     the jump network's prediction for every point of a data set.
+
+Inputs are drawn on the GPU from the seed: Gaussian blobs with uniform noise, min-max
+normalised, in random order, as the package's generators draw them on the host.
+"""
+import math
+import os
+import sys
+
+import numpy as np
+import torch
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+sys.path.insert(0, os.path.join(ROOT, "egg-sync_amd"))
+
+from egg_sync import algorithms, learned, solver  # noqa: E402
+
+WEIGHTS = os.path.join(ROOT, "egg-sync_amd", "egg_sync", "weights", "jump_d3.npz")
+DEV = "cuda"
+IN, HIDDEN, OUT = 12, 128, 3
+LR, STEP = 2e-3, 200
+
+
+def listed():
+    return [
+        # the small plain workload, through the drop-in call: latency
+        dict(name="dropin_2k_d2", kind="dropin", n=2000, d=2, eps=0.05, blobs=4),
+        # the harness's default point (n = 100k, d = 2, eps = 0.05)
+        dict(name="dropin_100k_d2", kind="dropin", n=100_000, d=2, eps=0.05, blobs=5),
+        # the benchmark's headline solve
+        dict(name="solve_1m_d3", kind="solve", n=1_000_000, d=3, eps=0.02, blobs=20),
+        # the benchmark's higher-dimensional solve
+        dict(name="solve_250k_d8", kind="highd", n=250_000, d=8, eps=0.1, blobs=10),
+        # a real data set's shape: some ten thousand rows, 14 columns
+        dict(name="solve_15k_d14", kind="highd", n=14_980, d=14, eps=0.2, blobs=6),
+        # a sweep: twelve data sets, two eps each, one call
+        dict(name="batch_24", kind="batch", sets=12, n_lo=1000, n_hi=50_000, eps=0.02, eps2=0.05),
+        # one pass with diagnostics, as a program that drives the loop itself runs it
+        dict(name="pass_100k_d3", kind="pass", n=100_003, d=3, eps=0.02, blobs=20),
+        # features of the benchmark-sized data set
+        dict(name="features_1m_d3", kind="features", n=1_000_000, d=3, eps=0.02, blobs=20),
+        # the reference's SynC at the harness's smaller sizes
+        dict(name="sync_8k_d2", kind="sync", n=8000, d=2, eps=0.05, blobs=5),
+        # the reference's brute-force GPU variant
+        dict(name="brute_8k_d3", kind="brute", n=8000, d=3, eps=0.05, blobs=5),
+        # the trainer's step
+        dict(name="train_8192", kind="train", batch=8192),
+        # the prediction slice of the trainer (1 << 20 rows)
+        dict(name="infer_1m", kind="infer", n=1 << 20),
+    ]
+
+
+def _log(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(["dropin", "solve", "highd", "batch", "pass", "features", "sync", "brute",
+                       "train", "infer"])
+    if kind == "dropin":
+        return dict(kind=kind, n=_log(rng, 500, 128_000), d=rng.randint(2, 4),
+                    eps=rng.choice([0.0125, 0.025, 0.05]), blobs=rng.randint(2, 16))
+    if kind == "solve":
+        return dict(kind=kind, n=_log(rng, 10_000, 500_000), d=rng.choice([2, 3]),
+                    eps=rng.choice([0.005, 0.01, 0.02]), blobs=rng.randint(5, 30))
+    if kind == "highd":
+        return dict(kind=kind, n=_log(rng, 2000, 60_000), d=rng.randint(5, 20),
+                    eps=rng.choice([0.05, 0.1, 0.2]), blobs=rng.randint(4, 16))
+    if kind == "batch":
+        return dict(kind=kind, sets=rng.randint(3, 12), n_lo=1000, n_hi=_log(rng, 5000, 50_000),
+                    eps=rng.choice([0.01, 0.02]), eps2=rng.choice([0.05, 0.1]))
+    if kind == "pass":
+        return dict(kind=kind, n=_log(rng, 2000, 150_000), d=rng.choice([2, 3, 5]),
+                    eps=rng.choice([0.01, 0.02, 0.05]), blobs=rng.randint(5, 30))
+    if kind == "features":
+        return dict(kind=kind, n=_log(rng, 10_000, 1_000_000), d=rng.choice([2, 3, 5]),
+                    eps=rng.choice([0.01, 0.02, 0.05]), blobs=rng.randint(5, 30))
+    if kind == "sync":
+        return dict(kind=kind, n=_log(rng, 1000, 16_000), d=rng.choice([2, 3]),
+                    eps=rng.choice([0.025, 0.05]), blobs=rng.randint(2, 16))
+    if kind == "brute":
+        return dict(kind=kind, n=_log(rng, 500, 12_000), d=rng.choice([2, 3, 4, 8]),
+                    eps=rng.choice([0.025, 0.05, 0.1]), blobs=rng.randint(2, 16))
+    if kind == "train":
+        return dict(kind=kind, batch=_log(rng, 256, 65_536))
+    return dict(kind=kind, n=_log(rng, 1000, 1 << 20))
+
+
+# ------------------------------------------------------------------ inputs --
+
+def _blobs(n, d, k, seed, noise, sigma_lo=0.005, sigma_hi=0.02, zipf=0.0):
+    """[n, d] float32 in [0, 1] on the GPU: k Gaussian blobs with a sigma per axis, sizes
+    equal or falling off as rank^-zipf, the rest uniform, min-max normalised."""
+    g = torch.Generator(device=DEV).manual_seed(seed * 1_000_003 + n * 31 + d)
+    u = lambda *s: torch.rand(*s, generator=g, device=DEV, dtype=torch.float64)  # noqa: E731
+    centre = 0.1 + 0.8 * u(k, d)
+    sigma = sigma_lo + (sigma_hi - sigma_lo) * u(k, d)
+    w = torch.arange(1, k + 1, device=DEV, dtype=torch.float64) ** -zipf
+    edge = torch.cumsum(w / w.sum(), 0) * (1.0 - noise)
+    which = torch.searchsorted(edge, u(n))
+    X = torch.randn(n, d, generator=g, device=DEV, dtype=torch.float64)
+    at = which.clamp(max=k - 1)
+    X = centre[at] + sigma[at] * X
+    X = torch.where((which >= k)[:, None], u(n, d), X)
+    lo, hi = X.min(0).values, X.max(0).values
+    return ((X - lo) / (hi - lo)).to(torch.float32).contiguous()
+
+
+def _points(c, seed):
+    """The data set of a case, by its kind."""
+    k = c["kind"]
+    if k in ("solve", "features", "pass"):  # the benchmark's generator: uneven blobs
+        return _blobs(c["n"], c["d"], c["blobs"], seed, 0.02, zipf=1.1)
+    if k == "highd":
+        return _blobs(c["n"], c["d"], c["blobs"], seed, 0.01, 0.03, 0.03)
+    return _blobs(c["n"], c["d"], c["blobs"], seed, 0.05, 0.03, 0.03)
+
+
+def _samples(n, seed):
+    """Rows as learned.features makes them -- position, cell mean sin and cos, last
+    displacement in units of eps -- and jump targets in units of eps."""
+    g = torch.Generator(device=DEV).manual_seed(seed * 7 + n)
+    x = torch.rand(n, 3, generator=g, device=DEV)
+    m = x + 0.004 * (torch.rand(n, 3, generator=g, device=DEV) - 0.5)
+    v = (0.3 * torch.randn(n, 3, generator=g, device=DEV)).clamp(-1, 1)
+    t = 0.7 * v + 0.3 * torch.randn(n, 3, generator=g, device=DEV)
+    return torch.cat([x, torch.sin(m), torch.cos(m), v], 1).contiguous(), t.contiguous()
+
+
+def _moments(count, seed):
+    """Adam's running moments of a network in the middle of its training."""
+    g = torch.Generator(device=DEV).manual_seed(seed * 11 + 5)
+    m = 1e-3 * torch.randn(count, generator=g, device=DEV)
+    v = 1e-5 * (0.1 + torch.rand(count, generator=g, device=DEV))
+    return m, v
+
+
+def _batch_shapes(c):
+    """(n, d, blobs) of a sweep's data sets: n log-uniform, fixed by the case."""
+    g = np.random.default_rng(c["sets"] * 1_000_003 + c["n_hi"])
+    lo, hi = math.log(c["n_lo"]), math.log(c["n_hi"])
+    return [(int(round(math.exp(g.uniform(lo, hi)))), int(g.choice([2, 3, 5, 8])),
+             int(g.integers(2, 31))) for _ in range(c["sets"])]
+
+
+def prepare(case, seed):
+    k = case["kind"]
+    if k == "train":
+        net = learned.JumpMLP.from_file(WEIGHTS)
+        m, v = _moments(net.n_params, seed)
+        net.m.copy_(m)
+        net.v.copy_(v)
+        net.step = STEP - 1
+        X, T = _samples(case["batch"], seed)
+        return dict(case=case, net=net, X=X, T=T)
+    if k == "infer":
+        return dict(case=case, net=learned.JumpMLP.from_file(WEIGHTS),
+                    X=_samples(case["n"], seed)[0])
+    if k == "batch":
+        sets = [_blobs(n, d, b, seed * 100 + j, 0.03, 0.01, 0.04)
+                for j, (n, d, b) in enumerate(_batch_shapes(case))]
+        D, specs = solver.pack_instances(sets, [[case["eps"], case["eps2"]]] * len(sets))
+        return dict(case=case, D=D, specs=specs)
+    X = _points(case, seed)
+    if k == "dropin" or k == "sync":
+        X = X.cpu()
+    state = dict(case=case, X=X)
+    if k == "features":
+        g = torch.Generator(device=DEV).manual_seed(seed + 17)
+        state["prev"] = X + 0.3 * case["eps"] * torch.randn(X.shape, generator=g, device=DEV)
+    return state
+
+
+def run(state):
+    c = state["case"]
+    k = c["kind"]
+    if k == "dropin":
+        labels, itr_times, _, _ = algorithms.EGG_SynC(state["X"], c["eps"])
+        return dict(labels=labels.to(torch.int64), passes=int(itr_times.numel()))
+    if k == "sync":
+        labels, itr_times, _, _ = algorithms.SynC(state["X"], c["eps"])
+        return dict(labels=labels, passes=int(itr_times.numel()))
+    if k == "solve" or k == "highd":
+        # max_iter bounds the rare data set that creeps for thousands of passes
+        r = solver.solve(state["X"], c["eps"], max_iter=100)
+        return dict(labels=r["labels"], X=r["X"], passes=r["stats"]["iterations"],
+                    cells=r["stats"]["n_cells"], clusters=r["stats"]["n_clusters"])
+    if k == "batch":
+        r = solver.solve_batch(state["D"], state["specs"], streams=8, max_iter=100)
+        return dict(labels=np.concatenate(r["labels"]),
+                    X=np.concatenate([x.reshape(-1) for x in r["X"]]),
+                    passes=np.array([q["iterations"] for q in r["results"]]),
+                    cells=np.array([q["n_cells"] for q in r["results"]]))
+    if k == "pass":
+        return solver.iteration(state["X"], c["eps"])
+    if k == "features":
+        return learned.features(state["X"], state["prev"], c["eps"])
+    if k == "brute":
+        r = solver.simple_solve(state["X"], c["eps"])
+        return dict(labels=r["labels"], X=r["X"], r=r["stats"]["rc"],
+                    passes=r["stats"]["iterations"])
+    if k == "train":
+        net = state["net"]
+        grad, loss = net.train_step(state["X"], state["T"], LR)
+        return dict(grad=grad, loss=loss, params=net.params, m=net.m, v=net.v)
+    return state["net"].forward(state["X"])
+
+
+def work(case):
+    k = case["kind"]
+    if k == "train":
+        b, p = case["batch"], HIDDEN * IN + HIDDEN + HIDDEN * HIDDEN + HIDDEN + OUT * HIDDEN + OUT
+        macs = IN * HIDDEN + HIDDEN * HIDDEN + HIDDEN * OUT
+        # forward, gradients by the weights, gradients by the two hidden layers
+        return dict(bytes=4 * (b * (IN + OUT) + 7 * p),
+                    flops=2 * b * (2 * macs + HIDDEN * HIDDEN + HIDDEN * OUT))
+    if k == "infer":
+        n = case["n"]
+        return dict(bytes=4 * n * (IN + OUT),
+                    flops=2 * n * (IN * HIDDEN + HIDDEN * HIDDEN + HIDDEN * OUT))
+    if k == "batch":
+        # rows in once, labels and positions out for each of the two eps
+        return dict(bytes=sum(4 * n * (d + 2 * (1 + d)) for n, d, _ in _batch_shapes(case)),
+                    flops=0)
+    n, d = case["n"], case["d"]
+    if k == "brute":  # one pass: a distance for every pair
+        return dict(bytes=4 * n * (2 * d + 1), flops=n * n * (3 * d))
+    if k == "features":
+        return dict(bytes=4 * n * (2 * d + 4 * d), flops=0)
+    if k == "pass":
+        return dict(bytes=4 * n * (2 * d + 5), flops=0)
+    return dict(bytes=4 * n * (2 * d + 1), flops=0)
+
+
+# ------------------------------------------------------ values in 64 bits --
+
+def _weights():
+    with np.load(WEIGHTS, allow_pickle=False) as z:
+        return torch.from_numpy(z["params"].astype(np.float64)).to(DEV)
+
+
+def _layers(p):
+    at, out = 0, []
+    for shape in ((HIDDEN, IN), (HIDDEN,), (HIDDEN, HIDDEN), (HIDDEN,), (OUT, HIDDEN), (OUT,)):
+        size = int(np.prod(shape))
+        out.append(p[at:at + size].view(shape))
+        at += size
+    return out
+
+
+def _network(p, X):
+    W1, b1, W2, b2, W3, b3 = _layers(p)
+    h = torch.relu(X.double() @ W1.t() + b1)
+    return torch.relu(h @ W2.t() + b2) @ W3.t() + b3
+
+
+def _cells(X, eps):
+    """The grid's side, width and every point's cell coordinates, by the solver's rule (FP32
+    division, truncated, clamped to the last cell)."""
+    d = X.shape[1]
+    e = np.float32(eps)
+    cs = np.float32(np.sqrt((float(e) / 2.0) ** 2 / d))
+    w = max(1, int(np.float32(1) / cs))
+    # by a tensor: a Python divisor would become a product with its reciprocal
+    q = X / torch.full_like(X, float(cs))
+    return cs, w, torch.trunc(q).to(torch.int64).clamp(0, w - 1)
+
+
+def _groups(cell):
+    """A number for every point's cell, and the cells."""
+    cells, at = torch.unique(cell, dim=0, return_inverse=True)
+    return cells, at
+
+
+def _exact_features(c, X, prev):
+    _, _, cell = _cells(X, c["eps"])
+    cells, at = _groups(cell)
+    x = X.double()
+    out = [x]
+    count = torch.bincount(at, minlength=len(cells)).double()
+    for f in (torch.sin, torch.cos):
+        total = torch.zeros(len(cells), x.shape[1], dtype=torch.float64, device=DEV)
+        out.append((total.index_add_(0, at, f(x)) / count[:, None])[at])
+    out.append((x - prev.double()) / float(np.float32(c["eps"])))
+    return torch.cat(out, 1)
+
+
+def _exact_pass(c, X):
+    """Every pair with the pass's own FP32 decisions (cell box wholly within eps, or partly and
+    the point within eps), the sums in 64 bits."""
+    n, d = X.shape
+    e = np.float32(c["eps"])
+    thr = np.float32(e * e)
+    while np.sqrt(thr) > e:
+        thr = np.nextafter(thr, np.float32(0))
+    while np.sqrt(np.nextafter(thr, np.float32(4))) <= e:
+        thr = np.nextafter(thr, np.float32(4))
+    thr = float(thr)
+    cs, _, cell = _cells(X, c["eps"])
+    cells, at = _groups(cell)
+    lo_face = cells.to(torch.float32) * float(cs)
+    hi_face = (cells + 1).to(torch.float32) * float(cs)
+    out = torch.empty(n, d, dtype=torch.float64, device=DEV)
+    rows = max(64, min(n, (1 << 25) // n))
+    for s in range(0, n, rows):
+        x = X[s:s + rows]
+        near = torch.zeros(x.shape[0], len(cells), device=DEV)
+        far, dist = torch.zeros_like(near), torch.zeros(x.shape[0], n, device=DEV)
+        for q in range(d):
+            a = (lo_face[None, :, q] - x[:, q, None]) ** 2
+            b = (hi_face[None, :, q] - x[:, q, None]) ** 2
+            near += torch.minimum(a, b)
+            far += torch.maximum(a, b)
+            df = x[:, q, None] - X[None, :, q]
+            dist += df * df
+        full = far <= thr
+        part = (near <= thr) & ~full
+        take = full[:, at] | (part[:, at] & (dist <= thr))
+        del a, b, df, near, far, dist, full, part
+        count = take.sum(1).double()
+        for q in range(d):
+            v = torch.sin(X[None, :, q].double() - x[:, q, None].double())
+            out[s:s + rows, q] = x[:, q].double() + (v * take).sum(1) / count
+    return out
+
+
+def exact(case, seed):
+    k = case["kind"]
+    if k == "infer":
+        return _network(_weights(), _samples(case["n"], seed)[0])
+    if k == "train":
+        X, T = _samples(case["batch"], seed)
+        p = _weights().requires_grad_(True)
+        loss = ((_network(p, X) - T.double()) ** 2).sum(1).mean()
+        loss.backward()
+        g = p.grad
+        m, v = (t.double() for t in _moments(p.numel(), seed))
+        b1, b2 = float(np.float32(0.9)), float(np.float32(0.999))
+        m, v = b1 * m + (1 - b1) * g, b2 * v + (1 - b2) * g * g
+        step = float(np.float32(LR)) * (m / (1 - b1 ** STEP)) / ((v / (1 - b2 ** STEP)).sqrt() + 1e-8)
+        return dict(grad=g, loss=float(loss), params=p.detach() - step, m=m, v=v)
+    if k == "features":
+        s = prepare(case, seed)
+        return _exact_features(case, s["X"], s["prev"])
+    if k == "pass":
+        # the counts, flags and the order are whole numbers; they are equal or wrong
+        return dict(X_next=_exact_pass(case, _points(case, seed)))
+    # A whole solve repeats FP32 decisions on its own rounded positions until nothing moves: its
+    # labels and final positions are a property of that sequence and have no value in 64 bits.
+    return None
