@@ -99,7 +99,8 @@ def draw(rng):
         return dict(kind=kind, n=_log(rng, 500, 12_000), d=rng.choice([2, 3, 4, 8]),
                     eps=rng.choice([0.025, 0.05, 0.1]), blobs=rng.randint(2, 16))
     if kind == "train":
-        return dict(kind=kind, batch=_log(rng, 256, 65_536))
+        # 32,768 rows is the largest batch whose layers fit the step's 4M-float workspace
+        return dict(kind=kind, batch=_log(rng, 256, 32_768))
     return dict(kind=kind, n=_log(rng, 1000, 1 << 20))
 
 
