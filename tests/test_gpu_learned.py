@@ -127,3 +127,40 @@ def test_learned_solve_verify_falls_back_only_on_disagreement(L, net):
     z = L.solve_learned(X, eps, net, t0=1, alpha=0.0, verify=True)
     assert z["same_partition"] and not z["fallback"]
     assert np.array_equal(z["labels"], L.solve_learned(X, eps, net, t0=1, alpha=0.0)["labels"])
+
+
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 127, 129, 65_537])
+def test_forward_at_tile_edges(L, n):
+    """Remainders of the 32-point MFMA tiles and of a workgroup's four.  Bound: every product and
+    sum of the three layers rounds once, at most 12 + 128 + 128 deep and six of them for the
+    biases and the halves, so the error is within 280 * 2^-24 of the same network on absolute
+    values (no ReLU: it only shrinks them)."""
+    import mlp_oracle as M
+    _say("forward", n)
+    net = L.JumpMLP(3, seed=3)
+    F, _ = _rand_batch(np.random.default_rng(n), n)
+    got = net.forward(F).cpu().numpy()
+    X = F.cpu().numpy().astype(np.float64)
+    ref, _ = M.forward(net.state(), X, 12, 128, 3)
+    q = {k: np.abs(v) for k, v in M.unpack(net.state(), 12, 128, 3).items()}
+    mag = (((np.abs(X) @ q["W1"].T + q["b1"]) @ q["W2"].T + q["b2"]) @ q["W3"].T + q["b3"])
+    assert (np.abs(got - ref) <= 280 * 2.0 ** -24 * mag).all()
+
+
+@pytest.mark.parametrize("B", [1, 31, 33, 257, 4097, 12_289, 33_000])
+def test_gradients_at_slice_edges(L, B):
+    """Batches at the edges of the training step's slices: 16, 32, 48 ... samples per workgroup,
+    a last workgroup of one sample, and one batch past 32,768.  Tolerances as in
+    test_gradients_match_oracle."""
+    import mlp_oracle as M
+    _say("train step", B)
+    net = L.JumpMLP(3, seed=5)
+    F, T = _rand_batch(np.random.default_rng(100 + B), B)
+    p0 = net.state()
+    g, loss = net.train_step(F, T, lr=1e-3)
+    lr, gr = M.loss_and_grad(p0, F.cpu().numpy(), T.cpu().numpy(), 12, 128, 3)
+    assert abs(loss - lr) <= 1e-5 * max(1.0, abs(lr))
+    g = g.cpu().numpy()
+    assert np.abs(g - gr).max() <= 2e-4 * np.abs(gr).max()
+    p1, _, _ = M.adam_step(p0, g.astype(np.float64), np.zeros_like(p0), np.zeros_like(p0), 1, 1e-3)
+    assert np.abs(net.state() - p1).max() <= 1e-6
