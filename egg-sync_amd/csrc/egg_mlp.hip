@@ -591,9 +591,16 @@ void gemm(const float *A, long long sam, long long sak, const float *B, long lon
           float *part, long long part_cap, hipStream_t s) {
     const int kslice = split_k(M, N, K, part_cap);
     const int S = (K + kslice - 1) / kslice;
-    dim3 grid((N + kT - 1) / kT, (M + kT - 1) / kT, S);
-    k_gemm_part<<<grid, kThreads, 0, s>>>(A, sam, sak, B, sbk, sbn, part, M, N, K, kslice);
-    k_gemm_reduce<<<blocks_for((long long)M * N), kThreads, 0, s>>>(part, S, M, N, bias, act, C, ldc);
+    // rows whose partial tiles fit `part` (all of them unless S is 1) and one grid
+    const int rows = (int)std::max<long long>(1, std::min<long long>(part_cap / N, 65535LL * kT) / kT) * kT;
+    for (int m0 = 0; m0 < M; m0 += rows) {
+        const int m = std::min(rows, M - m0);
+        dim3 grid((N + kT - 1) / kT, (m + kT - 1) / kT, S);
+        k_gemm_part<<<grid, kThreads, 0, s>>>(A + m0 * sam, sam, sak, B, sbk, sbn, part, m, N, K,
+                                              kslice);
+        k_gemm_reduce<<<blocks_for((long long)m * N), kThreads, 0, s>>>(part, S, m, N, bias, act,
+                                                                        C + m0 * ldc, ldc);
+    }
 }
 
 // The loss to the host (which waits for it) if asked for; launch errors.

@@ -164,3 +164,16 @@ def test_gradients_at_slice_edges(L, B):
     assert np.abs(g - gr).max() <= 2e-4 * np.abs(gr).max()
     p1, _, _ = M.adam_step(p0, g.astype(np.float64), np.zeros_like(p0), np.zeros_like(p0), 1, 1e-3)
     assert np.abs(net.state() - p1).max() <= 1e-6
+
+
+def test_gradients_of_a_batch_beyond_the_partial_tiles(L):
+    """A layer of 70,000 x 64 outputs does not fit the 4,194,304 floats of split-K partial tiles:
+    its rows are taken in parts.  Tolerances as in test_gradients_match_oracle."""
+    import mlp_oracle as M
+    _say("train step 8-64-64-2, 70,000 samples")
+    net = L.JumpMLP(2, hidden=64, seed=6)
+    F, T = _rand_batch(np.random.default_rng(7), 70_000, d=2)
+    g, loss = net.grad_and_loss(F, T)
+    lr, gr = M.loss_and_grad(net.state(), F.cpu().numpy(), T.cpu().numpy(), 8, 64, 2)
+    assert abs(loss - lr) <= 1e-5 * max(1.0, abs(lr))
+    assert np.abs(g.cpu().numpy() - gr).max() <= 2e-4 * np.abs(gr).max()
