@@ -104,3 +104,22 @@ def test_cap_edge_cases_and_torch_api(S):
         ref = S.simple_solve(X, eps)
         assert itr_times.shape == (ref["stats"]["iterations"],)
         assert np.array_equal(labels.cpu().numpy().astype(np.int32), ref["labels"])
+
+
+@pytest.mark.parametrize("d", [1, 3, 4, 8, 16, 17, 20])
+def test_pass_and_labels_at_tile_edges(S, O, d):
+    """Remainders of the pass's 8 or 16 targets and 64 or 128 sources and of the labels' 256, in
+    each LDS shape, from all points accepted to few: positions as in test_passes_match_oracle,
+    labels bit for bit."""
+    rng = np.random.default_rng(40 + d)
+    for n in (2, 7, 8, 15, 17, 63, 65, 127, 128, 129, 255, 257):
+        for eps in (0.2, 3.0 * np.sqrt(d)):
+            X = rng.random((n, d)).astype(f32)
+            X[n // 2] = X[0]
+            _say("pass", n, d, eps)
+            a = S.simple_solve(X, eps, lam=1.5, max_iter=1)
+            b = O.sync_solve(X, eps, lam=np.float32(1.5), max_iter=1)
+            assert np.abs(a["X"] - b["X"]).max() <= 1e-6
+            la, ka = S.simple_labels(X, eps)
+            lb, kb = O.simple_labels(X, eps)
+            assert np.array_equal(la, lb) and ka == kb
