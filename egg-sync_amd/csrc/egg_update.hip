@@ -18,6 +18,7 @@
 #include <algorithm>
 #include <cmath>
 
+#include "egg_candidates.h"
 #include "egg_internal.h"
 
 namespace egg {
@@ -112,19 +113,6 @@ __device__ __forceinline__ void walk_columns(const int *g0, int R, const Geo &g,
         }
         if (carry) break;
     }
-}
-
-// First cell of [cb, ce) whose g_od is >= lo_v (cells of a column are sorted
-// by g_od); the caller stops at the first cell above its range.
-__device__ __forceinline__ int column_lower(const int *__restrict__ cell_g_od, int cb, int ce,
-                                            int lo_v) {
-    int lo = cb, hi = ce;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (cell_g_od[mid] < lo_v) lo = mid + 1;
-        else hi = mid;
-    }
-    return lo;
 }
 
 template <int D>
@@ -1751,81 +1739,141 @@ __global__ __launch_bounds__(kBlock) void k_extra_mbr(
 }
 
 // SynC pass over the grid (SynC.cpp:16-56): every point within FP32 distance
-// eps (candidates: Chebyshev radius R+1 in all dims, which contains every such
-// point) contributes sinf(x_j - x) to the update and expf(-|x_j - x|) to r_p.
-// r_p and the block partial sums of r are FP64; the partials are combined in
-// a fixed order by k_rc_finish, so r_c is deterministic.
-constexpr int kRcBlocks = 1024;
+// eps (candidates: Chebyshev radius R+1 in the outer dimensions, which contains
+// every such point) contributes sinf(x_j - x) to the update and
+// expf(-|x_j - x|) to r_p, in ascending sorted position.
+//
+// A workgroup takes T consecutive targets, a wavefront each.  In a round every
+// wavefront tests its target's next S candidates, one per lane, packs the
+// accepted ones into LDS and evaluates their terms 64 at a time; after the
+// barrier, lanes of the first wavefronts (one per target and coordinate) and of
+// the last (r_p, in FP64) add the packed terms one after another -- the sums of
+// a scan by one thread, bit for bit -- while the next round's go to the other
+// half of the LDS.  Bound by the VALU: the terms (~45 instructions a
+// coordinate) once per 64 accepted pairs, ~40 instructions per 64 tested ones.
+// One thread per target ran the terms for every candidate any of 64 lanes
+// accepted, and 8,000 targets filled 125 of 1,024 SIMDs: n = 8,000, d = 2,
+// eps = 0.05: 3,760 us a pass, here 167.
+template <int D, bool WRITE>
+struct SyncShape {
+    static constexpr int NC = WRITE ? D + 1 : 1;             // terms per pair
+    static constexpr int T = NC <= 17 ? 16 : 8;              // targets, and wavefronts
+    static constexpr int S = NC <= 4 ? 128 : 64;             // candidates per round
+    static constexpr int kThreads = T * kWave;
+    static constexpr int kAdders = (D * T + kWave - 1) / kWave;
+    static_assert(2 * T * S * NC * 4 <= 144 * 1024, "LDS");
+    static_assert(!WRITE || kAdders < T, "the last wavefront adds r_p");
+};
 
 template <int D, bool WRITE>
-__global__ __launch_bounds__(kBlock) void k_update_sync(
+__global__ __launch_bounds__((SyncShape<D, WRITE>::kThreads))
+__attribute__((amdgpu_waves_per_eu(D <= 8 ? 8 : 4))) void k_update_sync(
     const float *__restrict__ Xs, float *__restrict__ Xout, const int *__restrict__ perm_s,
     int *__restrict__ perm_out, const int *__restrict__ point_cell,
     const int *__restrict__ cell_start, const int *__restrict__ cell_g,
-    const int *__restrict__ ob, const int *__restrict__ oe, Geo g, DevState *st,
-    double *__restrict__ rc_part) {
+    const int *__restrict__ ob, const int *__restrict__ oe, Geo g, const DevState *st,
+    double *__restrict__ ratio) {
     if (WRITE && st->done) return;
-    const int n = g.n, od = g.od, R = g.R + 1;
-    const int *cg_od = cell_g + (long long)od * n;
-    double racc = 0.0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        float x[D], sum[D];
-        int g0[D];
-        const int c0 = point_cell[i];
+    using Sh = SyncShape<D, WRITE>;
+    constexpr int T = Sh::T, S = Sh::S, NC = Sh::NC;
+    __shared__ float s_term[2][NC][T * S];
+    __shared__ int s_cnt[2][T];
+    const int n = g.n, lane = __lane_id();
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int i = blockIdx.x * T + w;  // this wavefront's target
+    float x[D];
+    Candidates<D> cand;
 #pragma unroll
-        for (int l = 0; l < D; l++) {
-            x[l] = Xs[(long long)l * n + i];
-            g0[l] = cell_g[(long long)l * n + c0];
-            sum[l] = 0.f;
-        }
-        const int g0od = select_dim<D>(g0, od);
-        int N = 0;
-        double r = 0.0;
-        Odo<D> odo;
-        odo.init(od, R);
-        while (!odo.finished) {
-            const int o = odo.outer(g0, g);
-            if (o >= 0) {
-                int cb = ob[o];
-                const int ce = oe[o];
-                if (od < D) cb = column_lower(cg_od, cb, ce, g0od - R);
-                for (int c = cb; c < ce; c++) {
-                    int gc[D];
+    for (int l = 0; l < D; l++) x[l] = Xs[(long long)l * n + min(i, n - 1)];
+    cand.init(g, cell_g, cell_start, ob, oe, point_cell[min(i, n - 1)], g.R + 1);
+    // the adding lanes' target and coordinate; the last wavefront adds r_p
+    const int at = lane % T, ac = w * (kWave / T) + lane / T;
+    const bool adds = WRITE && w < Sh::kAdders && ac < D, adds_r = w == T - 1 && lane < T;
+    float sum = 0.f;
+    double r = 0.0;
+    int N = 0;
+    bool left = i < n;
+    for (int k = 0;; k++) {
+        int cnt = 0;
+        if (left) {
+            float(*term)[T * S] = s_term[k & 1];
+            for (int step = 0; step < S / kWave; step++) {
+                left = cand.more();
+                if (!left) break;
+                const int f = cand.f0 + lane;
+                const bool in_range = f < cand.total;
+                const int j = cand.point(min(f, cand.total - 1));
+                cand.f0 += kWave;
+                float df[D], s = 0.f;
 #pragma unroll
-                    for (int l = 0; l < D; l++) gc[l] = cell_g[(long long)l * n + c];
-                    if (od < D && select_dim<D>(gc, od) > g0od + R) break;
-                    bool skip = false;
+                for (int l = 0; l < D; l++) {
+                    df[l] = Xs[(long long)l * n + j] - x[l];
+                    s += df[l] * df[l];
+                }
+                const bool in = in_range && s <= g.thr_eps;
+                const unsigned long long m = __ballot(in);
+                if (in) {
+                    const int e = w * S + cnt + __popcll(m & lanemask_lt());
+                    if (WRITE) {
 #pragma unroll
-                    for (int l = 0; l < D; l++)
-                        if (l > od && (gc[l] - g0[l] > R || g0[l] - gc[l] > R)) skip = true;
-                    if (skip) continue;
-                    for (int j = cell_start[c]; j < cell_start[c + 1]; j++) {
-                        float xq[D];
-                        const float s = dist2_to<D>(x, Xs, n, j, xq);
-                        if (s <= g.thr_eps) {
-                            if (WRITE) {
-#pragma unroll
-                                for (int l = 0; l < D; l++) sum[l] += sinf(xq[l] - x[l]);
-                            }
-                            N++;
-                            r += (double)expf(-fabsf(sqrtf(s)));
-                        }
+                        for (int l = 0; l < D; l++) term[l][e] = df[l];
                     }
+                    term[NC - 1][e] = s;
+                }
+                cnt += __popcll(m);
+            }
+            wave_sync();
+            for (int q = lane; q < cnt; q += kWave) {
+                const int e = w * S + q;
+                if (WRITE) {
+#pragma unroll
+                    for (int l = 0; l < D; l++) term[l][e] = sinf(term[l][e]);
+                }
+                term[NC - 1][e] = expf(-fabsf(sqrtf(term[NC - 1][e])));
+            }
+        }
+        if (lane == 0) s_cnt[k & 1][w] = cnt;
+        if (k > 0 && (adds || adds_r)) {
+            const int b = (k - 1) & 1, c = s_cnt[b][at];
+            const float *t = s_term[b][adds ? ac : NC - 1] + at * S;
+            N += c;
+            for (int q0 = 0; q0 < c; q0 += 8) {
+                float v[8];
+#pragma unroll
+                for (int q = 0; q < 8; q++) v[q] = t[q0 + q];  // S is a multiple of 8
+                if (adds) {
+#pragma unroll
+                    for (int q = 0; q < 8; q++)
+                        if (q0 + q < c) sum += v[q];
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 8; q++)
+                        if (q0 + q < c) r += (double)v[q];
                 }
             }
-            odo.next(od, R);
         }
-        if (WRITE) {
-#pragma unroll
-            for (int l = 0; l < D; l++) {
-                const float t = sum[l] / (float)N;
-                Xout[(long long)l * n + i] = x[l] + t;
-            }
-            perm_out[i] = perm_s[i];
-        }
-        racc += N > 0 ? r / (double)N : 1.0;
+        // one more round than the longest candidate list, to add its last terms
+        if (!__syncthreads_or(left || cnt > 0)) break;
     }
-    // deterministic block reduction
+    const int ia = blockIdx.x * T + at;
+    if (adds && ia < n) Xout[(long long)ac * n + ia] = Xs[(long long)ac * n + ia] + sum / (float)N;
+    if (adds_r && ia < n) {
+        ratio[ia] = N > 0 ? r / (double)N : 1.0;
+        if (WRITE) perm_out[ia] = perm_s[ia];
+    }
+}
+
+// Block partial sums of the points' r_p / N, combined in a fixed order by
+// k_rc_finish, so r_c is deterministic.
+constexpr int kRcBlocks = 1024;
+
+__global__ __launch_bounds__(kBlock) void k_rc_sum(const double *__restrict__ ratio, int n,
+                                                   const DevState *st, bool guard,
+                                                   double *__restrict__ rc_part) {
+    if (guard && st->done) return;
+    double racc = 0.0;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+        racc += ratio[i];
     __shared__ double s_r[kBlock / kWave];
 #pragma unroll
     for (int o = kWave / 2; o > 0; o >>= 1) racc += __shfl_xor(racc, o, kWave);
@@ -1977,21 +2025,22 @@ int rc_partials(int n) { return kRcBlocks; }
 
 void launch_update_sync(const Geo &g, GridBufs &b, DevState *st, double *rc_part, bool write_pos,
                         hipStream_t s) {
-#define SY_CASE(DD)                                                                          \
-    case DD:                                                                                 \
-        if (write_pos)                                                                       \
-            k_update_sync<DD, true><<<kRcBlocks, kBlock, 0, s>>>(                            \
-                b.Xs, b.X, b.perm_s, b.perm, b.point_cell, b.cell_start, b.cell_g, b.ob,     \
-                b.oe, g, st, rc_part);                                                       \
-        else                                                                                 \
-            k_update_sync<DD, false><<<kRcBlocks, kBlock, 0, s>>>(                           \
-                b.Xs, nullptr, b.perm_s, nullptr, b.point_cell, b.cell_start, b.cell_g,      \
-                b.ob, b.oe, g, st, rc_part);                                                 \
+    double *ratio = (double *)b.rdbg;  // [n] of its 4n ints, unused by this pass
+#define SY_LAUNCH(DD, W, X, P)                                                                    \
+    k_update_sync<DD, W><<<(g.n + SyncShape<DD, W>::T - 1) / SyncShape<DD, W>::T,                 \
+                           SyncShape<DD, W>::kThreads, 0, s>>>(                                   \
+        b.Xs, X, b.perm_s, P, b.point_cell, b.cell_start, b.cell_g, b.ob, b.oe, g, st, ratio)
+#define SY_CASE(DD)                                       \
+    case DD:                                              \
+        if (write_pos) SY_LAUNCH(DD, true, b.X, b.perm);  \
+        else SY_LAUNCH(DD, false, nullptr, nullptr);      \
         break;
     switch (g.d) {
         EGG_EACH_D(SY_CASE)
     }
 #undef SY_CASE
+#undef SY_LAUNCH
+    k_rc_sum<<<kRcBlocks, kBlock, 0, s>>>(ratio, g.n, st, write_pos, rc_part);
     k_rc_finish<<<1, kBlock, 0, s>>>(rc_part, kRcBlocks, g.n, st, write_pos);
 }
 

@@ -464,3 +464,22 @@ def test_real_harness_reads_data_files(tmp_path):
     assert [r["dataset"] for r in recs] == ["banknote", "banknote"]
     assert all(r["iterations"] == int(g["banknote_iterations"]) for r in recs)
     assert list(recs[0]["stage_times"]) == E.STAGES
+
+
+@pytest.mark.parametrize("d", [1, 3, 4, 8, 16, 17, 20])
+def test_sync_pass_at_tile_edges(S, O, d):
+    """The SynC pass and its labels at the remainders of the kernel's 8 or 16 targets and 64 or
+    128 candidates, in each LDS shape, from every pair within eps to few: positions within 1e-6
+    of the oracle's pass, r_c within 1e-7 (as above), labels the oracle's partition."""
+    from egg_sync import _native as nat
+    rng = np.random.default_rng(60 + d)
+    for n in (2, 7, 15, 17, 63, 65, 129, 300):
+        for eps in (0.2, 3.0 * np.sqrt(d)):
+            X = rng.random((n, d)).astype(np.float32)
+            X[n // 2] = X[0]
+            _say("sync pass", n, d, eps)
+            a = S.solve(X, eps, stop_rule=nat.STOP_RC, lam=1.5, max_iter=1)
+            b = O.sync_solve(X, eps, lam=np.float32(1.5), max_iter=1)
+            assert np.abs(a["X"] - b["X"]).max() <= 1e-6
+            assert abs(a["stats"]["rc"] - O.rc(X, eps)) <= 1e-7
+            assert O.same_partition(a["labels"], b["labels"])
