@@ -150,6 +150,8 @@ struct DebugOut {
 };
 void launch_update_egg(const Geo &g, GridBufs &b, DevState *st, const DebugOut *dbg,
                        hipStream_t s);
+// The groups sparse_group selects, point pair by point pair (egg_pairs.hip).
+void launch_update_pairs(const Geo &g, GridBufs &b, int *rdbg, DevState *st, hipStream_t s);
 void launch_extra_check(const Geo &g, GridBufs &b, DevState *st, hipStream_t s);
 // SynC pass: positions (write_pos) and r_c in FP64 -> st->rc.
 void launch_update_sync(const Geo &g, GridBufs &b, DevState *st, double *rc_part, bool write_pos,

@@ -20,6 +20,7 @@
 
 #include "egg_candidates.h"
 #include "egg_internal.h"
+#include "egg_wave.h"
 
 namespace egg {
 
@@ -162,14 +163,6 @@ struct SrcPt {
     float x[P], sv[P], cv[P];
 };
 
-// Makes the LDS writes of every lane visible to the reads of the others
-// (wavefront scope; the LDS serves one wavefront's accesses in order).
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Group of tile t: the largest k with tile_off[k] <= t.
 __device__ __forceinline__ int tile_group(const int *__restrict__ tile_off, int G, int t) {
     int lo = 0, hi = G - 1;
@@ -224,22 +217,6 @@ __device__ __forceinline__ bool cell_in_group_window(const int *__restrict__ cel
     }
     return in && !*stop;
 }
-
-__device__ __forceinline__ int next_tile(int *counter) {
-    int t = 0;
-    if (__lane_id() == 0) t = atomicAdd(counter, 1);
-    return __builtin_amdgcn_readfirstlane(t);
-}
-
-// Work claims of the queue kernels: wavefront w of the grid's W takes item w
-// first, without an atomic, and later items from the counter, offset by W.
-// A pass with fewer items than wavefronts (converged iterations) takes no
-// atomic at all; with more, each wavefront takes one per extra item.
-__device__ __forceinline__ int wave_index() {
-    return __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave);
-}
-
-__device__ __forceinline__ int wave_count() { return gridDim.x * (blockDim.x / kWave); }
 
 // Bitwise OR of v over the wavefront.
 __device__ __forceinline__ unsigned wave_or(unsigned v) {
@@ -1052,435 +1029,6 @@ __global__ __launch_bounds__(kBlock) void k_update_finish(
     if (__any(unsynced) && __lane_id() == 0) atomicAnd(&st->flag, 0);
 }
 
-// ---------------------------------------------------------- pair update --
-//
-// The update of the runs of the cell groups sparse_group selects (the runs
-// of sparse groups, or every run), point pair by point pair instead of cell
-// by cell.  `list` holds the target runs (nullptr: runs 0 .. count-1).  In a sparse grid (high-dimensional
-// data: 250k points in 248k cells at d = 8) the neighbour cells of a point are
-// the inner cells of (2R+1)^od outer cells, almost all holding a point or
-// none, and walking them costs far more than testing the points they hold.
-// Here every run of the grid is a source: sources come in blocks of kBlkRuns
-// consecutive runs (sorted order, so spatially compact) with bounding boxes,
-// and blocks in superblocks of kSupBlks.  One wavefront takes a tile of 64
-// target runs, prunes superblocks and blocks whose box lies farther from the
-// tile's box than any counted point can, and streams the remaining blocks
-// through LDS: the loading lane stages each source run's position, the
-// bounds of its cell's box (g cs and (g+1) cs, rounded as the reference rounds
-// them) and sin v, cos v - 1 of its offset v from the tile's anchor; every
-// lane then tests every staged run against its target.
-//
-// A pair within eps, or with a clamped source (such a point lies outside its
-// cell's box), gets the reference's cell decision for the source's cell
-// (EGG_SynC.cu:612-636): a full cell adds its totals (T_s cos x - T_c sin x,
-// EGG_SynC.cu:648-663) and its count once, when the lane meets the cell's
-// first run -- every run of a full cell is within the filter radius of the
-// target (it lies in the box, whose farthest corner is within eps, and FP32
-// rounding is monotone), so that run is always met; a partial cell adds
-// sin(x_q - x) and the length of each run within eps (EGG_SynC.cu:683-696);
-// neither -> nothing.  Only cells whose outer coordinates are within R of the
-// target's are candidates, as in the reference's neighbour list
-// (EGG_SynC.cu:368-536).  Blocks are visited in increasing order, which is
-// the reference's order of outer cells, cells and points, so the sums are
-// added in the oracle's order (runs weighted by their length); N and half are
-// exactly the reference's.
-
-// Per run: its cell, flags (bit 0: the first run of its cell, bit 1: a
-// coordinate clamped into cell w-1), position, cell coordinates and length,
-// indexed by run so that the pair update stages a block with one coalesced
-// load per field; per block of kBlkRuns runs: the bounding box of its
-// positions, whether it holds a clamped run, and its cell if all its runs
-// share one (-1 otherwise).  One wavefront per block.
-template <int D>
-__global__ __launch_bounds__(kBlock) void k_run_boxes(
-    const float *__restrict__ Xs, const int *__restrict__ run_start,
-    const int *__restrict__ point_cell, const int *__restrict__ cell_run,
-    const int *__restrict__ cell_g, Geo g, DevState *st, int *__restrict__ rcell,
-    int *__restrict__ rflag, float *__restrict__ Xr, int *__restrict__ gr,
-    int *__restrict__ rlen, float *__restrict__ bmin, float *__restrict__ bmax,
-    int *__restrict__ bclamp, int *__restrict__ bcell) {
-    if (st->done || st->sparse_count == 0) return;
-    const int n = g.n, runs = st->runs;
-    const int nblk = (runs + kBlkRuns - 1) / kBlkRuns, nb = n / kBlkRuns + 1;
-    const float wf = (float)g.w;
-    for (int b = wave_index(); b < nblk; b += wave_count()) {
-        const int r = b * kBlkRuns + __lane_id();
-        const bool on = r < runs;
-        float lo[D], hi[D];
-        int f = 0, c = -1;
-        if (on) {
-            const int i = run_start[r];
-            c = point_cell[i];
-            bool clamped = false;
-#pragma unroll
-            for (int l = 0; l < D; l++) {
-                const float x = Xs[(long long)l * n + i];
-                lo[l] = hi[l] = x;
-                clamped |= x / g.cs >= wf;  // cell_coord's clamp of w to w-1
-                Xr[(long long)l * n + r] = x;
-                gr[(long long)l * n + r] = cell_g[(long long)l * n + c];
-            }
-            f = (cell_run[c] == r ? 1 : 0) | (clamped ? 2 : 0);
-            rcell[r] = c;
-            rflag[r] = f;
-            rlen[r] = run_start[r + 1] - i;
-        } else {
-#pragma unroll
-            for (int l = 0; l < D; l++) {
-                lo[l] = __builtin_inff();
-                hi[l] = -__builtin_inff();
-            }
-        }
-        const bool any_clamp = __any((f & 2) != 0);
-        const int c_first = __builtin_amdgcn_readfirstlane(c);
-        const bool one_cell = !__any(on && c != c_first);
-#pragma unroll
-        for (int l = 0; l < D; l++) {
-            for (int o = kWave / 2; o > 0; o >>= 1) {
-                lo[l] = fminf(lo[l], __shfl_xor(lo[l], o, kWave));
-                hi[l] = fmaxf(hi[l], __shfl_xor(hi[l], o, kWave));
-            }
-            if (__lane_id() == 0) {
-                bmin[(long long)l * nb + b] = lo[l];
-                bmax[(long long)l * nb + b] = hi[l];
-            }
-        }
-        if (__lane_id() == 0) {
-            bclamp[b] = any_clamp ? 1 : 0;
-            bcell[b] = one_cell ? c_first : -1;
-        }
-    }
-}
-
-// Bounding box of every superblock of kSupBlks blocks, and whether it holds a
-// clamped run.
-template <int D>
-__global__ __launch_bounds__(kBlock) void k_super_boxes(
-    const float *__restrict__ bmin, const float *__restrict__ bmax,
-    const int *__restrict__ bclamp, Geo g, DevState *st, float *__restrict__ sbmin,
-    float *__restrict__ sbmax, int *__restrict__ sbclamp) {
-    if (st->done || st->sparse_count == 0) return;
-    const int n = g.n, runs = st->runs;
-    const int nblk = (runs + kBlkRuns - 1) / kBlkRuns, nb = n / kBlkRuns + 1;
-    const int nsup = (nblk + kSupBlks - 1) / kSupBlks, ns = n / (kBlkRuns * kSupBlks) + 1;
-    for (int sb = wave_index(); sb < nsup; sb += wave_count()) {
-        const int b = sb * kSupBlks + __lane_id();
-        const bool on = b < nblk;
-        const bool any_clamp = __any(on && bclamp[b] != 0);
-#pragma unroll
-        for (int l = 0; l < D; l++) {
-            float lo = on ? bmin[(long long)l * nb + b] : __builtin_inff();
-            float hi = on ? bmax[(long long)l * nb + b] : -__builtin_inff();
-            for (int o = kWave / 2; o > 0; o >>= 1) {
-                lo = fminf(lo, __shfl_xor(lo, o, kWave));
-                hi = fmaxf(hi, __shfl_xor(hi, o, kWave));
-            }
-            if (__lane_id() == 0) {
-                sbmin[(long long)l * ns + sb] = lo;
-                sbmax[(long long)l * ns + sb] = hi;
-            }
-        }
-        if (__lane_id() == 0) sbclamp[sb] = any_clamp ? 1 : 0;
-    }
-}
-
-// Whether box k of a (lo, hi) table ([D][stride]) lies within squared
-// distance thr of the box [alo, ahi] (thr_clamp if the box holds a clamped
-// run).  Box distances round like the point distances they bound; the
-// caller's thresholds carry a relative margin of 2^-10 for that.
-template <int D>
-__device__ __forceinline__ bool box_near(const float (&alo)[D], const float (&ahi)[D],
-                                         const float *__restrict__ blo,
-                                         const float *__restrict__ bhi, long long stride, int k,
-                                         float thr) {
-    float s = 0.f;
-#pragma unroll
-    for (int l = 0; l < D; l++) {
-        const float gap = fmaxf(0.f, fmaxf(blo[l * stride + k] - ahi[l], alo[l] - bhi[l * stride + k]));
-        s += gap * gap;
-    }
-    return s <= thr;
-}
-
-// Source runs of a block staged in LDS for the pair update.  Positions are
-// kept twice: row-major for the distance tests, where every lane reads the
-// same run (broadcast, 16-byte loads), and with the cell box bounds, cell
-// coordinates, length, flags and cell in columns for the accepted pairs,
-// where each lane reads a run of its own (consecutive runs in consecutive
-// banks).
-template <int D>
-struct PairStage {
-    static constexpr int P = (D + 3) / 4 * 4;
-    float xr[kBlkRuns][P];
-    float x[D][kBlkRuns], lo[D][kBlkRuns], hi[D][kBlkRuns];
-    int g[D][kBlkRuns];
-    int len[kBlkRuns], flag[kBlkRuns], cell[kBlkRuns];
-};
-
-// sin v: the polynomial of sin_small for |v| <= 1 when the caller knows that
-// bound holds (SMALL), else sinf.
-template <bool SMALL>
-__device__ __forceinline__ float sin_pair(float v) {
-    if (!SMALL) return sinf(v);
-    const float v2 = v * v;
-    float ps = -2.50521083854417e-08f;
-    ps = fmaf(ps, v2, 2.75573192239859e-06f);
-    ps = fmaf(ps, v2, -1.98412698412698e-04f);
-    ps = fmaf(ps, v2, 8.33333333333333e-03f);
-    ps = fmaf(ps, v2, -1.66666666666667e-01f);
-    return fmaf(v * v2, ps, v);
-}
-
-// SMALL: every pair the filter passes is closer than 1 in each coordinate
-// (filter radius below 1), so sin(x_q - x) takes the polynomial.
-template <int D, bool SMALL>
-__global__ __launch_bounds__(kBlock) void k_update_pairs(
-    const float *__restrict__ Xs, const int *__restrict__ cell_start,
-    const int *__restrict__ cell_g, const float *__restrict__ Ts, const float *__restrict__ Tc,
-    const int *__restrict__ run_start, const int *__restrict__ point_cell,
-    const int *__restrict__ cell_run, const int *__restrict__ list,
-    const int *__restrict__ rcell, const int *__restrict__ rflag,
-    const float *__restrict__ Xr, const int *__restrict__ gr, const int *__restrict__ rlen,
-    const float *__restrict__ bmin, const float *__restrict__ bmax,
-    const int *__restrict__ bclamp, const int *__restrict__ bcell,
-    const float *__restrict__ sbmin,
-    const float *__restrict__ sbmax, const int *__restrict__ sbclamp, float thr_filter,
-    float thr_clamp, float *__restrict__ rres, int *__restrict__ rdbg, Geo g, DevState *st) {
-    if (st->done) return;
-    const int count = st->sparse_count;
-    if (count == 0) return;
-    __shared__ PairStage<D> s_stage[kBlock / kWave];
-    PairStage<D> &S = s_stage[threadIdx.x / kWave];
-    const int n = g.n, od = g.od, R = g.R, runs = st->runs, lane = __lane_id();
-    const int nblk = (runs + kBlkRuns - 1) / kBlkRuns, nb = n / kBlkRuns + 1;
-    const int nsup = (nblk + kSupBlks - 1) / kSupBlks, ns = n / (kBlkRuns * kSupBlks) + 1;
-    const float thr = g.thr_eps, thr_half = g.thr_half;
-    const float box_thr = thr_filter * (1.0f + 0x1p-10f);
-    const float box_thr_clamp = thr_clamp * (1.0f + 0x1p-10f);
-    const int ntiles = (count + kWave - 1) / kWave;
-    bool unsynced = false;
-    for (int t = wave_index(); t < ntiles; t = wave_count() + next_tile(&st->ptile_next)) {
-        const int k = t * kWave + lane;
-        const bool active = k < count;
-        const int r = list ? list[active ? k : t * kWave] : (active ? k : t * kWave);
-        const int i = run_start[r];
-        const int c0 = point_cell[i];
-        const int own = cell_start[c0 + 1] - cell_start[c0];
-        float x[D], sum[D], sml[D], tlo[D], thi[D];
-        int g0[D];
-        bool border = false;
-#pragma unroll
-        for (int l = 0; l < D; l++) {
-            x[l] = Xs[(long long)l * n + i];
-            g0[l] = l < od ? cell_g[(long long)l * n + c0] : 0;
-            sum[l] = 0.f;
-            sml[l] = 0.f;
-            border |= on_border(x[l], g.cs);
-            tlo[l] = active ? x[l] : __builtin_inff();
-            thi[l] = active ? x[l] : -__builtin_inff();
-            for (int o = kWave / 2; o > 0; o >>= 1) {
-                tlo[l] = fminf(tlo[l], __shfl_xor(tlo[l], o, kWave));
-                thi[l] = fmaxf(thi[l], __shfl_xor(thi[l], o, kWave));
-            }
-        }
-        int N = 0, half = 0;
-        // the lane's decision for the last cell it classified: a cell's runs
-        // are consecutive in block order, so one box test serves all of them
-        int last_c = -1, last_cls = 0;  // 0 not counted, 1 full, 2 partial
-        for (int sb0 = 0; sb0 < nsup; sb0 += kWave) {
-            const int sbl = sb0 + lane;
-            const bool sp = sbl < nsup &&
-                            box_near<D>(tlo, thi, sbmin, sbmax, ns, sbl,
-                                        sbclamp[sbl] ? box_thr_clamp : box_thr);
-            for (unsigned long long ms = __ballot(sp); ms; ms &= ms - 1) {
-                const int sb = sb0 + __ffsll((long long)ms) - 1;
-                const int bl = sb * kSupBlks + lane;
-                const bool bp = bl < nblk &&
-                                box_near<D>(tlo, thi, bmin, bmax, nb, bl,
-                                            bclamp[bl] ? box_thr_clamp : box_thr);
-                for (unsigned long long mb = __ballot(bp); mb; mb &= mb - 1) {
-                    const int b = sb * kSupBlks + __ffsll((long long)mb) - 1;
-                    const int r0 = b * kBlkRuns;
-                    // a block whose runs share one cell c (a dense cell): one
-                    // box test of c per lane decides for all its runs, unless
-                    // c is partial for the lane or a border lane needs its
-                    // eps/2 count; if no lane needs the runs one by one, the
-                    // block is not streamed, and lanes for which c is full add
-                    // its totals in the block holding its first run
-                    const int bc = bcell[b];
-                    if (bc >= 0 && !bclamp[b]) {
-                        bool need = false, add_full = false;
-                        if (active) {
-                            int gc[D];
-                            bool win = true;
-#pragma unroll
-                            for (int l = 0; l < D; l++) {
-                                gc[l] = gr[(long long)l * n + r0];
-                                if (l < od && (gc[l] - g0[l] > R || g0[l] - gc[l] > R)) win = false;
-                            }
-                            if (win) {
-                                float sm, lg;
-                                box_dist<D>(gc, x, g.cs, sm, lg);
-                                const bool full = lg <= thr;
-                                need = (!full && sm <= thr) || (full && border && bc != c0);
-                                add_full = full;
-                            }
-                        }
-                        if (!__any(need)) {
-                            const int fr = cell_run[bc];
-                            if (add_full && fr >= r0 && fr < r0 + kBlkRuns) {
-                                const int cnt = cell_start[bc + 1] - cell_start[bc];
-#pragma unroll
-                                for (int l = 0; l < D; l++) {
-                                    const float a = Ts[(long long)l * n + bc] * cosf(x[l]);
-                                    const float bb = Tc[(long long)l * n + bc] * sinf(x[l]);
-                                    const float tt = a - bb;
-                                    sum[l] += tt;
-                                }
-                                N += cnt;
-                                if (border && bc == c0) half += cnt;
-                            }
-                            continue;
-                        }
-                    }
-                    const int rr = r0 + lane;
-                    if (rr < runs) {
-                        S.len[lane] = rlen[rr];
-                        S.flag[lane] = rflag[rr];
-                        S.cell[lane] = rcell[rr];
-#pragma unroll
-                        for (int l = 0; l < D; l++) {
-                            const int gl = gr[(long long)l * n + rr];
-                            const float xq = Xr[(long long)l * n + rr];
-                            S.xr[lane][l] = xq;
-                            S.x[l][lane] = xq;
-                            S.g[l][lane] = gl;
-                            S.lo[l][lane] = (float)gl * g.cs;
-                            S.hi[l][lane] = (float)(gl + 1) * g.cs;
-                        }
-                    }
-                    wave_sync();
-                    const int m = min(kBlkRuns, runs - b * kBlkRuns);
-                    // the staged runs this lane must look at: within the
-                    // filter radius, or clamped and within the wider one
-                    unsigned long long acc = 0;
-                    if (active) {
-                        for (int q = 0; q < m; q++) {
-                            float s = 0.f;
-#pragma unroll
-                            for (int l = 0; l < D; l++) {
-                                const float df = x[l] - S.xr[q][l];
-                                s += df * df;
-                            }
-                            const bool take = s <= thr_filter ||
-                                              ((S.flag[q] & 2) && s <= thr_clamp);
-                            acc |= take ? (1ull << q) : 0ull;
-                        }
-                    }
-                    // each lane walks its own accepted runs, lowest first (the
-                    // block's order, hence the oracle's)
-                    while (__any(acc != 0)) {
-                        if (acc) {
-                            const int q = __ffsll((long long)acc) - 1;
-                            acc &= acc - 1;
-                            const int c = S.cell[q];
-                            if (c != last_c) {
-                                // the box test of the source's cell, EGG_SynC.cu:612-634,
-                                // for a cell of the reference's neighbour list
-                                bool win = true;
-#pragma unroll
-                                for (int l = 0; l < D; l++) {
-                                    if (l < od) {
-                                        const int gq = S.g[l][q];
-                                        if (gq - g0[l] > R || g0[l] - gq > R) win = false;
-                                    }
-                                }
-                                float sm = 0.f, lg = 0.f;
-#pragma unroll
-                                for (int l = 0; l < D; l++) {
-                                    float lo = S.lo[l][q] - x[l];
-                                    float hi = S.hi[l][q] - x[l];
-                                    lo *= lo;
-                                    hi *= hi;
-                                    if (lo < hi) {
-                                        sm += lo;
-                                        lg += hi;
-                                    } else {
-                                        sm += hi;
-                                        lg += lo;
-                                    }
-                                }
-                                last_c = c;
-                                last_cls = !win ? 0 : (lg <= thr ? 1 : (sm <= thr ? 2 : 0));
-                            }
-                            if (last_cls == 1) {
-                                // full: totals and count once, at the cell's first run
-                                if (S.flag[q] & 1) {
-                                    const int cnt = cell_start[c + 1] - cell_start[c];
-#pragma unroll
-                                    for (int l = 0; l < D; l++) {
-                                        const float a = Ts[(long long)l * n + c] * cosf(x[l]);
-                                        const float bb = Tc[(long long)l * n + c] * sinf(x[l]);
-                                        const float tt = a - bb;
-                                        sum[l] += tt;
-                                    }
-                                    N += cnt;
-                                    if (border && c == c0) half += cnt;
-                                }
-                                if (border && c != c0) {
-                                    float s = 0.f;
-#pragma unroll
-                                    for (int l = 0; l < D; l++) {
-                                        const float df = x[l] - S.x[l][q];
-                                        s += df * df;
-                                    }
-                                    if (s <= thr_half) half += S.len[q];
-                                }
-                            } else if (last_cls == 2) {
-                                float s = 0.f;
-#pragma unroll
-                                for (int l = 0; l < D; l++) {
-                                    const float df = x[l] - S.x[l][q];
-                                    s += df * df;
-                                }
-                                if (s <= thr) {
-                                    const int lq = S.len[q];
-                                    const float w = (float)lq;  // exact: lq < 2^24
-#pragma unroll
-                                    for (int l = 0; l < D; l++)
-                                        sml[l] += w * sin_pair<SMALL>(S.x[l][q] - x[l]);
-                                    N += lq;
-                                }
-                            }
-                        }
-                    }
-                    wave_sync();
-                }
-            }
-        }
-        if (active) {
-            float xo[D];
-#pragma unroll
-            for (int l = 0; l < D; l++) {
-                float tt = sum[l] + sml[l];
-                tt = tt / (float)N;
-                xo[l] = x[l] + tt;
-            }
-            const bool synced = !((!border && N != own) || (border && N != half));
-#pragma unroll
-            for (int l = 0; l < D; l++) rres[(long long)l * n + r] = xo[l];
-            if (!synced) unsynced = true;
-            if (rdbg) {
-                rdbg[4 * (long long)r + 0] = N;
-                rdbg[4 * (long long)r + 1] = half;
-                rdbg[4 * (long long)r + 2] = border ? 1 : 0;
-                rdbg[4 * (long long)r + 3] = synced ? 1 : 0;
-            }
-        }
-    }
-    if (__any(unsynced) && lane == 0) atomicAnd(&st->flag, 0);
-}
-
 // Every point takes its run's result and carries its id over to the next
 // iteration's order.  The run of sorted position i is rpos[i] + rhead[i] - 1.
 template <int D>
@@ -1920,9 +1468,6 @@ static inline int grid_for(long long n) {
     return (int)b;
 }
 
-// Enough workgroups to fill the chip; they drain the tile queue and exit.
-constexpr int kQueueBlocks = 2048;
-
 static inline int queue_threads(const Geo &g) {
     return g.qthreads >= kWave && g.qthreads <= kBlock && g.qthreads % kWave == 0 ? g.qthreads
                                                                                  : kBlock;
@@ -1935,37 +1480,10 @@ static inline int queue_blocks(const Geo &g) {
     return (int)std::max<long long>(1, std::min<long long>(cap, (tiles_max + waves - 1) / waves));
 }
 
-// Filter radii of the pair update: pairs within eps, with a relative margin of
-// 2^-12 for points that cell_coord's FP32 division puts one ulp outside their
-// cell's box; for sources with a clamped coordinate (they lie up to 1 - w cs
-// outside the box of cell w-1 in each such dimension), eps + sqrt(d)(1 - w cs).
-static void pair_filters(const Geo &g, float &thr_filter, float &thr_clamp) {
-    thr_filter = g.thr_eps * (1.0f + 0x1p-12f);
-    const double gap = std::max(0.0, 1.0 - (double)g.w * (double)g.cs);
-    const double r = (double)g.eps + std::sqrt((double)g.d) * gap;
-    thr_clamp = std::max(thr_filter, (float)(r * r * (1.0 + 0x1p-10)));
-}
-
 void launch_update_egg(const Geo &g, GridBufs &b, DevState *st, const DebugOut *dbg,
                        hipStream_t s) {
     DebugOut d = dbg ? *dbg : DebugOut{nullptr, nullptr, nullptr, nullptr};
     const int qb = queue_blocks(g), qt = queue_threads(g);
-    const long long nblk_max = g.n / kBlkRuns + 1;
-    const int waves_per_block = kBlock / kWave;
-    const int pb = (int)std::min<long long>(16384, (nblk_max + waves_per_block - 1) / waves_per_block);
-    const int sb = (int)std::max<long long>(
-        1, std::min<long long>(1024, (nblk_max / kSupBlks + waves_per_block) / waves_per_block));
-    const int pq = (int)std::max<long long>(
-        1, std::min<long long>(kQueueBlocks, (nblk_max + waves_per_block - 1) / waves_per_block));
-    float thr_filter, thr_clamp;
-    pair_filters(g, thr_filter, thr_clamp);
-    // every filtered pair is closer than 1 in each coordinate
-    const bool pair_small = thr_clamp < 1.0f;
-#define PAIR_ARGS                                                                               \
-    b.Xs, b.cell_start, b.cell_g, b.Ts, b.Tc, b.run_start, b.point_cell, b.cell_run,            \
-        g.pair_mode == kPairAll ? nullptr : b.sparse_runs, b.rcell, b.rflag, b.Xr, b.gr,        \
-        b.rlen, b.bmin, b.bmax, b.bclamp, b.bcell, b.sbmin, b.sbmax, b.sbclamp, thr_filter,     \
-        thr_clamp, b.rres, rdbg, g, st
     int *rdbg = (d.N || d.half || d.border || d.synced) ? b.rdbg : nullptr;
 #define UPD_CASE(DD)                                                                          \
     case DD:                                                                                  \
@@ -1985,15 +1503,7 @@ void launch_update_egg(const Geo &g, GridBufs &b, DevState *st, const DebugOut *
                                                   b.utile_off, b.dtiles, b.rdbg, b.hacc,      \
                                                   b.rres, rdbg, g, st);                       \
         }                                                                                     \
-        k_run_boxes<DD><<<pb, kBlock, 0, s>>>(b.Xs, b.run_start, b.point_cell, b.cell_run,     \
-                                              b.cell_g, g, st, b.rcell, b.rflag, b.Xr, b.gr,  \
-                                              b.rlen, b.bmin, b.bmax, b.bclamp, b.bcell);     \
-        k_super_boxes<DD><<<sb, kBlock, 0, s>>>(b.bmin, b.bmax, b.bclamp, g, st, b.sbmin,     \
-                                                b.sbmax, b.sbclamp);                          \
-        if (pair_small)                                                                       \
-            k_update_pairs<DD, true><<<pq, kBlock, 0, s>>>(PAIR_ARGS);                        \
-        else                                                                                  \
-            k_update_pairs<DD, false><<<pq, kBlock, 0, s>>>(PAIR_ARGS);                       \
+        launch_update_pairs(g, b, rdbg, st, s);                                               \
         k_scatter_runs<DD><<<grid_for(g.n), kBlock, 0, s>>>(b.rhead, b.rpos, b.rres, rdbg,   \
                                                             b.perm_s, b.X, b.perm, g.n, st,   \
                                                             d);                               \
@@ -2002,7 +1512,6 @@ void launch_update_egg(const Geo &g, GridBufs &b, DevState *st, const DebugOut *
         EGG_EACH_D(UPD_CASE)
     }
 #undef UPD_CASE
-#undef PAIR_ARGS
 }
 
 void launch_extra_check(const Geo &g, GridBufs &b, DevState *st, hipStream_t s) {
