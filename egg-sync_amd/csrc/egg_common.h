@@ -37,7 +37,7 @@ constexpr int kHeavyRuns = 4096;  // a streamed range of at least this many runs
 constexpr int kUnitRuns = 1024;   // split into units of this many runs, any wavefront's work,
 constexpr int kHeavyCap = 65536;  // with up to this many ranges per pass in the queue,
 constexpr int kHeavyMaxD = 5;     // for d up to this (per-run fixed-point sums: (2d+2)*8 B)
-constexpr int kBlkRuns = 64;      // runs per source block of the pair update
+constexpr int kBlkRuns = 16;      // runs per source block of the pair update
 constexpr int kSupBlks = 64;      // source blocks per superblock
 
 // Expands X(D) for every dimension count the kernels are instantiated for;

@@ -105,20 +105,10 @@ struct GridBufs {
     int *untile, *utile_off;// [n] the same for the groups of k_update_tile (not sparse)
     float *rres;         // [d][n] new position of each run
     int *sparse_runs;    // [n]   runs of sparse cell groups
-    // pair update (k_update_pairs): per run its cell, flags (bit 0: first
-    // run of its cell, bit 1: a coordinate clamped into cell w-1), position,
-    // cell coordinates and length; bounding boxes of blocks of kBlkRuns
-    // consecutive runs and of superblocks of kSupBlks blocks, whether they
-    // hold a clamped run, and the cell of a block whose runs share one (-1
-    // otherwise)
-    int *rcell, *rflag;  // [n]
-    float *Xr;           // [d][n]
-    int *gr;             // [d][n]
-    int *rlen;           // [n]
-    float *bmin, *bmax;  // [d][n / kBlkRuns + 1]
-    int *bclamp, *bcell; // [n / kBlkRuns + 1]
-    float *sbmin, *sbmax;// [d][n / (kBlkRuns * kSupBlks) + 1]
-    int *sbclamp;        // [n / (kBlkRuns * kSupBlks) + 1]
+    // pair update (egg_pairs.hip): memory of its own (pair_scratch_bytes); it
+    // also uses keys_a / keys_b and partial, free between the summaries and the
+    // next grid build
+    char *pair;
     int *sparse_off;     // [n]   their offsets per group (exclusive scan)
     int *rdbg;           // [4n]  N / half / border / synced of each run (diagnostics;
                          //       also the saved N / half / border of deferred runs)
@@ -151,6 +141,7 @@ struct DebugOut {
 void launch_update_egg(const Geo &g, GridBufs &b, DevState *st, const DebugOut *dbg,
                        hipStream_t s);
 // The groups sparse_group selects, point pair by point pair (egg_pairs.hip).
+size_t pair_scratch_bytes(size_t n, size_t d);
 void launch_update_pairs(const Geo &g, GridBufs &b, int *rdbg, DevState *st, hipStream_t s);
 void launch_extra_check(const Geo &g, GridBufs &b, DevState *st, hipStream_t s);
 // SynC pass: positions (write_pos) and r_c in FP64 -> st->rc.

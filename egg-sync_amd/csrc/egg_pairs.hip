@@ -10,7 +10,7 @@
 // order, so spatially compact) with bounding boxes, and blocks in superblocks
 // of kSupBlks.  A wavefront takes a tile of 16 target runs, prunes superblocks
 // and blocks whose box lies farther from the tile's box than any counted point
-// can, and takes the remaining blocks one after another (k_update_pairs).
+// can, and takes the remaining blocks eight at a time (k_update_pairs).
 //
 // A pair within eps, or with a clamped source (such a point lies outside its
 // cell's box), gets the reference's cell decision for the source's cell
@@ -34,31 +34,83 @@
 
 namespace egg {
 
-// Per run: its cell, flags (bit 0: the first run of its cell, bit 1: a
-// coordinate clamped into cell w-1), position, cell coordinates and length,
-// indexed by run so that the pair update stages a block with one coalesced
-// load per field; per cell (at its first run): its sin and cos totals as one
-// row; per block of kBlkRuns runs: the bounding box of its positions, whether
-// it holds a clamped run, and its cell if all its runs share one (-1
-// otherwise).  One wavefront per block.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// What the pair update reads, by run so that a batch of sources is a few
+// coalesced 16-byte loads, and where it lies.
+//   rows    [NC][n][4]  position, then the centre of the run's cell: 2d floats
+//                       in NC = ceil(2d / 4) chunks
+//   meta    [n]         cell, flags (bit 0: first run of its cell, bit 1: a
+//                       coordinate clamped into cell w-1), length, points of the
+//                       cell (first runs)
+//   totals  [n][2d]     sin and cos totals of a cell
+//   blo/bhi [d][nb]     bounding boxes of blocks, bflag [nb] whether a block holds
+//                       a clamped run, bcell [nb] its cell if its runs share one
+//                       (-1 otherwise); slo/shi/sflag the same of superblocks
+struct PairData {
+    f32x4 *rows;
+    int4 *meta;
+    float *totals, *blo, *bhi, *slo, *shi;
+    int *bflag, *bcell, *sflag;
+    int nb, ns;  // strides of the box tables
+};
+
+// rows take the summaries' partials (16 d bytes a point of at most 16 NC), meta
+// the sort's keys (16 bytes a point), the rest is pair_scratch_bytes.
+static PairData pair_data(const Geo &g, const GridBufs &b) {
+    const size_t n = (size_t)g.n, d = (size_t)g.d;
+    PairData p;
+    p.nb = g.n / kBlkRuns + 1;
+    p.ns = g.n / (kBlkRuns * kSupBlks) + 1;
+    p.rows = (f32x4 *)b.partial;
+    p.meta = (int4 *)b.keys_a;
+    char *at = b.pair;
+    auto take = [&](size_t bytes) {
+        char *r = at;
+        at += (bytes + 255) & ~(size_t)255;
+        return r;
+    };
+    p.totals = (float *)take(8 * d * n);
+    p.blo = (float *)take(4 * d * p.nb);
+    p.bhi = (float *)take(4 * d * p.nb);
+    p.bflag = (int *)take(4 * (size_t)p.nb);
+    p.bcell = (int *)take(4 * (size_t)p.nb);
+    p.slo = (float *)take(4 * d * p.ns);
+    p.shi = (float *)take(4 * d * p.ns);
+    p.sflag = (int *)take(4 * (size_t)p.ns);
+    return p;
+}
+
+size_t pair_scratch_bytes(size_t n, size_t d) {
+    const size_t nb = n / kBlkRuns + 1, ns = n / ((size_t)kBlkRuns * kSupBlks) + 1;
+    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    const size_t used = al(8 * d * n) + 2 * al(4 * d * nb) + 2 * al(4 * nb) + 2 * al(4 * d * ns) +
+                        al(4 * ns);
+    // not below what earlier layouts held, so that the workspace keeps its size
+    return std::max(used, al(4 * n) * 3 + al(4 * d * n) * 2 + al(4 * d * (n / 64 + 1)) * 2 +
+                              al(4 * (n / 64 + 1)) * 2 + al(4 * d * (n / 4096 + 1)) * 2 +
+                              al(4 * (n / 4096 + 1)));
+}
+
+// The runs' rows, the cells' totals (at their first runs) and the blocks' boxes;
+// one wavefront per four blocks.
 template <int D>
 __global__ __launch_bounds__(kBlock) void k_run_boxes(
     const float *__restrict__ Xs, const int *__restrict__ run_start,
     const int *__restrict__ point_cell, const int *__restrict__ cell_run,
-    const int *__restrict__ cell_g, const float *__restrict__ Ts, const float *__restrict__ Tc,
-    Geo g, DevState *st, float *__restrict__ totals, int *__restrict__ rcell,
-    int *__restrict__ rflag, float *__restrict__ Xr, int *__restrict__ gr,
-    int *__restrict__ rlen, float *__restrict__ bmin, float *__restrict__ bmax,
-    int *__restrict__ bclamp, int *__restrict__ bcell) {
+    const int *__restrict__ cell_start, const int *__restrict__ cell_g,
+    const float *__restrict__ Ts, const float *__restrict__ Tc, Geo g, DevState *st, PairData p) {
     if (st->done || st->sparse_count == 0) return;
-    const int n = g.n, runs = st->runs;
-    const int nblk = (runs + kBlkRuns - 1) / kBlkRuns, nb = n / kBlkRuns + 1;
+    constexpr int NC = (2 * D + 3) / 4;
+    const int n = g.n, runs = st->runs, lane = __lane_id();
     const float wf = (float)g.w;
-    for (int b = wave_index(); b < nblk; b += wave_count()) {
-        const int r = b * kBlkRuns + __lane_id();
+    for (int b = wave_index(); b * kWave < runs; b += wave_count()) {
+        const int r = b * kWave + lane;
         const bool on = r < runs;
-        float lo[D], hi[D];
+        float lo[D], hi[D], row[4 * NC];
         int f = 0, c = -1;
+#pragma unroll
+        for (int l = 0; l < 4 * NC; l++) row[l] = 0.f;
         if (on) {
             const int i = run_start[r];
             c = point_cell[i];
@@ -68,18 +120,22 @@ __global__ __launch_bounds__(kBlock) void k_run_boxes(
                 const float x = Xs[(long long)l * n + i];
                 lo[l] = hi[l] = x;
                 clamped |= x / g.cs >= wf;  // cell_coord's clamp of w to w-1
-                Xr[(long long)l * n + r] = x;
-                gr[(long long)l * n + r] = cell_g[(long long)l * n + c];
+                row[l] = x;
+                row[D + l] = ((float)cell_g[(long long)l * n + c] + 0.5f) * g.cs;
             }
             f = (cell_run[c] == r ? 1 : 0) | (clamped ? 2 : 0);
-            rcell[r] = c;
-            rflag[r] = f;
-            rlen[r] = run_start[r + 1] - i;
+            p.meta[r] = make_int4(c, f, run_start[r + 1] - i,
+                                  f & 1 ? cell_start[c + 1] - cell_start[c] : 0);
+#pragma unroll
+            for (int k = 0; k < NC; k++) {
+                const f32x4 q = {row[4 * k], row[4 * k + 1], row[4 * k + 2], row[4 * k + 3]};
+                p.rows[(long long)k * n + r] = q;
+            }
             if (f & 1) {
 #pragma unroll
                 for (int l = 0; l < D; l++) {
-                    totals[(long long)c * 2 * D + l] = Ts[(long long)l * n + c];
-                    totals[(long long)c * 2 * D + D + l] = Tc[(long long)l * n + c];
+                    p.totals[(long long)c * 2 * D + l] = Ts[(long long)l * n + c];
+                    p.totals[(long long)c * 2 * D + D + l] = Tc[(long long)l * n + c];
                 }
             }
         } else {
@@ -89,23 +145,26 @@ __global__ __launch_bounds__(kBlock) void k_run_boxes(
                 hi[l] = -__builtin_inff();
             }
         }
-        const bool any_clamp = __any((f & 2) != 0);
-        const int c_first = __builtin_amdgcn_readfirstlane(c);
-        const bool one_cell = !__any(on && c != c_first);
+        const unsigned long long mine = 0xffffull << (lane & 48);  // the block's lanes
+        const bool any_clamp = (__ballot((f & 2) != 0) & mine) != 0;
+        const int c_first = __shfl(c, lane & 48, kWave);
+        const bool one_cell = (__ballot(on && c != c_first) & mine) == 0;
+        const bool writes = on && (lane & 15) == 0;
+        const int blk = r / kBlkRuns;
 #pragma unroll
         for (int l = 0; l < D; l++) {
-            for (int o = kWave / 2; o > 0; o >>= 1) {
+            for (int o = kBlkRuns / 2; o > 0; o >>= 1) {
                 lo[l] = fminf(lo[l], __shfl_xor(lo[l], o, kWave));
                 hi[l] = fmaxf(hi[l], __shfl_xor(hi[l], o, kWave));
             }
-            if (__lane_id() == 0) {
-                bmin[(long long)l * nb + b] = lo[l];
-                bmax[(long long)l * nb + b] = hi[l];
+            if (writes) {
+                p.blo[(long long)l * p.nb + blk] = lo[l];
+                p.bhi[(long long)l * p.nb + blk] = hi[l];
             }
         }
-        if (__lane_id() == 0) {
-            bclamp[b] = any_clamp ? 1 : 0;
-            bcell[b] = one_cell ? c_first : -1;
+        if (writes) {
+            p.bflag[blk] = any_clamp ? 1 : 0;
+            p.bcell[blk] = one_cell ? c_first : -1;
         }
     }
 }
@@ -113,48 +172,44 @@ __global__ __launch_bounds__(kBlock) void k_run_boxes(
 // Bounding box of every superblock of kSupBlks blocks, and whether it holds a
 // clamped run.
 template <int D>
-__global__ __launch_bounds__(kBlock) void k_super_boxes(
-    const float *__restrict__ bmin, const float *__restrict__ bmax,
-    const int *__restrict__ bclamp, Geo g, DevState *st, float *__restrict__ sbmin,
-    float *__restrict__ sbmax, int *__restrict__ sbclamp) {
+__global__ __launch_bounds__(kBlock) void k_super_boxes(Geo g, DevState *st, PairData p) {
     if (st->done || st->sparse_count == 0) return;
-    const int n = g.n, runs = st->runs;
-    const int nblk = (runs + kBlkRuns - 1) / kBlkRuns, nb = n / kBlkRuns + 1;
-    const int nsup = (nblk + kSupBlks - 1) / kSupBlks, ns = n / (kBlkRuns * kSupBlks) + 1;
+    const int nblk = (st->runs + kBlkRuns - 1) / kBlkRuns;
+    const int nsup = (nblk + kSupBlks - 1) / kSupBlks;
     for (int sb = wave_index(); sb < nsup; sb += wave_count()) {
         const int b = sb * kSupBlks + __lane_id();
         const bool on = b < nblk;
-        const bool any_clamp = __any(on && bclamp[b] != 0);
+        const bool any_clamp = __any(on && p.bflag[b] != 0);
 #pragma unroll
         for (int l = 0; l < D; l++) {
-            float lo = on ? bmin[(long long)l * nb + b] : __builtin_inff();
-            float hi = on ? bmax[(long long)l * nb + b] : -__builtin_inff();
+            float lo = on ? p.blo[(long long)l * p.nb + b] : __builtin_inff();
+            float hi = on ? p.bhi[(long long)l * p.nb + b] : -__builtin_inff();
             for (int o = kWave / 2; o > 0; o >>= 1) {
                 lo = fminf(lo, __shfl_xor(lo, o, kWave));
                 hi = fmaxf(hi, __shfl_xor(hi, o, kWave));
             }
             if (__lane_id() == 0) {
-                sbmin[(long long)l * ns + sb] = lo;
-                sbmax[(long long)l * ns + sb] = hi;
+                p.slo[(long long)l * p.ns + sb] = lo;
+                p.shi[(long long)l * p.ns + sb] = hi;
             }
         }
-        if (__lane_id() == 0) sbclamp[sb] = any_clamp ? 1 : 0;
+        if (__lane_id() == 0) p.sflag[sb] = any_clamp ? 1 : 0;
     }
 }
 
 // Whether box k of a (lo, hi) table ([D][stride]) lies within squared
-// distance thr of the box [alo, ahi] (thr_clamp if the box holds a clamped
-// run).  Box distances round like the point distances they bound; the
+// distance thr of the box a (D lower, D upper bounds; thr_clamp if the box holds
+// a clamped run).  Box distances round like the point distances they bound; the
 // caller's thresholds carry a relative margin of 2^-10 for that.
 template <int D>
-__device__ __forceinline__ bool box_near(const float (&alo)[D], const float (&ahi)[D],
-                                         const float *__restrict__ blo,
+__device__ __forceinline__ bool box_near(const float (&a)[2 * D], const float *__restrict__ blo,
                                          const float *__restrict__ bhi, long long stride, int k,
                                          float thr) {
     float s = 0.f;
 #pragma unroll
     for (int l = 0; l < D; l++) {
-        const float gap = fmaxf(0.f, fmaxf(blo[l * stride + k] - ahi[l], alo[l] - bhi[l * stride + k]));
+        const float gap =
+            fmaxf(0.f, fmaxf(blo[l * stride + k] - a[D + l], a[l] - bhi[l * stride + k]));
         s += gap * gap;
     }
     return s <= thr;
@@ -178,122 +233,123 @@ __device__ __forceinline__ float sin_pair(float v) {
 struct PairBounds {
     float thr_filter, thr_clamp;  // squared filter radii, of clamped sources
     float r, rounding;            // larger filter radius; relative error of the MFMA distance
-    float lo, hi;                 // squared distances surely <= / > thr_eps
+    float lo, hi;                 // face distances less D h^2 surely <= / > thr_eps
 };
 
 constexpr int kPairTargets = 16;  // targets of a tile, four lanes each
+constexpr int kBatchBlks = 8;     // source blocks of a batch
+constexpr int kBatch = kBatchBlks * kBlkRuns;
 
-// Source runs of a block staged in LDS.  x and c (the cell's centre) are rows
-// of 16-byte reads for the accepted pairs, where each lane reads a run of its
-// own; a row stride of 4 mod 8 floats spreads the rows over all banks.  f holds
-// the features of the distance product (row stride odd).
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
+// A batch of source runs in LDS (PairData's rows and meta), and per target the
+// accepted ones of them, in order.
 template <int D>
 struct PairStage {
-    static constexpr int P = (D + 3) / 4 * 4;
-    static constexpr int XS = P % 8 == 0 ? P + 4 : P;
-    static constexpr int KS = (D + 2 + 3) / 4;  // MFMA steps of the distance product
-    static constexpr int FS = 4 * KS + 1;
-    alignas(16) float x[kBlkRuns * XS];
-    alignas(16) float c[kBlkRuns * XS];
-    alignas(16) int4 meta[kBlkRuns];  // cell, flags, length, points of the cell (first runs)
-    float f[kBlkRuns * FS];
+    static constexpr int NC = (2 * D + 3) / 4;
+    f32x4 rows[NC][kBatch];
+    int4 meta[kBatch];
+    float cs[2 * D][kPairTargets];  // cos and sin of the targets
+    float box[2 * D];               // the tile's box
+    unsigned char list[kPairTargets][kBatch];
 };
 
-template <int D>
-__device__ __forceinline__ void read_row(const float *row, float (&v)[PairStage<D>::P]) {
-#pragma unroll
-    for (int l = 0; l < PairStage<D>::P; l += 4) {
-        const f32x4 q = *reinterpret_cast<const f32x4 *>(row + l);
-#pragma unroll
-        for (int k = 0; k < 4; k++) v[l + k] = q[k];
-    }
-}
-
-// The reference's decision for the cell of source run rr as seen from target x
-// in cell c0 (EGG_SynC.cu:612-634): 0 not counted (or not in the neighbour
-// list), 1 full, 2 partial.
-template <int D>
-__device__ int pair_class(const float (&x)[D], int c0, int rr, const int *__restrict__ gr,
-                          const int *__restrict__ cell_g, const Geo &g) {
-    int gc[D];
+// The reference's decision for cell c as seen from the target at sorted position
+// i in cell c0 (EGG_SynC.cu:612-634): 0 not counted (or not in the neighbour
+// list), 1 full, 2 partial.  A loop over memory: it is taken rarely, and its
+// registers would be the pair loop's.
+__device__ __forceinline__ int pair_class(const float *__restrict__ Xs, int i, int c0, int c,
+                                          const int *__restrict__ cell_g, const Geo &g) {
     bool win = true;
-#pragma unroll
-    for (int l = 0; l < D; l++) {
-        gc[l] = gr[(long long)l * g.n + rr];
+    float sm = 0.f, lg = 0.f;
+#pragma unroll 1
+    for (int l = 0; l < g.d; l++) {
+        const float x = Xs[(long long)l * g.n + i];
+        const int gc = cell_g[(long long)l * g.n + c];
         if (l < g.od) {
-            const int dg = gc[l] - cell_g[(long long)l * g.n + c0];
+            const int dg = gc - cell_g[(long long)l * g.n + c0];
             if (dg > g.R || dg < -g.R) win = false;
         }
+        float s1, l1;
+        box_dist<1>(&gc, &x, g.cs, s1, l1);
+        sm += s1;
+        lg += l1;
     }
-    float sm, lg;
-    box_dist<D>(gc, x, g.cs, sm, lg);
     return !win ? 0 : (lg <= g.thr_eps ? 1 : (sm <= g.thr_eps ? 2 : 0));
 }
 
-// Adds lane I of each group of four lanes' v to s on all four.
+// Lane I of each group of four lanes' v, on all four.
 template <int I>
-__device__ __forceinline__ float add_quad(float s, float v) {
-    return s + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), I * 0x55, 0xf, 0xf, true));
+__device__ __forceinline__ int quad_lane(int v) {
+    return __builtin_amdgcn_mov_dpp(v, I * 0x55, 0xf, 0xf, true);
 }
 
 __device__ __forceinline__ int quad_sum(int v) {
-    v += __shfl_xor(v, 1, kWave);
-    return v + __shfl_xor(v, 2, kWave);
+    return quad_lane<0>(v) + quad_lane<1>(v) + quad_lane<2>(v) + quad_lane<3>(v);
 }
 
-// One wavefront per tile of 16 targets (lanes 4t .. 4t+3 serve target t).  Per
-// block of 64 source runs:
-//  1. the squared distances of all 1,024 pairs by v_mfma_f32_16x16x4_f32,
-//     |v|^2 - 2 u.v + (|u|^2 - thr) relative to the tile's centre; its sign bits
-//     are the accepted pairs (one v_alignbit each).  thr holds the filter radius
-//     and a bound on the product's rounding, so that no pair within the filter
-//     is missed; what is accepted beyond it fails the tests below;
-//  2. the four lanes of a target take its accepted runs in turns of four and
-//     evaluate the FP32 distance, the cell's class and sin(x_q - x); the class
-//     comes from the distances to the cell's near and far faces by its centre
-//     (5 instructions a dimension against 8), and where those lie within
-//     rounding of eps, from the reference's own box test (pair_class);
-//  3. the four terms are added one after another (DPP broadcasts within the
-//     four lanes), each lane keeping the target's full sum;
-//  4. full cells met at their first run add their totals, each lane in its own
-//     dimensions.
-// 16 targets a tile instead of 64: a quarter of the idle lanes when targets'
-// counts differ, boxes that prune more, and four times the wavefronts where n
-// is small.  Bound by the VALU, ~200 instructions per 64 evaluated pairs.
+// Adds the terms of a target's four lanes to its sum one after another; every
+// lane keeps the whole sum.
+__device__ __forceinline__ float add_quad(float s, float v) {
+    const int t = __float_as_int(v);
+    s += __int_as_float(quad_lane<0>(t));
+    s += __int_as_float(quad_lane<1>(t));
+    s += __int_as_float(quad_lane<2>(t));
+    return s + __int_as_float(quad_lane<3>(t));
+}
+
+// One wavefront per tile of 16 targets; lanes 4t .. 4t + 3 serve target t.  Blocks
+// that survive the pruning are collected; per batch of eight (128 source runs):
+//  1. the squared distances of all 2,048 pairs by v_mfma_f32_16x16x4_f32,
+//     sum_l (-2 u_l v_l + v_l^2) + (|u|^2 - thr) relative to the tile's centre;
+//     its sign bits are the accepted pairs (one v_alignbit each).  thr holds the
+//     filter radius and a bound on the product's rounding, so that no pair within
+//     the filter is missed; what is accepted beyond it fails the tests below;
+//  2. every target's accepted runs are listed in LDS, in order; its four lanes
+//     take them in turns of four and evaluate the FP32 distance, the cell's class
+//     and sin(x_q - x).  The class comes from the distances to the cell's far and
+//     near faces by its centre, sum d^2 + D h^2 +- 2 h sum |d| (h half the side),
+//     and where those lie within rounding of eps, from the reference's own box
+//     test (pair_class);
+//  3. the four terms are added one after another (DPP broadcasts within the four
+//     lanes).  The matrix cores can do it too, bit for bit (four FMAs in ascending
+//     k), but v_mfma_f32_16x16x4_f32 takes 32 cycles of the same SIMD for what the
+//     four adds of a dimension take 16 for: +20% time;
+//  4. full cells met at their first run add their totals the same way.
+// Blocks of 16 runs prune better than blocks of 64, batches of 128 keep a target's
+// lanes busier, and 16 targets a tile give a wavefront per 16 runs where n is
+// small.  Bound by the VALU: ~190 instructions at d = 8 per 64 evaluated pairs, of
+// which 37 are in use on average in the first pass (the targets' counts differ).
 // n = 250,000, d = 8, eps = 0.1: 65 ms a pass with a lane per target and the
-// totals read (and sinf / cosf taken) inside the pair loop, here 35; n = 14,980,
-// d = 14: 7.3 ms (234 wavefronts), here 1.6.
+// totals read (and sinf / cosf taken) inside the pair loop, 35 with blocks of 64,
+// 28 here; n = 14,980, d = 14: 7.3 ms (234 wavefronts), 1.6, 1.1.
 // SMALL: every pair the filter passes is closer than 1 in each coordinate
 // (filter radius below 1), so sin(x_q - x) takes the polynomial.
+// The register budget keeps 4 wavefronts a SIMD up to d = 3, 3 up to d = 8.
 template <int D, bool SMALL>
-__global__ __launch_bounds__(kBlock) void k_update_pairs(
+__global__ __launch_bounds__(kBlock)
+__attribute__((amdgpu_waves_per_eu(D <= 3 ? 4 : (D <= 8 ? 3 : 1)))) void k_update_pairs(
     const float *__restrict__ Xs, const int *__restrict__ cell_start,
-    const int *__restrict__ cell_g, const float *__restrict__ totals,
-    const int *__restrict__ run_start, const int *__restrict__ point_cell,
-    const int *__restrict__ cell_run, const int *__restrict__ list,
-    const int *__restrict__ rcell, const int *__restrict__ rflag,
-    const float *__restrict__ Xr, const int *__restrict__ gr, const int *__restrict__ rlen,
-    const float *__restrict__ bmin, const float *__restrict__ bmax,
-    const int *__restrict__ bclamp, const int *__restrict__ bcell,
-    const float *__restrict__ sbmin, const float *__restrict__ sbmax,
-    const int *__restrict__ sbclamp, PairBounds pb, float *__restrict__ rres,
+    const int *__restrict__ cell_g, const int *__restrict__ run_start,
+    const int *__restrict__ point_cell, const int *__restrict__ cell_run,
+    const int *__restrict__ list, PairData p, PairBounds pb, float *__restrict__ rres,
     int *__restrict__ rdbg, Geo g, DevState *st) {
     if (st->done) return;
     const int count = st->sparse_count;
     if (count == 0) return;
     using Stage = PairStage<D>;
-    constexpr int P = Stage::P, XS = Stage::XS, KS = Stage::KS, FS = Stage::FS;
-    constexpr int DO = P / 4;  // dimensions of a lane's totals: 4e + sub
+    constexpr int NC = Stage::NC;
+    constexpr int KD = (D + 3) / 4;  // MFMA steps over the dimensions
     __shared__ Stage s_stage[kBlock / kWave];
     Stage &S = s_stage[threadIdx.x / kWave];
-    const int n = g.n, od = g.od, R = g.R, runs = st->runs, lane = __lane_id();
+    const float *S_f = reinterpret_cast<const float *>(S.rows);
+    const int n = g.n, runs = st->runs, lane = __lane_id();
     const int tq = lane >> 2, sub = lane & 3;   // target and lane of the target
     const int j16 = lane & 15, kq = lane >> 4;  // MFMA column (target) and k
-    const int nblk = (runs + kBlkRuns - 1) / kBlkRuns, nb = n / kBlkRuns + 1;
-    const int nsup = (nblk + kSupBlks - 1) / kSupBlks, ns = n / (kBlkRuns * kSupBlks) + 1;
-    const float thr = g.thr_eps, thr_half = g.thr_half, halfcs = 0.5f * g.cs;
+    const int nblk = (runs + kBlkRuns - 1) / kBlkRuns;
+    const int nsup = (nblk + kSupBlks - 1) / kSupBlks;
+    // the pair loop's constants, kept in vector registers: the scalar ones are
+    // short, and a spilled one costs the loop a v_readlane
+    float thr = g.thr_eps, thr_half = g.thr_half, lo = pb.lo, hi = pb.hi, cs = g.cs;
+    __asm__ volatile("" : "+v"(thr), "+v"(thr_half), "+v"(lo), "+v"(hi), "+v"(cs));
     const float box_thr = pb.thr_filter * (1.0f + 0x1p-10f);
     const float box_thr_clamp = pb.thr_clamp * (1.0f + 0x1p-10f);
     const int ntiles = (count + kPairTargets - 1) / kPairTargets;
@@ -306,253 +362,262 @@ __global__ __launch_bounds__(kBlock) void k_update_pairs(
         const int i = run_start[r];
         const int c0 = point_cell[i];
         const int own = cell_start[c0 + 1] - cell_start[c0];
-        float x[D], sml[D], tlo[D], thi[D], a[D];
-        float xo[DO], cxo[DO], sxo[DO], sum[DO];
+        // full cells' totals and partial cells' terms, on each of the four lanes
+        float x[D], sum[D], sml[D];
         bool border = false;
         float rho = 0.f;
 #pragma unroll
         for (int l = 0; l < D; l++) {
             x[l] = Xs[(long long)l * n + i];
-            sml[l] = 0.f;
+            sum[l] = sml[l] = 0.f;
             border |= on_border(x[l], g.cs);
-            tlo[l] = active ? x[l] : __builtin_inff();
-            thi[l] = active ? x[l] : -__builtin_inff();
+            float tlo = active ? x[l] : __builtin_inff();
+            float thi = active ? x[l] : -__builtin_inff();
             for (int o = kWave / 2; o > 2; o >>= 1) {
-                tlo[l] = fminf(tlo[l], __shfl_xor(tlo[l], o, kWave));
-                thi[l] = fmaxf(thi[l], __shfl_xor(thi[l], o, kWave));
+                tlo = fminf(tlo, __shfl_xor(tlo, o, kWave));
+                thi = fmaxf(thi, __shfl_xor(thi, o, kWave));
             }
-            a[l] = 0.5f * (tlo[l] + thi[l]);
-            rho = fmaf(thi[l] - tlo[l], thi[l] - tlo[l], rho);
+            S.box[l] = tlo;  // every lane, the same value
+            S.box[D + l] = thi;
+            rho = fmaf(thi - tlo, thi - tlo, rho);
         }
+        wave_sync();
+        if (sub == 0) {
 #pragma unroll
-        for (int e = 0; e < DO; e++) {
-            const int l = 4 * e + sub;
-            xo[e] = l < D ? Xs[(long long)l * n + i] : 0.f;
-            cxo[e] = cosf(xo[e]);
-            sxo[e] = sinf(xo[e]);
-            sum[e] = 0.f;
+            for (int l = 0; l < D; l++) {
+                S.cs[l][tq] = cosf(x[l]);
+                S.cs[D + l][tq] = sinf(x[l]);
+            }
         }
-        // the targets' side of the distance product: -2u, 1, |u|^2 - thr
-        float bf[KS];
+        const bool any_border = __any(border);
+        // the distance product: anchors af of the lane's dimensions 4s + kq, the
+        // targets' side -2u, and its constant |u|^2 - thr (on lanes kq = 0)
+        float af[KD], bf[KD], b1 = 0.f;
         {
             // |u| <= half the box's diagonal; the sources that matter are
             // within it plus the filter radius
             const float reach = sqrtf(rho) + pb.r;
             const float slack = pb.rounding * (reach * reach + pb.r * pb.r);
-            const int from = 4 * j16;
             float u2 = 0.f;
 #pragma unroll
-            for (int s = 0; s < KS; s++) bf[s] = 0.f;
+            for (int s = 0; s < KD; s++) af[s] = bf[s] = 0.f;
 #pragma unroll
             for (int l = 0; l < D; l++) {
-                const float u = __shfl(x[l], from, kWave) - a[l];
+                const float al = 0.5f * (S.box[l] + S.box[D + l]);
+                const float u = __shfl(x[l], 4 * j16, kWave) - al;
                 u2 = fmaf(u, u, u2);
-                if (kq == l % 4) bf[l / 4] = -2.f * u;
-            }
-            const bool on = t * kPairTargets + j16 < count;
-            if (kq == D % 4) bf[D / 4] = 1.f;
-            if (kq == (D + 1) % 4) bf[(D + 1) / 4] = on ? u2 - pb.thr_filter - slack : 1e30f;
-        }
-        int N = 0, half = 0;
-        for (int sb0 = 0; sb0 < nsup; sb0 += kWave) {
-            const int sbl = sb0 + lane;
-            const bool sp = sbl < nsup &&
-                            box_near<D>(tlo, thi, sbmin, sbmax, ns, sbl,
-                                        sbclamp[sbl] ? box_thr_clamp : box_thr);
-            for (unsigned long long ms = __ballot(sp); ms; ms &= ms - 1) {
-                const int sb = sb0 + __ffsll((long long)ms) - 1;
-                const int bl = sb * kSupBlks + lane;
-                const bool bp = bl < nblk &&
-                                box_near<D>(tlo, thi, bmin, bmax, nb, bl,
-                                            bclamp[bl] ? box_thr_clamp : box_thr);
-                for (unsigned long long mb = __ballot(bp); mb; mb &= mb - 1) {
-                    const int b = sb * kSupBlks + __ffsll((long long)mb) - 1;
-                    const int r0 = b * kBlkRuns;
-                    // a block whose runs share one cell c (a dense cell): one
-                    // box test of c per target decides for all its runs, unless
-                    // c is partial for it or a border target needs its eps/2
-                    // count; if no target needs the runs one by one, the block
-                    // is not staged, and targets for which c is full add its
-                    // totals in the block holding its first run
-                    const int bc = bcell[b];
-                    if (bc >= 0 && !bclamp[b]) {
-                        const int cls = active ? pair_class<D>(x, c0, r0, gr, cell_g, g) : 0;
-                        if (!__any(cls == 2 || (cls == 1 && border && bc != c0))) {
-                            const int fr = cell_run[bc];
-                            if (cls == 1 && fr >= r0 && fr < r0 + kBlkRuns) {
-                                const float *row = totals + (long long)bc * 2 * D;
-#pragma unroll
-                                for (int e = 0; e < DO; e++) {
-                                    const int l = 4 * e + sub;
-                                    if (l < D) {
-                                        const float p1 = row[l] * cxo[e];
-                                        const float p2 = row[D + l] * sxo[e];
-                                        const float tt = p1 - p2;
-                                        sum[e] += tt;
-                                    }
-                                }
-                                if (sub == 0) {
-                                    const int cnt = cell_start[bc + 1] - cell_start[bc];
-                                    N += cnt;
-                                    if (border && bc == c0) half += cnt;
-                                }
-                            }
-                            continue;
-                        }
-                    }
-                    {
-                        const int rr = r0 + lane;
-                        const bool on = rr < runs;
-                        float v2 = 0.f;
-                        int fl = 0;
-                        if (on) {
-                            const int c = rcell[rr];
-                            fl = rflag[rr];
-                            S.meta[lane] = make_int4(
-                                c, fl, rlen[rr], fl & 1 ? cell_start[c + 1] - cell_start[c] : 0);
-                        }
-#pragma unroll
-                        for (int l = 0; l < D; l++) {
-                            float v = 0.f;
-                            if (on) {
-                                const float xq = Xr[(long long)l * n + rr];
-                                S.x[lane * XS + l] = xq;
-                                S.c[lane * XS + l] =
-                                    ((float)gr[(long long)l * n + rr] + 0.5f) * g.cs;
-                                v = xq - a[l];
-                            }
-                            v2 = fmaf(v, v, v2);
-                            S.f[lane * FS + l] = v;
-                        }
-                        // a clamped run is accepted up to its wider radius
-                        if (fl & 2) v2 -= pb.thr_clamp - pb.thr_filter;
-                        S.f[lane * FS + D] = on ? v2 : 1e30f;
-                        S.f[lane * FS + D + 1] = 1.f;
-#pragma unroll
-                        for (int l = D + 2; l < 4 * KS; l++) S.f[lane * FS + l] = 0.f;
-                    }
-                    wave_sync();
-                    // lane (j16, kq): sign bits of target j16 and sources 16kq .. 16kq+15
-                    unsigned bits = 0;
-#pragma unroll
-                    for (int tau = 3; tau >= 0; tau--) {
-                        const float *row =
-                            S.f + (16 * (j16 >> 2) + 4 * tau + (j16 & 3)) * FS + kq;
-                        f32x4 d = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                        for (int s = 0; s < KS; s++)
-                            d = __builtin_amdgcn_mfma_f32_16x16x4f32(row[4 * s], bf[s], d, 0, 0, 0);
-#pragma unroll
-                        for (int q = 3; q >= 0; q--)
-                            bits = __builtin_amdgcn_alignbit(bits, __float_as_uint(d[q]), 31);
-                    }
-                    unsigned long long acc =
-                        (unsigned)__shfl((int)bits, tq, kWave) |
-                        (unsigned)__shfl((int)bits, tq + 16, kWave) << 16;
-                    acc |= (unsigned long long)((unsigned)__shfl((int)bits, tq + 32, kWave) |
-                                                (unsigned)__shfl((int)bits, tq + 48, kWave) << 16)
-                           << 32;
-                    // this lane's runs are the sub-th, (sub+4)-th, ... of the target's
-#pragma unroll
-                    for (int q = 0; q < 3; q++)
-                        if (sub > q) acc &= acc - 1;
-                    unsigned long long fullm = 0;  // full cells' first runs
-                    while (__any(acc != 0)) {
-                        float term[D];
-#pragma unroll
-                        for (int l = 0; l < D; l++) term[l] = 0.f;
-                        if (acc) {
-                            const int q = __ffsll((long long)acc) - 1;
-                            acc &= acc - 1;
-                            acc &= acc - 1;
-                            acc &= acc - 1;
-                            acc &= acc - 1;
-                            float xq[P], cq[P];
-                            read_row<D>(S.x + q * XS, xq);
-                            read_row<D>(S.c + q * XS, cq);
-                            const int4 meta = S.meta[q];
-                            float s = 0.f, lg = 0.f, sm = 0.f;
-#pragma unroll
-                            for (int l = 0; l < D; l++) {
-                                xq[l] -= x[l];
-                                s += xq[l] * xq[l];
-                                const float d = fabsf(x[l] - cq[l]);
-                                const float df = d + halfcs, dn = d - halfcs;
-                                lg = fmaf(df, df, lg);
-                                sm = fmaf(dn, dn, sm);
-                            }
-                            // sm > thr where the outer coordinates differ by more
-                            // than R, up to rounding, which pair_class decides
-                            int cls = lg <= pb.lo ? 1 : (sm <= pb.lo ? 2 : 0);
-                            if ((lg > pb.lo && lg < pb.hi) || (sm > pb.lo && sm < pb.hi))
-                                cls = pair_class<D>(x, c0, r0 + q, gr, cell_g, g);
-                            if (cls == 1) {
-                                if (meta.y & 1) fullm |= 1ull << q;
-                                if (border && meta.x != c0 && s <= thr_half) half += meta.z;
-                            } else if (cls == 2 && s <= thr) {
-                                const float w = (float)meta.z;  // exact: < 2^24
-#pragma unroll
-                                for (int l = 0; l < D; l++) term[l] = w * sin_pair<SMALL>(xq[l]);
-                                N += meta.z;
-                            }
-                        }
-#pragma unroll
-                        for (int l = 0; l < D; l++) {
-                            sml[l] = add_quad<0>(sml[l], term[l]);
-                            sml[l] = add_quad<1>(sml[l], term[l]);
-                            sml[l] = add_quad<2>(sml[l], term[l]);
-                            sml[l] = add_quad<3>(sml[l], term[l]);
-                        }
-                    }
-                    // the target's full cells, in order, on all four lanes
-                    if (__any(fullm != 0)) {
-                        unsigned flo = (unsigned)fullm, fhi = (unsigned)(fullm >> 32);
-                        flo |= (unsigned)__shfl_xor((int)flo, 1, kWave);
-                        fhi |= (unsigned)__shfl_xor((int)fhi, 1, kWave);
-                        flo |= (unsigned)__shfl_xor((int)flo, 2, kWave);
-                        fhi |= (unsigned)__shfl_xor((int)fhi, 2, kWave);
-                        fullm = flo | (unsigned long long)fhi << 32;
-                        while (fullm) {
-                            const int q = __ffsll((long long)fullm) - 1;
-                            fullm &= fullm - 1;
-                            const int4 meta = S.meta[q];
-                            const float *row = totals + (long long)meta.x * 2 * D;
-#pragma unroll
-                            for (int e = 0; e < DO; e++) {
-                                const int l = 4 * e + sub;
-                                if (l < D) {
-                                    const float p1 = row[l] * cxo[e];
-                                    const float p2 = row[D + l] * sxo[e];
-                                    const float tt = p1 - p2;
-                                    sum[e] += tt;
-                                }
-                            }
-                            if (sub == 0) {
-                                N += meta.w;
-                                if (border && meta.x == c0) half += meta.w;
-                            }
-                        }
-                    }
-                    wave_sync();
+                if (kq == l % 4) {
+                    af[l / 4] = al;
+                    bf[l / 4] = -2.f * u;
                 }
             }
+            const bool on = t * kPairTargets + j16 < count;
+            if (kq == 0) b1 = on ? u2 - pb.thr_filter - slack : 1e30f;
+        }
+        const float one_last = 4 * (KD - 1) + kq < D ? 1.f : 0.f;
+        int N = 0, half = 0;
+        // blocks still to come: superblocks of ms, blocks of mb; `pend` holds on
+        // lane k the k-th block collected (bit 30: it has a clamped run)
+        unsigned long long ms = 0, mb = 0;
+        int sb_next = 0, sbase = 0, bbase = 0;
+        // the last cell whose runs filled a whole block: the targets' classes
+        int last_bc = -1, last_cls = 0;
+        bool last_need = false;
+        for (;;) {
+            int np = 0, pend = 0;
+            while (np < kBatchBlks) {
+                if (!mb) {
+                    while (!ms && sb_next < nsup) {
+                        const int sbl = sb_next + lane;
+                        const bool sp = sbl < nsup &&
+                                        box_near<D>(S.box, p.slo, p.shi, p.ns, sbl,
+                                                    p.sflag[sbl] ? box_thr_clamp : box_thr);
+                        ms = __ballot(sp);
+                        sbase = sb_next;
+                        sb_next += kWave;
+                    }
+                    if (!ms) break;
+                    bbase = (sbase + __ffsll((long long)ms) - 1) * kSupBlks;
+                    ms &= ms - 1;
+                    const int bl = bbase + lane;
+                    const bool bp = bl < nblk &&
+                                    box_near<D>(S.box, p.blo, p.bhi, p.nb, bl,
+                                                p.bflag[bl] ? box_thr_clamp : box_thr);
+                    mb = __ballot(bp);
+                    continue;
+                }
+                const int b = bbase + __ffsll((long long)mb) - 1;
+                mb &= mb - 1;
+                const int bc = p.bcell[b], clamped = p.bflag[b];
+                if (bc >= 0 && !clamped) {
+                    // a block whose runs share one cell (a dense cell): one box
+                    // test per target decides for all its runs, unless the cell
+                    // is partial for it or a border target needs its eps/2 count.
+                    // If no target needs the runs one by one, the block is passed
+                    // by, unless the cell's first run is in it and some target is
+                    // to add the cell's totals there
+                    if (bc != last_bc) {
+                        last_bc = bc;
+                        last_cls = active ? pair_class(Xs, i, c0, bc, cell_g, g) : 0;
+                        last_need = __any(last_cls == 2 || (last_cls == 1 && border && bc != c0));
+                    }
+                    if (!last_need) {
+                        const int fr = cell_run[bc] - b * kBlkRuns;
+                        if (fr < 0 || fr >= kBlkRuns || !__any(last_cls == 1)) continue;
+                    }
+                }
+                if (lane == np) pend = b | (clamped ? 1 << 30 : 0);
+                np++;
+            }
+            if (np == 0) break;
+            // the batch to LDS; slots past the last block or run repeat run
+            // runs - 1 and are masked out below
+#pragma unroll
+            for (int h = 0; h < kBatch / kWave; h++) {
+                const int slot = h * 4 + kq;
+                const int b = __shfl(pend, slot, kWave) & 0x3fffffff;
+                const unsigned rr = (unsigned)min(b * kBlkRuns + j16, runs - 1);
+#pragma unroll
+                for (int q = 0; q < NC; q++)
+                    S.rows[q][h * kWave + lane] = (p.rows + (long long)q * n)[rr];
+                S.meta[h * kWave + lane] = p.meta[rr];
+            }
+            wave_sync();
+            // lane (j16, kq): bit 4 s + q = target j16 accepts run 4 kq + q of
+            // block s
+            unsigned bits = 0;
+#pragma unroll
+            for (int s = kBatchBlks - 1; s >= 0; s--) {
+                if (s >= np) continue;
+                f32x4 d = {0.f, 0.f, 0.f, 0.f};
+                float v[KD];
+#pragma unroll
+                for (int q = 0; q < KD; q++) {
+                    v[q] = S_f[(q * kBatch + s * kBlkRuns + j16) * 4 + kq] - af[q];
+                    d = __builtin_amdgcn_mfma_f32_16x16x4f32(v[q], bf[q], d, 0, 0, 0);
+                }
+#pragma unroll
+                for (int q = 0; q < KD; q++)
+                    d = __builtin_amdgcn_mfma_f32_16x16x4f32(v[q] * v[q], q + 1 < KD ? 1.f : one_last,
+                                                             d, 0, 0, 0);
+                // a block with a clamped run is accepted up to the wider radius
+                const bool wide = __builtin_amdgcn_readlane(pend, s) >> 30;
+                const float wider = wide && kq == 0 ? pb.thr_clamp - pb.thr_filter : 0.f;
+                d = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, b1 - wider, d, 0, 0, 0);
+#pragma unroll
+                for (int q = 3; q >= 0; q--)
+                    bits = __builtin_amdgcn_alignbit(bits, __float_as_uint(d[q]), 31);
+            }
+            // lane (tq, sub): the target's bits of blocks 2 sub and 2 sub + 1
+            unsigned own_bits = 0;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const unsigned two = (unsigned)__shfl((int)bits, tq + 16 * q, kWave) >> (8 * sub);
+                own_bits |= (two & 15u) << (4 * q) | ((two >> 4) & 15u) << (16 + 4 * q);
+            }
+            {
+                // runs past the end of the last block
+                const int r0 = runs - (__shfl(pend, 2 * sub, kWave) & 0x3fffffff) * kBlkRuns;
+                const int r1 = runs - (__shfl(pend, 2 * sub + 1, kWave) & 0x3fffffff) * kBlkRuns;
+                if (r0 < kBlkRuns) own_bits &= ~0u << 16 | ((1u << r0) - 1u);
+                if (r1 < kBlkRuns) own_bits &= 0xffffu | ((1u << r1) - 1u) << 16;
+            }
+            // the target's list of accepted places in the batch
+            const int mine = __popc(own_bits);
+            const int n0 = quad_lane<0>(mine), n1 = quad_lane<1>(mine), n2 = quad_lane<2>(mine);
+            const int tot = n0 + n1 + n2 + quad_lane<3>(mine);
+            int at = (sub > 0 ? n0 : 0) + (sub > 1 ? n1 : 0) + (sub > 2 ? n2 : 0);
+            while (own_bits) {
+                S.list[tq][at++] = (unsigned char)(32 * sub + __builtin_ctz(own_bits));
+                own_bits &= own_bits - 1;
+            }
+            wave_sync();
+            // the accepted pairs, straight-line code: lanes past the end of their
+            // list evaluate some staged run with weight 0
+            int nfull = 0;  // full cells' first runs met; listed in place of read entries
+            for (int rank = sub; __any(rank < tot); rank += 4) {
+                const bool in = rank < tot;
+                const int q = S.list[tq][min(rank, kBatch - 1)] & (kBatch - 1);
+                float row[4 * NC];
+#pragma unroll
+                for (int c = 0; c < NC; c++) {
+                    const f32x4 v = S.rows[c][q];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) row[4 * c + e] = v[e];
+                }
+                const int4 meta = S.meta[q];
+                float s = 0.f, d2 = 0.f, d1 = 0.f;
+#pragma unroll
+                for (int l = 0; l < D; l++) {
+                    row[l] -= x[l];
+                    s += row[l] * row[l];
+                    const float d = row[D + l] - x[l];
+                    d2 = fmaf(d, d, d2);
+                    d1 += fabsf(d);
+                }
+                const float lg = fmaf(cs, d1, d2), sm = fmaf(-cs, d1, d2);
+                bool full = lg <= lo, part = !full && sm <= lo;
+                // sm > thr where the outer coordinates differ by more than R, up to
+                // rounding, which pair_class decides
+                const bool unsure = in && ((lg > lo && lg < hi) || (sm > lo && sm < hi));
+                if (__any(unsure)) {
+                    if (unsure) {
+                        const int cls = pair_class(Xs, i, c0, meta.x, cell_g, g);
+                        full = cls == 1;
+                        part = cls == 2;
+                    }
+                }
+                const int len = in && part && s <= thr ? meta.z : 0;
+                N += len;
+                if (__any(len > 0)) {
+                    const float w = (float)len;  // exact: < 2^24
+#pragma unroll
+                    for (int l = 0; l < D; l++)
+                        sml[l] = add_quad(sml[l], w * sin_pair<SMALL>(row[l]));
+                }
+                full = full && in;
+                if (any_border) {
+                    if (full && border && meta.x != c0 && s <= thr_half) half += meta.z;
+                }
+                const bool first = full && (meta.y & 1);
+                const unsigned quad = (unsigned)(__ballot(first) >> (lane & 60)) & 15u;
+                if (first)
+                    S.list[tq][nfull + __popc(quad & ((1u << sub) - 1u))] = (unsigned char)q;
+                nfull += __popc(quad);
+            }
+            // the target's full cells, in order, its lanes in turns of four
+            for (int rank = sub; __any(rank < nfull); rank += 4) {
+                float term[D];
+#pragma unroll
+                for (int l = 0; l < D; l++) term[l] = 0.f;
+                if (rank < nfull) {
+                    const int4 meta = S.meta[S.list[tq][rank]];
+                    const float *row = p.totals + (long long)meta.x * 2 * D;
+#pragma unroll
+                    for (int l = 0; l < D; l++) {
+                        const float p1 = row[l] * S.cs[l][tq];
+                        const float p2 = row[D + l] * S.cs[D + l][tq];
+                        term[l] = p1 - p2;
+                    }
+                    N += meta.w;
+                    if (border && meta.x == c0) half += meta.w;
+                }
+#pragma unroll
+                for (int l = 0; l < D; l++) sum[l] = add_quad(sum[l], term[l]);
+            }
+            wave_sync();
         }
         N = quad_sum(N);
         half = quad_sum(half);
         if (active) {
             const bool synced = !((!border && N != own) || (border && N != half));
             if (!synced) unsynced = true;
+            if (sub == 0) {
 #pragma unroll
-            for (int e = 0; e < DO; e++) {
-                const int l = 4 * e + sub;
-                float part = sml[4 * e];
-#pragma unroll
-                for (int q = 1; q < 4; q++)
-                    if (4 * e + q < D && sub == q) part = sml[4 * e + q];
-                if (l < D) {
-                    float tt = sum[e] + part;
+                for (int l = 0; l < D; l++) {
+                    float tt = sum[l] + sml[l];
                     tt = tt / (float)N;
-                    rres[(long long)l * n + r] = xo[e] + tt;
+                    rres[(long long)l * n + r] = x[l] + tt;
                 }
             }
             if (rdbg && sub == 0) {
@@ -572,10 +637,12 @@ __global__ __launch_bounds__(kBlock) void k_update_pairs(
 // outside the box of cell w-1 in each such dimension), eps + sqrt(d)(1 - w cs).
 // The MFMA distance: d + 4 FMAs on terms of at most (|u| + |v|)^2 + thr, and as
 // many roundings in |u|^2 and |v|^2; 4d + 32 covers them four times over.
-// The face distances: both ways of taking them (the reference's from g cs and
-// (g+1) cs, here from the cell's centre) are within 2^-24 (4 sqrt(d) / eps +
-// d + 10) of the exact ones, relative, near eps; four times that separates
-// "surely" from pair_class.
+// The face distances: the reference takes them from g cs and (g+1) cs, the pair
+// loop from the cell's centre as sum d^2 +- 2 h sum |d| + D h^2.  Near eps both are
+// within 2^-24 (4 sqrt(d) / eps + 3 d + 10) of the exact ones, relative (positions
+// round by 2^-24, and sum d^2 + 2 h sum |d| stays below 2.3 eps^2 where the near
+// distance is eps); four times that separates "surely" from pair_class.  lo and hi
+// bound the distances less D h^2.
 static PairBounds pair_bounds(const Geo &g) {
     PairBounds p;
     p.thr_filter = g.thr_eps * (1.0f + 0x1p-12f);
@@ -584,39 +651,34 @@ static PairBounds pair_bounds(const Geo &g) {
     p.thr_clamp = std::max(p.thr_filter, (float)(r * r * (1.0 + 0x1p-10)));
     p.r = (float)(std::sqrt((double)p.thr_clamp) * (1.0 + 0x1p-20));
     p.rounding = (float)((4 * g.d + 32) * 0x1p-24);
-    const double m = 0x1p-24 * (16.0 * std::sqrt((double)g.d) / (double)g.eps + 4.0 * g.d + 64.0);
-    p.lo = m < 0.5 ? (float)((double)g.thr_eps * (1.0 - m)) : -1.0f;
-    p.hi = m < 0.5 ? (float)((double)g.thr_eps * (1.0 + m)) : INFINITY;
+    const double m = 0x1p-24 * (16.0 * std::sqrt((double)g.d) / (double)g.eps + 12.0 * g.d + 64.0);
+    const double dh2 = 0.25 * g.d * (double)g.cs * (double)g.cs;
+    p.lo = m < 0.5 ? (float)((double)g.thr_eps * (1.0 - m) - dh2) : -INFINITY;
+    p.hi = m < 0.5 ? (float)((double)g.thr_eps * (1.0 + m) - dh2) : INFINITY;
     return p;
 }
 
 void launch_update_pairs(const Geo &g, GridBufs &b, int *rdbg, DevState *st, hipStream_t s) {
-    const long long nblk_max = g.n / kBlkRuns + 1;
     const int waves = kBlock / kWave;
-    const int pb = (int)std::min<long long>(16384, (nblk_max + waves - 1) / waves);
-    const int sb = (int)std::max<long long>(
-        1, std::min<long long>(1024, (nblk_max / kSupBlks + waves) / waves));
+    const int pb = (int)std::min<long long>(16384, ((long long)g.n / kWave + waves) / waves);
+    const long long nsup_max = g.n / (kBlkRuns * kSupBlks) + 1;
+    const int sb = (int)std::min<long long>(1024, (nsup_max + waves - 1) / waves);
     const long long tiles_max = g.n / kPairTargets + 1;
     const int pq = (int)std::min<long long>(kQueueBlocks, (tiles_max + waves - 1) / waves);
     const PairBounds bounds = pair_bounds(g);
-    // the summaries' partials are free: 4 d (n + ...) floats for 2 d per cell
-    float *totals = b.partial;
+    const PairData data = pair_data(g, b);
     // every filtered pair is closer than 1 in each coordinate
     const bool pair_small = bounds.thr_clamp < 1.0f;
-#define PAIR_LAUNCH(DD, SMALL)                                                                  \
-    k_update_pairs<DD, SMALL><<<pq, kBlock, 0, s>>>(                                            \
-        b.Xs, b.cell_start, b.cell_g, totals, b.run_start, b.point_cell, b.cell_run,            \
-        g.pair_mode == kPairAll ? nullptr : b.sparse_runs, b.rcell, b.rflag, b.Xr, b.gr,        \
-        b.rlen, b.bmin, b.bmax, b.bclamp, b.bcell, b.sbmin, b.sbmax, b.sbclamp, bounds, b.rres, \
-        rdbg, g, st)
+#define PAIR_LAUNCH(DD, SMALL)                                                                \
+    k_update_pairs<DD, SMALL><<<pq, kBlock, 0, s>>>(                                          \
+        b.Xs, b.cell_start, b.cell_g, b.run_start, b.point_cell, b.cell_run,                  \
+        g.pair_mode == kPairAll ? nullptr : b.sparse_runs, data, bounds, b.rres, rdbg, g, st)
 #define PAIR_CASE(DD)                                                                          \
     case DD:                                                                                   \
         k_run_boxes<DD><<<pb, kBlock, 0, s>>>(b.Xs, b.run_start, b.point_cell, b.cell_run,     \
-                                              b.cell_g, b.Ts, b.Tc, g, st, totals, b.rcell,    \
-                                              b.rflag, b.Xr, b.gr, b.rlen, b.bmin, b.bmax,     \
-                                              b.bclamp, b.bcell);                              \
-        k_super_boxes<DD><<<sb, kBlock, 0, s>>>(b.bmin, b.bmax, b.bclamp, g, st, b.sbmin,      \
-                                                b.sbmax, b.sbclamp);                           \
+                                              b.cell_start, b.cell_g, b.Ts, b.Tc, g, st,       \
+                                              data);                                           \
+        k_super_boxes<DD><<<sb, kBlock, 0, s>>>(g, st, data);                                  \
         if (pair_small) PAIR_LAUNCH(DD, true);                                                 \
         else PAIR_LAUNCH(DD, false);                                                           \
         break;

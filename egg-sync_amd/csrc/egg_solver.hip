@@ -189,21 +189,7 @@ Layout carve(void *base, const Geo &g) {
     b.utile_off = c.take<int>(n);
     b.rres = c.take<float>(n * d);
     b.sparse_runs = c.take<int>(n);
-    b.rcell = c.take<int>(n);
-    b.rflag = c.take<int>(n);
-    b.Xr = c.take<float>(n * d);
-    b.gr = c.take<int>(n * d);
-    b.rlen = c.take<int>(n);
-    {
-        const size_t nb = n / kBlkRuns + 1, ns = n / ((size_t)kBlkRuns * kSupBlks) + 1;
-        b.bmin = c.take<float>(nb * d);
-        b.bmax = c.take<float>(nb * d);
-        b.bclamp = c.take<int>(nb);
-        b.bcell = c.take<int>(nb);
-        b.sbmin = c.take<float>(ns * d);
-        b.sbmax = c.take<float>(ns * d);
-        b.sbclamp = c.take<int>(ns);
-    }
+    b.pair = c.take<char>(pair_scratch_bytes(n, d));
     b.sparse_off = c.take<int>(n);
     b.rdbg = c.take<int>(4 * n);
     b.hacc = g.d <= kHeavyMaxD ? c.take<long long>((2 * d + 2) * n) : nullptr;

@@ -483,3 +483,24 @@ def test_sync_pass_at_tile_edges(S, O, d):
             assert np.abs(a["X"] - b["X"]).max() <= 1e-6
             assert abs(a["stats"]["rc"] - O.rc(X, eps)) <= 1e-7
             assert O.same_partition(a["labels"], b["labels"])
+
+
+@pytest.mark.parametrize("d", [1, 2, 3, 5, 8, 16, 17])
+def test_pair_update_at_batch_edges(S, O, d):
+    """The pair update (every group) at the remainders of its tiles of 16 targets, blocks of 16 runs,
+    batches of 128 and superblocks of 1,024, with clamped points (coordinate 1), points on cell
+    faces and runs of several points, from every pair within eps to few: the pass's positions
+    within 1e-6 of the oracle's, as in test_iteration_bit_exact."""
+    rng = np.random.default_rng(80 + d)
+    for n in (1, 2, 15, 16, 17, 127, 128, 129, 1023, 1025):
+        for eps in (0.02, 0.15, 0.4 * np.sqrt(d)):
+            X = (rng.random((n, d)) * 0.6 + 0.2).astype(np.float32)
+            cs = S.nat.geometry(n, d, eps)["cs"]
+            X[: n // 8] = 1.0 - X[: n // 8] * 0.05
+            X[n // 4: n // 3, 0] = np.float32(3 * cs)
+            X[n // 2: n // 2 + 5] = X[n // 2]
+            X[-1, d - 1] = 1.0
+            _say("pair update", n, d, eps)
+            a = S.solve(X, eps, max_iter=1, pair_groups=2)
+            b = O.egg_iteration(X, eps)
+            assert np.abs(a["X"] - b["X_next"]).max() <= 1e-6, (n, eps)
