@@ -301,7 +301,7 @@ int launch_labels(int d, const float *X, int n, float thr, int *C, int *incl, in
         EGG_EACH_D(LAB_CASE)
     }
 #undef LAB_CASE
-    scan_exclusive(incl, pos, n, nullptr, tmp, k, nullptr, s);
+    scan_exclusive(incl, pos, n, tmp, k, s);
     k_brute_rename<<<std::min((n + kBlock - 1) / kBlock, 4096), kBlock, 0, s>>>(C, pos, n);
     return hip_err(hipGetLastError());
 }

@@ -25,9 +25,13 @@ constexpr int kBlock = 256;       // threads per block (4 wavefronts)
 constexpr int kWave = 64;
 constexpr int kScanItems = 8;     // items per thread in scans
 constexpr int kScanTile = kBlock * kScanItems;
+constexpr int kScanNarrow = 2;    // in scans of few values: of up to kScanNarrowMax, and of
+constexpr int kScanNarrowMax = 1 << 16;   // up to kTablesNarrowMax where the points are
+constexpr int kTablesNarrowMax = 1 << 18; // gathered on the way
 constexpr int kSortItems = 8;     // items per thread in radix passes
 constexpr int kSortTile = kBlock * kSortItems;
 constexpr int kSumChunk = 256;    // max points per summary work item
+constexpr int kSumSmall = 32;     // groups up to this many points share a wavefront's summary
 constexpr int kTile = 64;         // max runs per update tile (one wavefront)
 constexpr int kDefaultGroup = 1;  // default cells per tile group along the last coordinate
 constexpr int kAnchorBlock = 8;   // group widths are powers of two dividing this
@@ -64,6 +68,12 @@ __host__ __device__ __forceinline__ bool sparse_group(int runs, int all_runs, in
     const bool sparse_grid = (long long)all_runs < (long long)kSparseFactor * cells;
     if (mode == kPairAuto && d >= kPairAllMinD) return sparse_grid;
     return runs < kSparseRuns && sparse_grid;
+}
+
+// Whether a pass that has sparse groups has only those (sparse_group does not
+// look at the group's runs then): the pair update takes every run.
+__host__ __device__ __forceinline__ bool pairs_take_all(int mode, int d) {
+    return mode == kPairAll || (mode == kPairAuto && d >= kPairAllMinD);
 }
 
 // Grid geometry and thresholds, computed on the host (EGG_SynC.cu:1249-1260).
@@ -140,7 +150,6 @@ struct DevState {
     int flag;          // local-sync flag of the current iteration (1 = synced)
     int flag_local;    // flag before the extra check (diagnostics)
     int C;             // non-empty cells of the current grid
-    int W;             // summary work items
     int capped;        // 1 if max_iter stopped the loop
     int max_iter;      // 0 = unlimited
     int stop_rule;     // 0: EGG local sync + extra check; 1: r_c >= lam
@@ -155,7 +164,6 @@ struct DevState {
     int G;             // cell groups of the update tiles
     int S;             // non-empty sub-cells
     int sparse_count;  // runs of sparse cell groups (k_update_pairs)
-    int WS;            // sub-cell summary work items
     double rc;         // order parameter of the last r_c evaluation
     // heavy streamed ranges of the update (k_update_heavy): descriptors
     // created (high 32 bits) and work units allocated (low 32 bits), the
@@ -165,7 +173,7 @@ struct DevState {
     int ndt;
     int ptile_next;    // work-queue head of the pair update (k_update_pairs)
     // run_start[0 .. runs] describes runs of bitwise-equal positions in the
-    // current order of the positions (set by k_runs; an update moves every
+    // current order of the positions (set by k_tables; an update moves every
     // point of a run alike, so the runs survive it and the next grid build
     // sorts runs instead of points)
     int runs_valid;

@@ -5,52 +5,36 @@
 
 namespace egg {
 
-// Exclusive scan of n int32 values (n_dev, if given, overrides n at run time;
-// it must not exceed n).  `tmp` needs scan_tmp_ints(n) ints.  The sum of all
-// values is written to *total if total != nullptr.  In-place allowed.
-// With `lookback`, arrays of more than one tile are scanned in one launch
-// (decoupled look-back); tmp then holds the scans' shared state and must be
-// zero before the first such scan (scan_tmp_reset) -- each scan leaves it
-// ready for the next on the same stream.
+// Exclusive scan of n int32 values; `tmp` needs scan_tmp_ints(n) ints.  The
+// sum of all values is written to *total if total != nullptr.  In-place allowed.
 size_t scan_tmp_ints(int n);
-void scan_exclusive(const int *in, int *out, int n, const int *n_dev, int *tmp, int *total,
-                    const DevState *st, hipStream_t s, bool lookback = false);
-// Zeroes the look-back state in tmp (scan_tmp_ints(n) ints); not for graph capture.
+void scan_exclusive(const int *in, int *out, int n, int *tmp, int *total, hipStream_t s);
+// The grid build's scans (egg_scan.h) keep their shared state, up to
+// kMaxScanCh channels, in scan_tmp_ints(n) ints of their own.  It must be zero
+// before the first of them (scan_tmp_reset, not for graph capture); each scan
+// leaves it ready for the next on the same stream.
+constexpr int kMaxScanCh = 4;
 int scan_tmp_reset(int *tmp, int n, hipStream_t s);
-// Nonzero if a look-back scan using tmp gave up waiting (an internal error).
+// Nonzero if a scan using tmp gave up waiting (an internal error).
 int scan_tmp_error(const int *tmp, hipStream_t s, int *err);
 
-// Exclusive scans of nch (<= kMaxScanCh) int32 arrays of the same length in
-// one pass: channel c scans in[c] into out[c] (in place allowed) and writes
-// its sum to *total[c] if that is not null.
-constexpr int kMaxScanCh = 4;
-struct ScanSet {
-    const int *in[kMaxScanCh];
-    int *out[kMaxScanCh];
-    int *total[kMaxScanCh];
-};
-void scan_exclusive_multi(const ScanSet &ss, int nch, int n, const int *n_dev, int *tmp,
-                          const DevState *st, hipStream_t s, bool lookback = false);
-
-// The same stable order from one workgroup comparing every pair of the first
-// *n_dev keys (for a few hundred keys, where the radix passes' launches
-// dominate); the result is in the *_b buffers (returns 1).
-constexpr int kSmallSortRuns = 1024;
-int small_sort(const uint64_t *keys_a, uint64_t *keys_b, int *vals_b, int n, int kw,
-               const int *n_dev, const DevState *st, hipStream_t s);
+// Stable order of the grid build's keys, st->sort_m <= kRankSortMax of them, by
+// comparing every pair: sorted position q holds element sidx[q]; for runs of the
+// previous grid (st->lens_m > 0) also where their points go (off, src).
+constexpr int kRankSortMax = 24576;
+void rank_sort(const uint64_t *keys, int *sidx, int n, int kw, const int *run_start, int *off,
+               int *src, const DevState *st, const DevState *st_loop, hipStream_t s);
 
 // Stable LSD radix sort of (key, position) pairs by key bits [0, key_bits),
 // 8 bits per pass.  keys_a/keys_b: [kw][n] u64; vals_a/vals_b: [n] int32.
-// On entry keys are in keys_a and vals are implicit (0..m-1); m = *n_dev
-// (<= n) if n_dev is given, else n.  With n_dev, *hist_n_dev must hold
-// 256 * max(1, ceil(m / kSortTile)) (the histogram entries of the tiles that
-// hold elements).  Returns 0 if the sorted result is in the *_a buffers, 1 if
+// On entry keys are in keys_a and vals are implicit (0..m-1), m = *n_dev
+// (<= n); *hist_n_dev must hold 256 * max(1, ceil(m / kSortTile)) (the
+// histogram entries of the tiles that hold elements).  Returns 0 if the sorted result is in the *_a buffers, 1 if
 // in *_b, -1 if no pass was needed (identity order).
 size_t sort_tmp_ints(int n);
 int radix_sort(uint64_t *keys_a, uint64_t *keys_b, int *vals_a, int *vals_b, int n, int kw,
                int key_bits, int *hist, int *scan_tmp, const DevState *st, hipStream_t s,
-               bool lookback = false, const int *n_dev = nullptr,
-               const int *hist_n_dev = nullptr);
+               const int *n_dev, const int *hist_n_dev);
 
 // A heavy streamed range of an update tile: tile t, candidate cell c, the
 // range's runs (runs [r0, r0 + total) if smask is 0, else the runs of
@@ -73,43 +57,39 @@ struct GridBufs {
     int *vals_a, *vals_b;
     int *hist;           // [256][ntiles]
     int *scan_tmp;
-    int *head, *hpos;    // [n] cell-head flags of the sorted positions and their scan
     int *point_cell;     // [n]
+    int *point_run;      // [n] run and sub-cell of each sorted position
+    int *point_sub;      // [n]
+    int *run_off;        // [n] sorted runs of the previous grid: first new position,
+    int *run_src;        // [n] first old position
+    int *scratch;        // [n] of the label passes
     int *cell_start;     // [n+1]
     int *cell_g;         // [d][n]
     int *cell_outer;     // [n]
     int *ob, *oe;        // [O]
-    int *nchunk, *wi_off;// [n]
-    // runs: maximal stretches of bitwise-equal consecutive positions (sorted
-    // order); rhead / rpos are their head flags and the flags' scan
-    int *rhead, *rpos;   // [n]
+    // runs: maximal stretches of bitwise-equal consecutive positions (sorted order)
     int *run_start;      // [n+1] first sorted position of each run
     int *cell_run;       // [n+1] first run of each cell
-    // sub-cells (see cell_mid): shead / spos head flags and their scan,
-    // first sorted position, first sub-cell of each cell, fine coordinates
-    // 2g + split bit, first run, totals as Ts / Tc, summary work items
-    int *shead, *spos;   // [n]
+    // sub-cells (see cell_mid): first sorted position, first sub-cell of each
+    // cell, fine coordinates 2g + split bit, first run, totals as Ts / Tc
     int *sub_start;      // [n+1]
     int *cell_sub;       // [n+1]
     int *sub_g;          // [d][n]
     int *sub_run;        // [n+1]
     float *TsS, *TcS;    // [d][n]
     unsigned *smin, *smax;  // [d][n] bounding box of each sub-cell's points (ord_key)
-    int *snchunk, *swi_off; // [n]
     // update tiles: cells are grouped (consecutive cells of one outer cell,
     // equal inner coordinates but the last, last one in the same block of gw
     // cells); a tile holds <= 64 runs of one group
-    int *gflag, *gpos;   // [n] group-head flag of each cell and its exclusive scan
     int *grp_cell;       // [n+1] first cell of each group, grp_cell[G] = C
-    int *ntile, *tile_off;// [n]  tiles per group, exclusive scan (every group: extra check)
-    int *untile, *utile_off;// [n] the same for the groups of k_update_tile (not sparse)
+    int *tile_off;       // [n] first tile of each group (every group: extra check)
+    int *utile_off;      // [n] the same for the groups of k_update_tile (not sparse)
     float *rres;         // [d][n] new position of each run
     int *sparse_runs;    // [n]   runs of sparse cell groups
     // pair update (egg_pairs.hip): memory of its own (pair_scratch_bytes); it
     // also uses keys_a / keys_b and partial, free between the summaries and the
     // next grid build
     char *pair;
-    int *sparse_off;     // [n]   their offsets per group (exclusive scan)
     int *rdbg;           // [4n]  N / half / border / synced of each run (diagnostics;
                          //       also the saved N / half / border of deferred runs)
     // heavy streamed ranges (k_update_heavy): their sums, per run, in
@@ -119,7 +99,7 @@ struct GridBufs {
     HeavyDesc *hdesc;    // [kHeavyCap]
     int *dtiles;         // [n]   tiles whose runs finish in k_update_finish
     float *Ts, *Tc;      // [d][n]
-    float *partial;      // [n + n/kSumChunk + 1][4*d]
+    float *partial;      // [n + n/kSumChunk + 1][4*d]: summary partials, see summary_slot
     int *pairs;          // [2 * pair_cap] extra-check (p, q) sorted positions
     int pair_cap;
 };
@@ -127,11 +107,13 @@ struct GridBufs {
 void launch_aos_to_soa(const float *aos, float *soa, int *perm, int n, int d, hipStream_t s);
 void launch_soa_to_aos_by_perm(const float *soa, const int *perm, float *aos, int n, int d,
                                hipStream_t s);
-void launch_fill(int *p, int count, int v, const DevState *st, hipStream_t s);
-// keys + sort + gather + cells + outer ranges.  Writes st->C.
-// small: the previous grid holds at most kSmallSortRuns runs (small_sort).
+// Sort and grid tables; writes st->C.  st_loop (nullable): nothing runs once
+// its loop has stopped; with `begin` the build opens a loop iteration (the pass
+// state is reset).  keep_runs: the update moves each run of equal positions
+// alike, so the next build may sort runs.  small: at most kRankSortMax elements
+// to sort (rank_sort).
 void build_grid(const Geo &g, GridBufs &b, DevState *st_loop, DevState *st, hipStream_t s,
-                bool small = false);
+                bool keep_runs, bool small = false, bool begin = false);
 void cell_summaries(const Geo &g, GridBufs &b, DevState *st_loop, DevState *st, hipStream_t s);
 
 // Update / extra check / r_c (egg_update.hip).
@@ -152,10 +134,8 @@ void launch_set_flag(DevState *st, hipStream_t s);
 void launch_finish(DevState *st, hipStream_t s);
 
 // Labels (egg_labels.hip).
-void launch_labels_egg(const Geo &g, GridBufs &b, int *labels, int *multi, int *lab_off,
-                       DevState *st, hipStream_t s);
-void launch_labels_sync(const Geo &g, GridBufs &b, int *labels, int *invperm, DevState *st,
-                        hipStream_t s);
+void launch_labels_egg(const Geo &g, GridBufs &b, int *labels, DevState *st, hipStream_t s);
+void launch_labels_sync(const Geo &g, GridBufs &b, int *labels, DevState *st, hipStream_t s);
 void launch_validate(const float *aos, long long count, int *err, hipStream_t s);
 
 }  // namespace egg

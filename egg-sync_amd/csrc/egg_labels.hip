@@ -4,6 +4,7 @@
 
 #include "egg_candidates.h"
 #include "egg_internal.h"
+#include "egg_scan.h"
 
 namespace egg {
 
@@ -14,31 +15,35 @@ static inline int grid_for(long long n) {
     return (int)b;
 }
 
-__global__ void k_label_flags(const int *__restrict__ cell_start, const DevState *st,
-                              int *__restrict__ multi) {
-    const int C = st->C;
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < C; c += gridDim.x * blockDim.x)
-        multi[c] = (cell_start[c + 1] - cell_start[c]) > 1 ? 1 : 0;
-}
+// Cluster id of each cell with more than one point (the scan of such cells), -1
+// for the others.
+struct LabelScan {
+    const int *cell_start;
+    int *label;
+    DevState *st;
+    __device__ int count() const { return st->C; }
+    __device__ void load(int c, int (&v)[1]) const {
+        v[0] = cell_start[c + 1] - cell_start[c] > 1 ? 1 : 0;
+    }
+    __device__ void store(int c, const int (&v)[1], const int (&ex)[1]) const {
+        label[c] = v[0] ? ex[0] : -1;
+    }
+    __device__ void finish(const int (&tot)[1]) const { st->n_clusters = tot[0]; }
+};
 
 // GPU_synCluster_float_grid: a point gets its cell's cluster id when the cell
 // holds more than one point, else -1.  Ids are compacted to 0..k-1 in cell
 // order (the reference leaves gaps; only the partition is meaningful).
-__global__ void k_labels_egg(const int *__restrict__ point_cell, const int *__restrict__ multi,
-                             const int *__restrict__ lab_off, const int *__restrict__ perm_s,
+__global__ void k_labels_egg(const int *__restrict__ point_cell,
+                             const int *__restrict__ cell_label, const int *__restrict__ perm_s,
                              int n, int *__restrict__ labels) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const int c = point_cell[i];
-        labels[perm_s[i]] = multi[c] ? lab_off[c] : -1;
-    }
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+        labels[perm_s[i]] = cell_label[point_cell[i]];
 }
 
-void launch_labels_egg(const Geo &g, GridBufs &b, int *labels, int *multi, int *lab_off,
-                       DevState *st, hipStream_t s) {
-    const int gb = grid_for(g.n);
-    k_label_flags<<<gb, kBlock, 0, s>>>(b.cell_start, st, multi);
-    scan_exclusive(multi, lab_off, g.n, &st->C, b.scan_tmp, &st->n_clusters, nullptr, s, true);
-    k_labels_egg<<<gb, kBlock, 0, s>>>(b.point_cell, multi, lab_off, b.perm_s, g.n, labels);
+void launch_labels_egg(const Geo &g, GridBufs &b, int *labels, DevState *st, hipStream_t s) {
+    launch_scan<1>(LabelScan{b.cell_start, b.scratch, st}, g.n, b.scan_tmp, nullptr, s);
+    k_labels_egg<<<grid_for(g.n), kBlock, 0, s>>>(b.point_cell, b.scratch, b.perm_s, g.n, labels);
 }
 
 __global__ void k_invert(const int *__restrict__ perm_s, int n, int *__restrict__ inv) {
@@ -154,8 +159,8 @@ __global__ __launch_bounds__(kLabBlock) void k_labels_sync(
     if (t == 0) st->n_clusters = cl;
 }
 
-void launch_labels_sync(const Geo &g, GridBufs &b, int *labels, int *invperm, DevState *st,
-                        hipStream_t s) {
+void launch_labels_sync(const Geo &g, GridBufs &b, int *labels, DevState *st, hipStream_t s) {
+    int *invperm = b.scratch;
     k_invert<<<grid_for(g.n), kBlock, 0, s>>>(b.perm_s, g.n, invperm);
 #define LS_CASE(DD)                                                                           \
     case DD:                                                                                  \

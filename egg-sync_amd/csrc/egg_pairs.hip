@@ -672,7 +672,7 @@ void launch_update_pairs(const Geo &g, GridBufs &b, int *rdbg, DevState *st, hip
 #define PAIR_LAUNCH(DD, SMALL)                                                                \
     k_update_pairs<DD, SMALL><<<pq, kBlock, 0, s>>>(                                          \
         b.Xs, b.cell_start, b.cell_g, b.run_start, b.point_cell, b.cell_run,                  \
-        g.pair_mode == kPairAll ? nullptr : b.sparse_runs, data, bounds, b.rres, rdbg, g, st)
+        pairs_take_all(g.pair_mode, g.d) ? nullptr : b.sparse_runs, data, bounds, b.rres, rdbg, g, st)
 #define PAIR_CASE(DD)                                                                          \
     case DD:                                                                                   \
         k_run_boxes<DD><<<pb, kBlock, 0, s>>>(b.Xs, b.run_start, b.point_cell, b.cell_run,     \

@@ -133,7 +133,6 @@ struct Layout {
     double *rc_part = nullptr;
     double *rc_trace = nullptr;
     int *cells_trace = nullptr;
-    int *it_before = nullptr;
     int *err = nullptr;
     size_t bytes = 0;
 };
@@ -154,22 +153,19 @@ Layout carve(void *base, const Geo &g) {
     const size_t hist = sort_tmp_ints(g.n);
     b.hist = c.take<int>(hist);
     b.scan_tmp = c.take<int>(scan_tmp_ints((int)std::max(n, hist)) + 16);
-    b.head = c.take<int>(n);
-    b.hpos = c.take<int>(n);
     b.point_cell = c.take<int>(n);
+    b.point_run = c.take<int>(n);
+    b.point_sub = c.take<int>(n);
+    b.run_off = c.take<int>(n);
+    b.run_src = c.take<int>(n);
+    b.scratch = c.take<int>(n);
     b.cell_start = c.take<int>(n + 1);
     b.cell_g = c.take<int>(n * d);
     b.cell_outer = c.take<int>(n);
     b.ob = c.take<int>((size_t)g.O);
     b.oe = c.take<int>((size_t)g.O);
-    b.nchunk = c.take<int>(n);
-    b.wi_off = c.take<int>(n);
-    b.rhead = c.take<int>(n);
-    b.rpos = c.take<int>(n);
     b.run_start = c.take<int>(n + 1);
     b.cell_run = c.take<int>(n + 1);
-    b.shead = c.take<int>(n);
-    b.spos = c.take<int>(n);
     b.sub_start = c.take<int>(n + 1);
     b.cell_sub = c.take<int>(n + 1);
     b.sub_g = c.take<int>(n * d);
@@ -178,19 +174,12 @@ Layout carve(void *base, const Geo &g) {
     b.TcS = c.take<float>(n * d);
     b.smin = c.take<unsigned>(n * d);
     b.smax = c.take<unsigned>(n * d);
-    b.snchunk = c.take<int>(n);
-    b.swi_off = c.take<int>(n);
-    b.gflag = c.take<int>(n);
-    b.gpos = c.take<int>(n);
     b.grp_cell = c.take<int>(n + 1);
-    b.ntile = c.take<int>(n);
     b.tile_off = c.take<int>(n);
-    b.untile = c.take<int>(n);
     b.utile_off = c.take<int>(n);
     b.rres = c.take<float>(n * d);
     b.sparse_runs = c.take<int>(n);
     b.pair = c.take<char>(pair_scratch_bytes(n, d));
-    b.sparse_off = c.take<int>(n);
     b.rdbg = c.take<int>(4 * n);
     b.hacc = g.d <= kHeavyMaxD ? c.take<long long>((2 * d + 2) * n) : nullptr;
     b.hdesc = c.take<HeavyDesc>(kHeavyCap);
@@ -206,8 +195,12 @@ Layout carve(void *base, const Geo &g) {
     L.rc_part = c.take<double>((size_t)rc_partials(g.n));
     L.rc_trace = c.take<double>(kTraceCap);
     L.cells_trace = c.take<int>(kTraceCap);
-    L.it_before = c.take<int>(1);
     L.err = c.take<int>(1);
+    // room the solve does not use, so that the size of a workspace, and with it the
+    // largest n the fixed scratch array holds, stays what callers have sized for
+    const size_t wide = (std::max(n, hist) + kScanTile - 1) / kScanTile + 1;
+    c.off += 10 * align_up(4 * n) + align_up(4) + align_up(4 * (8 * wide + 20)) -
+             align_up(4 * (scan_tmp_ints((int)std::max(n, hist)) + 16));
     L.bytes = c.off;
     return L;
 }
@@ -328,23 +321,15 @@ __global__ void k_features(const float *__restrict__ Xs, const int *__restrict__
 }
 
 // End of a loop iteration: finish_iteration, then record r_c and C of the
-// iteration that just ran.
-__global__ void k_iter_end(DevState *st, const int *it_before, double *rc_trace,
-                           int *cells_trace, int cap) {
-    if (!st->done) finish_iteration(st);
+// iteration that just ran (nothing once the loop has stopped).
+__global__ void k_iter_end(DevState *st, double *rc_trace, int *cells_trace, int cap) {
+    if (st->done) return;
+    finish_iteration(st);
     const int it = st->iter;
-    if (it == *it_before) return;  // the loop had already stopped
     if (it >= 1 && it <= cap) {
         rc_trace[it - 1] = st->rc;
         cells_trace[it - 1] = st->C;
     }
-}
-
-// Start of a loop iteration: the iteration count before it, then the pass
-// state reset (nothing once the loop has stopped).
-__global__ void k_iter_begin(DevState *st, int *it_before) {
-    *it_before = st->iter;
-    if (!st->done) reset_pass_state(st);
 }
 
 int grid_blocks(long long n) {
@@ -424,13 +409,12 @@ double ms_between(hipEvent_t a, hipEvent_t b) {
 }
 
 // One pass of the loop body (EGG_SynC.cu:1323-1491), fully on the device.
-// small: the grid holds at most kSmallSortRuns runs (the grid build sorts
-// them in one launch).
+// small: at most kRankSortMax elements to sort (the grid build sorts them in
+// one launch).
 void enqueue_iteration(const Geo &g, Layout &L, const egg_sync_options &opt, hipStream_t s,
                        hipEvent_t *ev, bool small = false) {
     if (ev) (void)hipEventRecord(ev[0], s);
-    k_iter_begin<<<1, 1, 0, s>>>(L.st, L.it_before);
-    build_grid(g, L.b, L.st, L.st, s, small);
+    build_grid(g, L.b, L.st, L.st, s, opt.stop_rule == EGG_SYNC_STOP_EGG, small, true);
     if (opt.stop_rule == EGG_SYNC_STOP_EGG) cell_summaries(g, L.b, L.st, L.st, s);
     if (ev) (void)hipEventRecord(ev[1], s);
     if (opt.stop_rule == EGG_SYNC_STOP_EGG) {
@@ -441,7 +425,7 @@ void enqueue_iteration(const Geo &g, Layout &L, const egg_sync_options &opt, hip
         launch_update_sync(g, L.b, L.st, L.rc_part, true, s);
         if (ev) (void)hipEventRecord(ev[2], s);
     }
-    k_iter_end<<<1, 1, 0, s>>>(L.st, L.it_before, L.rc_trace, L.cells_trace, kTraceCap);
+    k_iter_end<<<1, 1, 0, s>>>(L.st, L.rc_trace, L.cells_trace, kTraceCap);
     if (ev) (void)hipEventRecord(ev[3], s);
 }
 
@@ -555,9 +539,9 @@ int solve_device_impl(const float *d_D, int64_t n64, int d, float eps,
     }
     double st_build = 0, st_upd = 0, st_extra = 0;
     int done_iters = 0;
-    // runs only merge, so once a state read shows at most kSmallSortRuns
-    // valid runs, every later grid build may sort them in one launch
-    bool small = false;
+    // runs only merge, so once a state read shows at most kRankSortMax valid
+    // runs, every later grid build may sort them in one launch
+    bool small = n <= kRankSortMax;
     auto ensure_graph = [&]() -> int {
         if (!opt.use_graph) return 0;
         std::vector<char> key;
@@ -613,9 +597,8 @@ int solve_device_impl(const float *d_D, int64_t n64, int d, float eps,
         }
         done_iters = h_state->iter;
         if (h_state->done) break;
-        const bool want = h_state->runs_valid && h_state->runs <= kSmallSortRuns;
-        if (want != small) {
-            small = want;
+        if (!small && h_state->runs_valid && h_state->runs <= kRankSortMax) {
+            small = true;
             rc = ensure_graph();
             if (rc) return rc;
         }
@@ -625,13 +608,13 @@ int solve_device_impl(const float *d_D, int64_t n64, int d, float eps,
     // final grid on the converged positions and labels (EGG_SynC.cu:1504-1541)
     hipEvent_t *fe = opt.timing ? &E.ev[4 * K] : nullptr;
     if (fe) (void)hipEventRecord(fe[0], s);
-    build_grid(g, L.b, nullptr, L.st, s,
-               loop_state.runs_valid && loop_state.runs <= kSmallSortRuns);
+    small = small || (loop_state.runs_valid && loop_state.runs <= kRankSortMax);
+    build_grid(g, L.b, nullptr, L.st, s, false, small);
     int *labels_dev = d_labels ? d_labels : L.labels;
     if (opt.label_rule == EGG_SYNC_LABELS_CELLS)
-        launch_labels_egg(g, L.b, labels_dev, L.b.nchunk, L.b.wi_off, L.st, s);
+        launch_labels_egg(g, L.b, labels_dev, L.st, s);
     else
-        launch_labels_sync(g, L.b, labels_dev, L.b.head, L.st, s);
+        launch_labels_sync(g, L.b, labels_dev, L.st, s);
     if (opt.compute_rc && opt.stop_rule == EGG_SYNC_STOP_EGG)
         launch_update_sync(g, L.b, L.st, L.rc_part, false, s);
     if (fe) (void)hipEventRecord(fe[1], s);
@@ -907,9 +890,10 @@ int solve_batch_impl(const float *d_D, const egg_sync_instance *inst, int n_inst
     // instances still iterating; finished ones are no longer enqueued
     std::vector<char> live(n_inst, 0);
     for (int k : active) live[k] = 1;
-    // instances whose grid holds at most kSmallSortRuns runs (plain launches
-    // only: a captured graph keeps the radix sort)
+    // instances with at most kRankSortMax elements to sort (for captured graphs
+    // by their points only: a graph keeps the sort it was captured with)
     std::vector<char> small(n_inst, 0);
+    for (int k : active) small[k] = G[k].n <= kRankSortMax;
     auto enqueue_batch = [&](hipStream_t origin) -> int {
         int r = fork_streams(bw, origin, S);
         if (r) return r;
@@ -990,7 +974,7 @@ int solve_batch_impl(const float *d_D, const egg_sync_instance *inst, int n_inst
             live[k] = !hk.done;
             n_live += live[k];
             max_iter_seen = std::max(max_iter_seen, hk.iter);
-            if (!opt.use_graph) small[k] = hk.runs_valid && hk.runs <= kSmallSortRuns;
+            if (!opt.use_graph && hk.runs_valid && hk.runs <= kRankSortMax) small[k] = 1;
         }
         if (n_live == 0) break;
         if (opt.use_graph && n_live != graph_live) {
@@ -1007,12 +991,13 @@ int solve_batch_impl(const float *d_D, const egg_sync_instance *inst, int n_inst
         for (int k : per[j]) {
             Layout &L = Ls[k];
             const DevState &hk = bw.h_states[k];
-            build_grid(G[k], L.b, nullptr, L.st, sj, hk.runs_valid && hk.runs <= kSmallSortRuns);
+            build_grid(G[k], L.b, nullptr, L.st, sj, false,
+                       small[k] || (hk.runs_valid && hk.runs <= kRankSortMax));
             int32_t *lab = d_labels + row_off[k];
             if (opt.label_rule == EGG_SYNC_LABELS_CELLS)
-                launch_labels_egg(G[k], L.b, lab, L.b.nchunk, L.b.wi_off, L.st, sj);
+                launch_labels_egg(G[k], L.b, lab, L.st, sj);
             else
-                launch_labels_sync(G[k], L.b, lab, L.b.head, L.st, sj);
+                launch_labels_sync(G[k], L.b, lab, L.st, sj);
             if (opt.compute_rc && opt.stop_rule == EGG_SYNC_STOP_EGG)
                 launch_update_sync(G[k], L.b, L.st, L.rc_part, false, sj);
             if (d_final)
@@ -1139,7 +1124,7 @@ int egg_sync_build_grid_device(const float *d_D, int64_t n, int32_t d, float eps
     hipStream_t s;
     int rc = setup_single(d_D, n, d, eps, d_order_in, g, L, s, stream);
     if (rc) return rc;
-    build_grid(g, L.b, nullptr, L.st, s);
+    build_grid(g, L.b, nullptr, L.st, s, false, g.n <= kRankSortMax);
     const size_t nn = (size_t)g.n;
     if (d_order_out)
         HIP_TRY(hipMemcpyAsync(d_order_out, L.b.perm_s, 4 * nn, hipMemcpyDeviceToDevice, s));
@@ -1172,7 +1157,7 @@ int egg_sync_iteration_device(const float *d_D, int64_t n, int32_t d, float eps,
     if (rc) return rc;
     DebugOut dbg{d_N, d_half, d_border, d_synced};
     launch_set_flag(L.st, s);
-    build_grid(g, L.b, L.st, L.st, s);
+    build_grid(g, L.b, L.st, L.st, s, true, g.n <= kRankSortMax);
     cell_summaries(g, L.b, L.st, L.st, s);
     launch_update_egg(g, L.b, L.st, &dbg, s);
     launch_extra_check(g, L.b, L.st, s);
@@ -1197,7 +1182,7 @@ int egg_sync_features_device(const float *d_D, const float *d_prev, int64_t n, i
     hipStream_t s;
     int rc = setup_single(d_D, n, d, eps, nullptr, g, L, s, stream);
     if (rc) return rc;
-    build_grid(g, L.b, nullptr, L.st, s);
+    build_grid(g, L.b, nullptr, L.st, s, false, g.n <= kRankSortMax);
     cell_summaries(g, L.b, nullptr, L.st, s);
     k_features<<<grid_blocks(g.n), kBlock, 0, s>>>(L.b.Xs, L.b.perm_s, L.b.point_cell,
                                                    L.b.cell_start, L.b.Ts, L.b.Tc, d_prev, g.n, d,
@@ -1215,7 +1200,7 @@ int egg_sync_rc_device(const float *d_D, int64_t n, int32_t d, float eps, double
     hipStream_t s;
     int rc = setup_single(d_D, n, d, eps, nullptr, g, L, s, stream);
     if (rc) return rc;
-    build_grid(g, L.b, nullptr, L.st, s);
+    build_grid(g, L.b, nullptr, L.st, s, false, g.n <= kRankSortMax);
     launch_update_sync(g, L.b, L.st, L.rc_part, false, s);
     DevState hs;
     HIP_TRY(hipMemcpyAsync(&hs, L.st, sizeof hs, hipMemcpyDeviceToHost, s));

@@ -1030,10 +1030,10 @@ __global__ __launch_bounds__(kBlock) void k_update_finish(
 }
 
 // Every point takes its run's result and carries its id over to the next
-// iteration's order.  The run of sorted position i is rpos[i] + rhead[i] - 1.
+// iteration's order.
 template <int D>
 __global__ __launch_bounds__(kBlock) void k_scatter_runs(
-    const int *__restrict__ rhead, const int *__restrict__ rpos, const float *__restrict__ rres,
+    const int *__restrict__ point_run, const float *__restrict__ rres,
     const int *__restrict__ rdbg, const int *__restrict__ perm_s, float *__restrict__ Xout,
     int *__restrict__ perm_out, int n, DevState *st, DebugOut dbg) {
     if (st->done) return;
@@ -1041,7 +1041,7 @@ __global__ __launch_bounds__(kBlock) void k_scatter_runs(
     if (blockIdx.x == 0 && threadIdx.x == 0) st->flag_local = st->flag;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         perm_out[i] = perm_s[i];
-        const int r = rpos[i] + rhead[i] - 1;
+        const int r = point_run[i];
 #pragma unroll
         for (int l = 0; l < D; l++) Xout[(long long)l * n + i] = rres[(long long)l * n + r];
         if (rdbg) {
@@ -1504,7 +1504,7 @@ void launch_update_egg(const Geo &g, GridBufs &b, DevState *st, const DebugOut *
                                                   b.rres, rdbg, g, st);                       \
         }                                                                                     \
         launch_update_pairs(g, b, rdbg, st, s);                                               \
-        k_scatter_runs<DD><<<grid_for(g.n), kBlock, 0, s>>>(b.rhead, b.rpos, b.rres, rdbg,   \
+        k_scatter_runs<DD><<<grid_for(g.n), kBlock, 0, s>>>(b.point_run, b.rres, rdbg,       \
                                                             b.perm_s, b.X, b.perm, g.n, st,   \
                                                             d);                               \
         break;

@@ -504,3 +504,44 @@ def test_pair_update_at_batch_edges(S, O, d):
             a = S.solve(X, eps, max_iter=1, pair_groups=2)
             b = O.egg_iteration(X, eps)
             assert np.abs(a["X"] - b["X_next"]).max() <= 1e-6, (n, eps)
+
+
+@pytest.mark.parametrize("d", [1, 2, 3, 9])
+def test_grid_build_at_tile_edges(S, O, d):
+    """The grid build and the summaries at the remainders of their wavefronts (64), tiles (512) and
+    of the sort by comparison (24,576), with cells of 31 to 513 points (the summaries' windows
+    of 32 and chunks of 256) and bitwise-equal points: one pass, bit for bit in its counts and flags and
+    within 1e-6 in its positions, as in test_iteration_bit_exact; and a second pass, which sorts
+    the runs of the first, equal in every bit to a pass that sorts the points."""
+    rng = np.random.default_rng(90 + d)
+    eps = 0.05 * np.sqrt(d)
+    for n in (1, 2, 63, 64, 65, 511, 512, 513, 1025, 3000, 24576, 24577):
+        X = rng.random((n, d)).astype(f32)
+        if n >= 3000:
+            at = 0
+            for k, size in enumerate((31, 32, 33, 64, 65, 255, 256, 257, 513)):
+                X[at:at + size] = (0.05 + 0.1 * k + 1e-4 * rng.random((size, d))).astype(f32)
+                at += size
+            X[at:at + 300] = X[at]
+        X = X[rng.permutation(n)]
+        _say("grid build", n, d)
+        a = S.iteration(X, eps)
+        b = O.egg_iteration(X, eps)
+        for k in ("order", "N", "half", "border", "synced"):
+            assert np.array_equal(a[k], b[k]), (n, k)
+        assert np.abs(a["X_next"] - b["X_next"]).max() <= 1e-6, n
+        two = S.iteration(a["X_next"], eps, a["order"])
+        assert np.array_equal(S.solve(X, eps, max_iter=2)["X"],
+                              two["X_next"] if not a["flag_final"] else a["X_next"]), n
+
+
+def test_grid_tables_on_both_sides_of_the_wide_tiles(S, O):
+    """Grids of 2^18 points and one more, where the tiles of the tables grow."""
+    rng = np.random.default_rng(95)
+    for n in (1 << 18, (1 << 18) + 1):
+        X = rng.random((n, 2)).astype(f32)
+        _say("grid tables", n)
+        a, b = S.build_grid(X, 0.02), O.build_grid(X, 0.02)
+        assert a["C"] == b["C"]
+        for k in ("order", "cell_of", "cell_start", "cell_g", "ob", "oe"):
+            assert np.array_equal(a[k], b[k]), (n, k)
