@@ -13,14 +13,16 @@
 // reference), pruned in the remaining dimensions to |dg| <= R+1 by a binary
 // search over the column's cells (sorted by g_od): cells farther than that
 // fail the reference's box test by more than a cell side, so results do not
-// change.  Up to d = 3 the masked sums over streamed runs run on the matrix
-// cores (stream_chunk_mfma), in the same order of FP32 additions.
+// change.  Up to kStreamMaxD dimensions the tests and masked sums over streamed runs
+// run on the matrix cores (egg_stream.h), in the same order of FP32 additions.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "egg_candidates.h"
 #include "egg_internal.h"
-#include "egg_wave.h"
+#include "egg_scan.h"
+#include "egg_stream.h"
 
 namespace egg {
 
@@ -296,134 +298,36 @@ __device__ __forceinline__ int stream_total(int r0, int r1, int s0, unsigned sma
     return total;
 }
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+// Calls f(a, b) for the maximal stretches of runs [a, b) of a streamed range, in
+// order.
+template <typename Fn>
+__device__ __forceinline__ void each_stretch(int r0, int r1, int s0, unsigned smask,
+                                             const int *__restrict__ sub_run, Fn &&f) {
+    if (!smask) {
+        f(r0, r1);
+        return;
+    }
+    for (unsigned long long mm = smask; mm;) {
+        const int k = __builtin_ctzll(mm), len = __builtin_ctzll(~(mm >> k));
+        f(__builtin_amdgcn_readfirstlane(sub_run[s0 + k]),
+          __builtin_amdgcn_readfirstlane(sub_run[s0 + k + len]));
+        mm &= ~(((1ull << len) - 1) << k);
+    }
+}
 
-// stream_chunk for d <= 3 with the masked sums on the matrix cores.  Each
-// source q is one step: the lanes test it against eps (the same FP32
-// distance as below), and two v_mfma_f32_4x4x1_16b add the row
-// [w sv_0..2 | w | w cv_0..2 | 0] of q (w = run length) times each lane's
-// 0/1 test result into 64 x 8 accumulators (16 blocks of 4 targets x 4
-// columns per instruction: block b holds targets 4(b&7)+i, +32 in the second
-// instruction, and columns 4(b>>3)+j; lane l supplies row l&3 of block l>>2's
-// A and column l&3 of its B, and holds that block's rows 0-3 of column l&3 in
-// its four result registers).  K = 1, so every accumulator takes one
-// FP32 add per source, of the value or of 0, in source order: the sums are
-// those of the scalar loop below bit for bit, the VALU is spared the six
-// masked adds and the count per source.  A lane's sums enter the accumulator
-// layout through LDS before the chunk and leave it after.  The count column
-// is exact while a chunk's count stays below 2^24, hence n < 2^24.
+// Notes runs [lo, hi) of a streamed range (counted from its start, at most 17
+// stretches) for the lanes of mask.
 template <int D>
-__device__ __forceinline__ void stream_chunk_mfma(int base, int total, int r0, int s0,
-                                                  unsigned smask, const int *__restrict__ sub_run,
-                                                  const int *__restrict__ run_start,
-                                                  const float *__restrict__ Xs, int n,
-                                                  const float (&a0)[D], const float (&x)[D],
-                                                  float thr, bool acc, SrcPt<D> *src,
-                                                  float (&ssv)[D], float (&scm)[D], int &m_part) {
-    static_assert(D <= 3 && SrcPt<D>::P == 4, "row of a source: sv[0..3] then cv[0..3]");
-    const int lane = __lane_id();
-    // 64 x 8 transpose buffer inside src, rows of kTr = 9 floats: an odd
-    // stride puts a row-wise access of 32 lanes in 32 different banks, and
-    // the accumulator-layout access too (9 * 4k + j covers 0..31 mod 32)
-    constexpr int kTr = 9;
-    static_assert(kWave * kTr <= kWave * (int)(sizeof(SrcPt<D>) / sizeof(float)), "T fits in src");
-    float *T = reinterpret_cast<float *>(src);
-    // the accumulators this lane holds: targets tc + r (and 32 + tc + r), column cc
-    const int tc = lane & 28, cc = 4 * (lane >> 5) + (lane & 3);
-#pragma unroll
-    for (int l = 0; l < 4; l++) {
-        T[lane * kTr + l] = l < D ? ssv[l] : 0.f;
-        T[lane * kTr + 4 + l] = l < D ? scm[l] : 0.f;
-    }
-    T[lane * kTr + 3] = 0.f;  // count column: this chunk's count only
-    wave_sync();
-    f32x4 d1, d2;
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        d1[r] = T[(tc + r) * kTr + cc];
-        d2[r] = T[(32 + tc + r) * kTr + cc];
-    }
-    wave_sync();
-    const int rr = stream_run(base + lane, total, r0, s0, smask, sub_run);
-    if (rr >= 0) {
-        const int j = run_start[rr];
-        const float w = (float)(run_start[rr + 1] - j);  // exact: < 2^24
-        float sv[D], cv[D];
-#pragma unroll
-        for (int l = 0; l < D; l++) {
-            const float xq = Xs[(long long)l * n + j];
-            src[lane].x[l] = xq;
-            sincosm1_small(xq - a0[l], sv[l], cv[l]);
-        }
-#pragma unroll
-        for (int l = 0; l < 4; l++) {
-            src[lane].sv[l] = l < D ? w * sv[l] : 0.f;
-            src[lane].cv[l] = l < D ? w * cv[l] : 0.f;
-        }
-        src[lane].sv[3] = w;
-    }
-    wave_sync();
-    const int m = __builtin_amdgcn_readfirstlane(min(kWave, total - base));
-    const float thr_l = acc ? thr : -1.f;  // lanes without acc add zeros
-    constexpr int kS = sizeof(SrcPt<D>) / sizeof(float);
-    const float *row = src[0].sv;  // row[q * kS + c]: column c of source q
-    // per source: the lanes' 0/1 test results, lanes 0-31's to both halves of
-    // the first MFMA's operand (targets 0-31) and 32-63's to the second's
-    int k = 0;
-    for (; k + 4 <= m; k += 4) {  // four sources per step: their LDS reads first
-        float q[4][D], b[4], a[4];
-#pragma unroll
-        for (int jj = 0; jj < 4; jj++) {
-#pragma unroll
-            for (int l = 0; l < D; l++) q[jj][l] = src[k + jj].x[l];
-            b[jj] = row[(k + jj) * kS + cc];
-        }
-#pragma unroll
-        for (int jj = 0; jj < 4; jj++) {
-            float sq = 0.f;
-#pragma unroll
-            for (int l = 0; l < D; l++) {
-                const float df = x[l] - q[jj][l];
-                sq += df * df;
-            }
-            a[jj] = sq <= thr_l ? 1.f : 0.f;
-        }
-#pragma unroll
-        for (int jj = 0; jj < 4; jj++) {
-            const auto pr = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[jj]),
-                                                             __float_as_uint(a[jj]), false, false);
-            d1 = __builtin_amdgcn_mfma_f32_4x4x1f32(__uint_as_float(pr[0]), b[jj], d1, 0, 0, 0);
-            d2 = __builtin_amdgcn_mfma_f32_4x4x1f32(__uint_as_float(pr[1]), b[jj], d2, 0, 0, 0);
-        }
-    }
-    for (; k < m; k++) {
-        float sq = 0.f;
-#pragma unroll
-        for (int l = 0; l < D; l++) {
-            const float df = x[l] - src[k].x[l];
-            sq += df * df;
-        }
-        const float a = sq <= thr_l ? 1.f : 0.f;
-        const auto pr =
-            __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(a), false, false);
-        const float b = row[k * kS + cc];
-        d1 = __builtin_amdgcn_mfma_f32_4x4x1f32(__uint_as_float(pr[0]), b, d1, 0, 0, 0);
-        d2 = __builtin_amdgcn_mfma_f32_4x4x1f32(__uint_as_float(pr[1]), b, d2, 0, 0, 0);
-    }
-    wave_sync();
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        T[(tc + r) * kTr + cc] = d1[r];
-        T[(32 + tc + r) * kTr + cc] = d2[r];
-    }
-    wave_sync();
-#pragma unroll
-    for (int l = 0; l < D; l++) {
-        ssv[l] = T[lane * kTr + l];
-        scm[l] = T[lane * kTr + 4 + l];
-    }
-    m_part += (int)T[lane * kTr + 3];
-    wave_sync();
+__device__ __forceinline__ void stream_add(Stream<D> &sm, int lo, int hi, int r0, int r1, int s0,
+                                           unsigned smask, unsigned long long mask,
+                                           const int *__restrict__ sub_run,
+                                           bool count_near = false) {
+    int before = 0;
+    each_stretch(r0, r1, s0, smask, sub_run, [&](int a, int b) {
+        const int ca = max(a, a + lo - before), cb = min(b, a + hi - before);
+        before += b - a;
+        if (ca < cb) sm.add(ca, cb, mask, count_near);
+    });
 }
 
 // One chunk of a streamed range: runs [base, base + 64) of it go through
@@ -440,13 +344,6 @@ __device__ __forceinline__ void stream_chunk(int base, int total, int r0, int s0
                                              float thr, bool acc, bool any_acc, SrcPt<D> *src,
                                              int *len, float (&ssv)[D], float (&scm)[D],
                                              int &m_part) {
-    if constexpr (D <= 3) {
-        if (any_acc && n < (1 << 24)) {
-            stream_chunk_mfma<D>(base, total, r0, s0, smask, sub_run, run_start, Xs, n, a0, x, thr,
-                                 acc, src, ssv, scm, m_part);
-            return;
-        }
-    }
     const int lane = __lane_id();
     const int rr = stream_run(base + lane, total, r0, s0, smask, sub_run);
     int my_len = 1;
@@ -560,9 +457,7 @@ __device__ __forceinline__ void add_fixed(long long *__restrict__ hacc, int n, i
 }
 
 // The tile's per-lane setup: position (the anchor for lanes without a run),
-// anchor a0 -- the centre of the tile's cell in the outer dimensions and of
-// its block of kAnchorBlock cells in the inner ones, the same for every
-// group width that divides kAnchorBlock -- and sin / cos of u = x - a0.
+// anchor a0 (tile_anchor) and sin / cos of u = x - a0.
 template <int D>
 __device__ __forceinline__ void tile_setup(const TileLane &tl, const float *__restrict__ Xs,
                                            const int *__restrict__ cell_g, const Geo &g,
@@ -572,8 +467,7 @@ __device__ __forceinline__ void tile_setup(const TileLane &tl, const float *__re
 #pragma unroll
     for (int l = 0; l < D; l++) {
         g0[l] = cell_g[(long long)l * n + tl.gc0];
-        a0[l] = l < g.od ? ((float)g0[l] + 0.5f) * g.cs
-                         : ((float)(g0[l] & ~(kAnchorBlock - 1)) + 0.5f * kAnchorBlock) * g.cs;
+        a0[l] = tile_anchor(g0[l], l, g);
         x[l] = tl.active ? Xs[(long long)l * n + tl.i] : a0[l];
         sincos_small(x[l] - a0[l], su[l], cu[l]);
     }
@@ -611,6 +505,20 @@ __device__ __forceinline__ bool finish_run(const float (&x)[D], const float (&su
     return synced;
 }
 
+// The matrix path (egg_stream.h) serves up to kStreamMaxD dimensions and n < 2^24.
+constexpr int kStreamMaxD = 5;
+
+// A wavefront's LDS in k_update_heavy: sources of the scalar paths, or the matrix
+// path's chunk.
+template <int D, bool MM>
+struct TileLds {
+    union {
+        SrcPt<D> src[kWave];
+        std::conditional_t<MM, StreamLds<D>, int> stream;
+    };
+    int len[kWave];
+};
+
 // kernel_itr_grid_STAD5_5_1 (EGG_SynC.cu:551-763).  Per lane: full cells add
 // the cell totals (EGG_SynC.cu:648-663); partial cells are streamed through
 // LDS in chunks of 64 runs -- each lane loads one run and computes sin v and
@@ -623,12 +531,10 @@ __device__ __forceinline__ bool finish_run(const float (&x)[D], const float (&su
 // so the result keeps the accuracy of a direct sum of sinf(x_q - x).  Border
 // lanes count their eps/2-neighbours in other full cells from the same
 // chunks (EGG_SynC.cu:666-681).
-// Up to 3 dimensions the compiler is held to 6 wavefronts per SIMD (80
-// VGPRs, a few spills: the tile's constants); more resident wavefronts hide
-// the LDS and L2 latency of the streaming loop (config 1: -8%).
+// This form serves more than kStreamMaxD dimensions and n >= 2^24; k_update_dense
+// the others.
 template <int D>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(D <= 3 ? 6 : 1)))
-void k_update_tile(
+__global__ __launch_bounds__(kBlock) void k_update_tile(
     const float *__restrict__ Xs, const int *__restrict__ cell_start,
     const int *__restrict__ cell_g, const float *__restrict__ Ts, const float *__restrict__ Tc,
     const int *__restrict__ ob, const int *__restrict__ oe, const int *__restrict__ run_start,
@@ -899,10 +805,493 @@ void k_update_tile(
     if (__any(unsynced) && lane == 0) atomicAnd(&st->flag, 0);
 }
 
+// v, without the compiler's knowledge of it: keeps addresses made from it from
+// being formed ahead of a rare branch, and held in registers until then.
+__device__ __forceinline__ int opaque(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// A wavefront's LDS in k_update_dense: the records of a batch of cells, those of the
+// sub-cells of the next few of them, and, not at the same time, boxes for the eps/2
+// counts or the matrix path's chunk.
+template <int D>
+struct DenseLds {
+    struct Cell {
+        float lo[D], hi[D], ts[D], tc[D];
+        int c, pts, sub0, nsub, run0, run1;
+    } cell[kWave];
+    struct Box {
+        float lo[D], hi[D], ts[D], tc[D];
+        int pts, run0;
+    };
+    Box box[kWave];
+    union {
+        SrcPt<D> src[kWave];
+        StreamLds<D> stream;
+    };
+};
+
+// k_update_tile for up to kStreamMaxD dimensions and n < 2^24: the same tests and
+// the same sums in the same order, arranged for the time a tile takes by itself (a
+// pass ends with its densest tile) and for the VALU.
+//   Candidate cells come 64 at a time.  A lane finds the window of one column by
+// itself, a lane of the next step takes one cell, loads its record and tests it
+// against the box of the tile's targets: cells beyond eps of the whole box are
+// dropped and cells within eps of all of it are marked, by the formula each target
+// would use (FP32 rounding is monotone, so the box bounds every target's result).
+// The rest of the work on a cell reads its record from LDS: no global load is waited
+// for.  Sub-cells are treated alike, their records loaded a cell ahead.
+//   Streamed ranges are noted and summed together on the matrix cores (Stream), from
+// one place in the code: the loop over the cells returns to its head for it.
+// Bound by the VALU: per cell some 250 instructions of tests, per 8 sources 37 beside
+// the matrix instructions.  Held to three wavefronts a SIMD (162 registers): with four
+// the spills cost more than the fourth hides (100 ms against 81 in one state of it).
+// Against k_update_tile (which had the sums alone on the matrix cores), whole solve,
+// n = 1,000,000, d = 3, eps = 0.02: 88 -> 70 ms; one pass of n = 100,003, d = 3: 4.0 ->
+// 3.4 ms; n = 100,000, d = 2: 5.1 -> 3.9; d = 5 passes of a batch 116 -> 75 us.
+template <int D>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(D <= 3 ? 3 : 3)))
+void k_update_dense(GridBufs b, int *__restrict__ rdbg, Geo g, DevState *st) {
+    if (st->done) return;
+    __shared__ DenseLds<D> s_lds[kBlock / kWave];
+    DenseLds<D> &lds = s_lds[threadIdx.x / kWave];
+    const float *__restrict__ Xs = b.Xs;
+    const int *__restrict__ run_start = b.run_start;
+    const int n = g.n, R = g.R, od = g.od, lane = __lane_id();
+    const int G = st->G, T = st->TU;
+    const float thr = g.thr_eps, thr_half = g.thr_half;
+    const float thr_in = thr * (1.0f - 64.0f * 0x1p-24f);
+    const float thr_out = thr * (1.0f + 64.0f * 0x1p-24f);
+    const float thr_half_in = thr_half * (1.0f - 64.0f * 0x1p-24f);
+    const float thr_half_out = thr_half * (1.0f + 64.0f * 0x1p-24f);
+    const int *cg_od = b.cell_g + (long long)od * n;
+    bool unsynced = false;
+    for (int t = wave_index(); t < T; t = wave_count() + next_tile(&st->tile_next)) {
+        const TileLane tl =
+            tile_lane(t, b.utile_off, G, b.grp_cell, b.cell_run, run_start, b.point_cell);
+        const int cl = tl.cl, r = tl.r;
+        const bool active = tl.active;
+        float x[D], sx[D], cx[D], sum[D];
+        float tlo[D], thi[D], ux = 0.f;  // box of the targets, bound on |u_x|^2 (Stream)
+        int g0[D];
+        bool border = false, nan = false;
+#pragma unroll
+        for (int l = 0; l < D; l++) {
+            g0[l] = __builtin_amdgcn_readfirstlane(b.cell_g[(long long)l * n + tl.gc0]);
+            x[l] = active ? Xs[(long long)l * n + tl.i] : tile_anchor(g0[l], l, g);
+            sum[l] = 0.f;
+            sx[l] = sinf(x[l]);
+            cx[l] = cosf(x[l]);
+            border |= active && on_border(x[l], g.cs);
+            nan |= active && !(x[l] == x[l]);
+            float lo = active ? x[l] : INFINITY, hi = active ? x[l] : -INFINITY;
+#pragma unroll
+            for (int o = kWave / 2; o > 0; o >>= 1) {
+                lo = fminf(lo, __shfl_xor(lo, o, kWave));
+                hi = fmaxf(hi, __shfl_xor(hi, o, kWave));
+            }
+            tlo[l] = uniform(lo);
+            thi[l] = uniform(hi);
+            const float ctr = cell_mid(g0[l], g.cs);
+            const float far = fmaxf(fabsf(lo - ctr), fabsf(hi - ctr));
+            ux += far * far;
+        }
+        if (__any(nan)) {  // in no box: let nothing be decided by it
+#pragma unroll
+            for (int l = 0; l < D; l++) {
+                tlo[l] = -INFINITY;
+                thi[l] = INFINITY;
+            }
+        }
+        Stream<D> sm;
+        sm.init(ux, g);
+        int N = 0, half = 0;
+        bool deferred = false;  // some range went to k_update_heavy
+        auto defer_tile = [&]() __attribute__((always_inline)) {
+            if (!deferred) {
+                deferred = true;
+                if (active) {
+                    const int hr = opaque(r);
+#pragma unroll
+                    for (int k = 0; k < 2 * D + 2; k++) b.hacc[(long long)k * n + hr] = 0;
+                }
+                if (lane == 0) b.dtiles[atomicAdd(&st->ndt, 1)] = t;
+            }
+        };
+        // queues a heavy range of cell c; false if the queue is full
+        auto queue_range = [&](int c, int r0, int s0, unsigned smask, int total,
+                               int half_kind) __attribute__((always_inline)) {
+            const int nunits = (total + kUnitRuns - 1) / kUnitRuns;
+            unsigned long long old = 0;
+            if (lane == 0)
+                old = atomicAdd(&st->heavy_pack, (1ull << 32) | (unsigned long long)nunits);
+            const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)old);
+            const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(old >> 32));
+            const bool queued = hi < (unsigned)kHeavyCap;
+            if (queued && lane == 0)
+                b.hdesc[hi] = HeavyDesc{t, c, r0, s0, smask, total, (int)lo, nunits, half_kind};
+            // one lane's branch must not make the loop's state look like the lanes' own
+            return __builtin_amdgcn_readfirstlane(queued) != 0;
+        };
+        // a heavy range of streamed runs waiting for the loop's head: next unit, -1
+        // before it was offered to the queue
+        bool heavy = false;
+        int hu = 0, hc = 0, hr0 = 0, hr1 = 0, hs0 = 0;
+        unsigned hmask = 0;
+        unsigned long long haccs = 0;
+
+        // the columns of the box [g0 - R, g0 + R]^od inside the grid, dim 0 fastest,
+        // 64 at a time: lane k's first cell in the window and the cells before it
+        int rows = 1, row0 = 0, ccell = 0, coff = 0, ctotal = 0, f0 = 0;
+        int ghi[D];  // the tile's group: coordinates g0 .. ghi
+#pragma unroll
+        for (int l = 0; l < D; l++) {
+            ghi[l] = l < D - 1 ? g0[l] : b.cell_g[(long long)l * n + tl.gc1 - 1];
+            if (l < od) rows *= min(g.w - 1, g0[l] + R) - max(0, g0[l] - R) + 1;
+        }
+        const int win_lo = select_dim<D>(g0, od) - R - 1, win_hi = select_dim<D>(ghi, od) + R + 1;
+        unsigned long long keep = 0, all_full = 0;  // of the cells in lds.cell
+        // lane k: sub-cells of cell k if they are to be looked at, and those before
+        int scnt = 0, soff = 0;
+        // cells whose sub-cells are in lds.box, from place sbase on; of those, by
+        // the targets' box: wholly within eps, straddling it
+        unsigned long long staged = 0, sub_in = 0, sub_mixed = 0;
+        int sbase = 0;
+        auto stage_subs = [&](int k) __attribute__((always_inline)) {
+            sbase = __builtin_amdgcn_readlane(soff, k);
+            staged = __ballot(scnt > 0 && soff >= sbase && soff + scnt <= sbase + kWave);
+            const int i = sbase + lane;
+            int q = 0;  // the cell of place i: the last that starts at or before it
+#pragma unroll
+            for (int st = kWave / 2; st > 0; st >>= 1) q += __shfl(soff, q + st) <= i ? st : 0;
+            const int at = i - __shfl(soff, q);
+            int cls = 0;
+            if (at < __shfl(scnt, q) && (staged >> q & 1)) {
+                typename DenseLds<D>::Box sub;
+                const int s = lds.cell[q].sub0 + at;
+                float mx = 0.f, mn = 0.f;
+#pragma unroll
+                for (int l = 0; l < D; l++) {
+                    sub.lo[l] = ord_val(b.smin[(long long)l * n + s]);
+                    sub.hi[l] = ord_val(b.smax[(long long)l * n + s]);
+                    sub.ts[l] = b.TsS[(long long)l * n + s];
+                    sub.tc[l] = b.TcS[(long long)l * n + s];
+                    const float dl = sub.lo[l] - thi[l], dh = sub.hi[l] - tlo[l];
+                    const float el = sub.lo[l] - tlo[l], eh = sub.hi[l] - thi[l];
+                    mx += fmaxf(fmaxf(dl * dl, dh * dh), fmaxf(el * el, eh * eh));
+                    mn += thi[l] < sub.lo[l] ? dl * dl : (tlo[l] > sub.hi[l] ? dh * dh : 0.f);
+                }
+                sub.pts = b.sub_start[s + 1] - b.sub_start[s];
+                sub.run0 = b.sub_run[s];
+                lds.box[lane] = sub;
+                cls = mx <= thr_in ? 1 : (mn >= thr_out ? 0 : 2);
+            }
+            sub_in = __ballot(cls == 1);
+            sub_mixed = __ballot(cls == 2);
+            wave_sync();
+        };
+        // Lanes with `hcnt` count the points of a range of runs (stream_run) of cell
+        // c within eps/2.
+        auto half_scan = [&](int c, int r0, int r1, int s0, unsigned smask,
+                             bool hcnt) __attribute__((always_inline)) {
+            const int total = stream_total(r0, r1, s0, smask, b.sub_run);
+            if (total >= kHeavyRuns) {
+                // a count: exact in any order, so k_update_heavy may take it
+                defer_tile();
+                if (queue_range(c, r0, s0, smask, total, 1)) return;
+            }
+            stream_add<D>(sm, 0, total, r0, r1, s0, smask, __ballot(hcnt), b.sub_run, true);
+        };
+        for (;;) {
+            bool last = false;
+            if (!keep && !heavy) {
+                if (f0 >= ctotal) {
+                    if (row0 < rows) {
+                        int rest = row0 + lane, o = 0, cb = 0, ce = 0;
+                        const bool on = rest < rows;
+#pragma unroll
+                        for (int l = 0; l < D; l++) {
+                            if (l < od) {
+                                const int lo = max(0, g0[l] - R);
+                                const int ext = min(g.w - 1, g0[l] + R) - lo + 1;
+                                o += (lo + rest % ext) * g.wpow[l];
+                                rest /= ext;
+                            }
+                        }
+                        if (on) {
+                            cb = b.ob[o];
+                            ce = b.oe[o];
+                        }
+                        if (od < D) {
+                            // first cells at or above win_lo, above win_hi
+                            int l1 = cb, h1 = ce, l2 = cb, h2 = ce;
+                            while (l1 < h1 || l2 < h2) {
+                                const int m1 = (l1 + h1) >> 1, m2 = (l2 + h2) >> 1;
+                                const int v1 = l1 < h1 ? cg_od[m1] : 0;
+                                const int v2 = l2 < h2 ? cg_od[m2] : 0;
+                                if (l1 < h1) {
+                                    if (v1 < win_lo) l1 = m1 + 1;
+                                    else h1 = m1;
+                                }
+                                if (l2 < h2) {
+                                    if (v2 <= win_hi) l2 = m2 + 1;
+                                    else h2 = m2;
+                                }
+                            }
+                            cb = l1;
+                            ce = max(l1, l2);
+                        }
+                        const int cnt = ce - cb;
+                        const int incl = wave_incl_scan(cnt);
+                        ccell = cb;
+                        coff = incl - cnt;
+                        ctotal = __builtin_amdgcn_readlane(incl, kWave - 1);
+                        row0 += kWave;
+                        f0 = 0;
+                        continue;
+                    }
+                    last = true;
+                } else {
+                    const int f = f0 + lane;
+                    const bool on = f < ctotal;
+                    int q = 0;  // last column that starts at or before f
+#pragma unroll
+                    for (int s = kWave / 2; s > 0; s >>= 1) q += __shfl(coff, q + s) <= f ? s : 0;
+                    const int c = __shfl(ccell, q) + f - __shfl(coff, q);
+                    bool in = on, all = on;
+                    int nsub = 0;
+                    if (on) {
+                        typename DenseLds<D>::Cell rec;
+                        rec.c = c;
+                        const int p0 = b.cell_start[c], s0 = b.cell_sub[c];
+                        rec.pts = b.cell_start[c + 1] - p0;
+                        rec.sub0 = s0;
+                        rec.nsub = nsub = b.cell_sub[c + 1] - s0;
+                        rec.run0 = b.cell_run[c];
+                        rec.run1 = b.cell_run[c + 1];
+                        float near = 0.f, far = 0.f;
+#pragma unroll
+                        for (int l = 0; l < D; l++) {
+                            const int gc = b.cell_g[(long long)l * n + c];
+                            rec.ts[l] = b.Ts[(long long)l * n + c];
+                            rec.tc[l] = b.Tc[(long long)l * n + c];
+                            if (l > od && (gc - ghi[l] > R + 1 || g0[l] - gc > R + 1)) in = false;
+                            const float lo = (float)gc * g.cs, hi = (float)(gc + 1) * g.cs;
+                            rec.lo[l] = lo;
+                            rec.hi[l] = hi;
+                            // bounds of box_dist over the targets' box
+                            const float dl = lo - thi[l], dh = hi - tlo[l];
+                            near += dl > 0.f ? dl * dl : (dh < 0.f ? dh * dh : 0.f);
+                            const float el = lo - tlo[l], eh = hi - thi[l];
+                            far += fmaxf(fmaxf(dl * dl, dh * dh), fmaxf(el * el, eh * eh));
+                        }
+                        in = in && !(near > thr);
+                        all = far <= thr;
+                        lds.cell[lane] = rec;
+                    }
+                    wave_sync();
+                    keep = __ballot(in);
+                    all_full = __ballot(all);
+                    f0 += kWave;
+                    staged = 0;
+                    if (!keep) continue;
+                    scnt = in && !all && g.sub_bits && nsub <= 32 ? nsub : 0;
+                    soff = wave_incl_scan(scnt) - scnt;
+                }
+            }
+            if (last || heavy || __builtin_amdgcn_readfirstlane(sm.nseg) > kWave - 34) {  // a cell adds two ranges
+                sm.flush(lds.stream, x, active, g0, g, Xs, run_start);
+                if (heavy) {
+                    // the float sums so far go to hacc, so that what follows does
+                    // not depend on who sums the range (all sums are additive)
+                    float ssv[D], scm[D];
+#pragma unroll
+                    for (int l = 0; l < D; l++) {
+                        ssv[l] = sm.sin_sum(l);
+                        scm[l] = sm.cos_sum(l);
+                    }
+                    if (active) add_fixed<D>(b.hacc, n, opaque(r), ssv, scm, sm.count());
+                    sm.clear_sums();
+                    const int total = stream_total(hr0, hr1, hs0, hmask, b.sub_run);
+                    if (hu < 0) {
+                        hu = 0;
+                        heavy = !queue_range(hc, hr0, hs0, hmask, total, 0);
+                    }
+                    if (heavy) {
+                        // queue full: this wavefront sums the range itself, unit by
+                        // unit in fixed point, as k_update_heavy would
+                        heavy = hu < total;
+                        if (heavy)
+                            stream_add<D>(sm, hu, min(total, hu + kUnitRuns), hr0, hr1, hs0,
+                                          hmask, haccs, b.sub_run);
+                        hu += kUnitRuns;
+                    }
+                    continue;
+                }
+                if (last) break;
+            }
+            const int k = __builtin_ctzll(keep);
+            keep &= keep - 1;
+            const typename DenseLds<D>::Cell &rec = lds.cell[k];
+            bool full = active, part = false;
+            if (!(all_full >> k & 1)) {
+                float near = 0.f, far = 0.f;  // box_dist
+#pragma unroll
+                for (int l = 0; l < D; l++) {
+                    float lo = rec.lo[l] - x[l], hi = rec.hi[l] - x[l];
+                    lo *= lo;
+                    hi *= hi;
+                    near += lo < hi ? lo : hi;
+                    far += lo < hi ? hi : lo;
+                }
+                full = active && far <= thr;
+                part = active && !full && near <= thr;
+            }
+            const int c = __builtin_amdgcn_readfirstlane(rec.c);
+            if (full) {
+#pragma unroll
+                for (int l = 0; l < D; l++) {
+                    const float p = rec.ts[l] * cx[l];
+                    const float q = rec.tc[l] * sx[l];
+                    const float tt = p - q;
+                    sum[l] += tt;
+                }
+                N += rec.pts;
+                if (border && c == cl) half += rec.pts;
+            }
+            if (all_full >> k & 1 && !__any(border && c != cl)) continue;
+            const int s0 = __builtin_amdgcn_readfirstlane(rec.sub0);
+            const int ns = __builtin_amdgcn_readfirstlane(rec.nsub);
+            const int r0 = __builtin_amdgcn_readfirstlane(rec.run0);
+            const int r1 = __builtin_amdgcn_readfirstlane(rec.run1);
+            const bool by_subs = g.sub_bits && ns <= 32;
+            const bool need_half = full && border && c != cl;
+            if (__any(need_half)) {
+                // eps/2-neighbours in another full cell: sub-cells wholly
+                // within eps/2 of a lane count whole, those straddling
+                // eps/2 for some lane are streamed for the wavefront
+                if (by_subs) {
+                    unsigned hin = 0, hst = 0;
+                    stage_boxes<D>(b.smin, b.smax, n, s0, ns, lds.src);
+                    if (need_half) {
+                        for (int i = 0; i < ns; i++) {
+                            const int cls = sub_class_box<D>(lds.src[i].x, lds.src[i].sv, x,
+                                                             thr_half_in, thr_half_out);
+                            if (cls == 1) hin |= 1u << i;
+                            else if (cls == 2) hst |= 1u << i;
+                        }
+                    }
+                    wave_sync();
+                    const unsigned hu32 = wave_or(hst);
+                    const unsigned ht = hin & ~hu32;
+                    for (unsigned mm = wave_or(ht); mm; mm &= mm - 1) {
+                        const int i = __builtin_ctz(mm);
+                        if ((ht >> i) & 1u) half += b.sub_start[s0 + i + 1] - b.sub_start[s0 + i];
+                    }
+                    if (hu32) half_scan(c, 0, 0, s0, hu32, need_half);
+                } else {
+                    half_scan(c, r0, r1, 0, 0u, need_half);
+                }
+            }
+            if (all_full >> k & 1) continue;
+            const unsigned long long parts = __ballot(part);
+            unsigned umask = 0;
+            int at = 0;  // place of the cell's sub-cells in lds.box
+            if (parts && by_subs) {
+                // sub-cells of a partial cell: wholly within eps, wholly beyond or
+                // straddling it, for all targets by their box where that decides, else
+                // for each; those some lane straddles are streamed once for the
+                // wavefront and tested point by point by every lane with a partial
+                // cell; others wholly within eps add their totals
+                if (!(staged >> k & 1)) stage_subs(k);
+                at = __builtin_amdgcn_readlane(soff, k) - sbase;
+                const typename DenseLds<D>::Box *box = lds.box + at;
+                const unsigned below = ns < 32 ? (1u << ns) - 1u : ~0u;
+                unsigned in_some = (unsigned)(sub_in >> at) & below;
+                const unsigned mixed = (unsigned)(sub_mixed >> at) & below;
+                unsigned imask = part ? in_some : 0u;
+                for (unsigned mm = mixed; mm; mm &= mm - 1) {
+                    const int i = __builtin_ctz(mm);
+                    const int cl2 = part ? sub_class_box<D>(box[i].lo, box[i].hi, x, thr_in, thr_out)
+                                         : 0;
+                    if (cl2 == 1) imask |= 1u << i;
+                    if (__any(cl2 == 1)) in_some |= 1u << i;
+                    if (__any(cl2 == 2)) umask |= 1u << i;
+                }
+                for (unsigned mm = in_some & ~umask; mm; mm &= mm - 1) {
+                    const int i = __builtin_ctz(mm);
+                    if ((imask >> i) & 1u) {
+#pragma unroll
+                        for (int l = 0; l < D; l++) {
+                            const float p = box[i].ts[l] * cx[l];
+                            const float q = box[i].tc[l] * sx[l];
+                            const float tt = p - q;
+                            sum[l] += tt;
+                        }
+                        N += box[i].pts;
+                    }
+                }
+            }
+            if (!parts || (by_subs && !umask)) continue;
+            if (r1 - r0 >= kHeavyRuns && stream_total(r0, r1, s0, umask, b.sub_run) >= kHeavyRuns) {
+                defer_tile();
+                heavy = true;
+                hu = -1;
+                hc = c;
+                hr0 = r0;
+                hr1 = r1;
+                hs0 = s0;
+                hmask = umask;
+                haccs = parts;
+            } else if (!umask) {
+                sm.add(r0, r1, parts);
+            } else {
+                for (unsigned long long mm = umask; mm;) {
+                    const int i = __builtin_ctzll(mm), len = __builtin_ctzll(~(mm >> i));
+                    sm.add(lds.box[at + i].run0, i + len < ns ? lds.box[at + i + len].run0 : r1,
+                           parts);
+                    mm &= ~(((1ull << len) - 1) << i);
+                }
+            }
+        }
+        float su[D], cu[D], ssv[D], scm[D];
+#pragma unroll
+        for (int l = 0; l < D; l++) {
+            sincos_small(x[l] - tile_anchor(g0[l], l, g), su[l], cu[l]);
+            ssv[l] = sm.sin_sum(l);
+            scm[l] = sm.cos_sum(l);
+        }
+        const int m_part = sm.count();
+        half += (int)sm.near;
+        const int ro = opaque(r);
+        if (deferred) {
+            // the sums so far wait for the heavy ranges: full-cell totals in
+            // rres, N / half / border in dsave, streamed sums into hacc
+            if (active) {
+#pragma unroll
+                for (int l = 0; l < D; l++) b.rres[(long long)l * n + ro] = sum[l];
+                b.rdbg[4 * (long long)ro + 0] = N;
+                b.rdbg[4 * (long long)ro + 1] = half;
+                b.rdbg[4 * (long long)ro + 2] = border ? 1 : 0;
+                add_fixed<D>(b.hacc, n, ro, ssv, scm, m_part);
+            }
+            continue;
+        }
+        if (active) {
+            const int own = b.cell_start[cl + 1] - b.cell_start[cl];
+            if (!finish_run<D>(x, su, cu, sum, ssv, scm, N, m_part, half, border, own, n, ro,
+                               b.rres, rdbg))
+                unsynced = true;
+        }
+    }
+    if (__any(unsynced) && lane == 0) atomicAnd(&st->flag, 0);
+}
+
 // Work units of the heavy ranges (kUnitRuns runs each), from a queue over
 // all of them: every wavefront rebuilds the tile's lanes, tests the unit's
 // runs as the tile kernel would and adds its sums in fixed point.
-template <int D>
+template <int D, bool MM>
 __global__ __launch_bounds__(kBlock) void k_update_heavy(
     const float *__restrict__ Xs, const int *__restrict__ cell_g,
     const int *__restrict__ run_start, const int *__restrict__ cell_run,
@@ -912,10 +1301,10 @@ __global__ __launch_bounds__(kBlock) void k_update_heavy(
     if (st->done) return;
     const int nd = (int)min((unsigned long long)kHeavyCap, st->heavy_pack >> 32);
     if (nd == 0) return;
-    __shared__ SrcPt<D> s_src[kBlock / kWave][kWave];
-    __shared__ int s_len[kBlock / kWave][kWave];
-    SrcPt<D> *src = s_src[threadIdx.x / kWave];
-    int *len = s_len[threadIdx.x / kWave];
+    __shared__ TileLds<D, MM> s_lds[kBlock / kWave];
+    TileLds<D, MM> &lds = s_lds[threadIdx.x / kWave];
+    SrcPt<D> *src = lds.src;
+    int *len = lds.len;
     const int n = g.n, G = st->G;
     const float thr = g.thr_eps;
     // descriptors k < nd hold consecutive unit ranges in the order of k
@@ -939,23 +1328,47 @@ __global__ __launch_bounds__(kBlock) void k_update_heavy(
         box_dist<D>(gc, x, g.cs, sm, lg);
         const int k = u - hd.ubase;
         const int b1 = min(hd.total, (k + 1) * kUnitRuns);
-        if (hd.half) {
-            // border lanes of the tile, the range's cell full for them and
-            // not their own: points within eps/2
-            bool border = false;
+        const bool acc = tl.active && !(lg <= thr) && sm <= thr;
+        // border lanes of the tile, a half range's cell full for them and not
+        // their own: points within eps/2
+        bool border = false;
 #pragma unroll
-            for (int l = 0; l < D; l++) border |= on_border(x[l], g.cs);
-            const bool hcnt = tl.active && lg <= thr && border && hd.c != tl.cl;
-            int cnt = 0;
+        for (int l = 0; l < D; l++) border |= on_border(x[l], g.cs);
+        const bool hcnt = tl.active && lg <= thr && border && hd.c != tl.cl;
+        float ps[D], pc[D];
+        int pm = 0, cnt = 0;
+#pragma unroll
+        for (int l = 0; l < D; l++) ps[l] = pc[l] = 0.f;
+        if constexpr (MM) {
+            float ux = 0.f;
+#pragma unroll
+            for (int l = 0; l < D; l++) {
+                const float v = tl.active ? x[l] - cell_mid(g0[l], g.cs) : 0.f;
+                ux += v * v;
+            }
+#pragma unroll
+            for (int o = kWave / 2; o > 0; o >>= 1) ux = fmaxf(ux, __shfl_xor(ux, o, kWave));
+            Stream<D> q;
+            q.init(ux, g);
+            stream_add<D>(q, k * kUnitRuns, b1, hd.r0, hd.r0 + hd.total, hd.s0, hd.smask,
+                          __ballot(hd.half ? hcnt : acc), sub_run, hd.half != 0);
+            q.flush(lds.stream, x, tl.active, g0, g, Xs, run_start);
+#pragma unroll
+            for (int l = 0; l < D; l++) {
+                ps[l] = q.sin_sum(l);
+                pc[l] = q.cos_sum(l);
+            }
+            pm = q.count();
+            cnt = (int)q.near;
+        } else if (hd.half) {
             for (int base = k * kUnitRuns; base < b1; base += kWave) {
-                const int rr = stream_run(base + __lane_id(), b1, hd.r0, hd.s0, hd.smask,
-                                          sub_run);
+                const int rr =
+                    stream_run(base + __lane_id(), b1, hd.r0, hd.s0, hd.smask, sub_run);
                 if (rr >= 0) {
                     const int j = run_start[rr];
                     len[__lane_id()] = run_start[rr + 1] - j;
 #pragma unroll
-                    for (int l = 0; l < D; l++)
-                        src[__lane_id()].x[l] = Xs[(long long)l * n + j];
+                    for (int l = 0; l < D; l++) src[__lane_id()].x[l] = Xs[(long long)l * n + j];
                 }
                 wave_sync();
                 const int m = min(kWave, b1 - base);
@@ -972,21 +1385,18 @@ __global__ __launch_bounds__(kBlock) void k_update_heavy(
                 }
                 wave_sync();
             }
+        } else {
+            for (int base = k * kUnitRuns; base < b1; base += kWave)
+                stream_chunk<D>(base, b1, hd.r0, hd.s0, hd.smask, sub_run, run_start, Xs, n, a0,
+                                x, thr, acc, __any(acc), src, len, ps, pc, pm);
+        }
+        if (hd.half) {
             if (hcnt)
                 atomicAdd((unsigned long long *)hacc + (long long)(2 * D + 1) * n + tl.r,
                           (unsigned long long)cnt);
-            continue;
+        } else if (acc) {
+            add_fixed<D>(hacc, n, tl.r, ps, pc, pm);
         }
-        const bool acc = tl.active && !(lg <= thr) && sm <= thr;
-        const bool any_acc = __any(acc);
-        float ps[D], pc[D];
-        int pm = 0;
-#pragma unroll
-        for (int l = 0; l < D; l++) ps[l] = pc[l] = 0.f;
-        for (int base = k * kUnitRuns; base < b1; base += kWave)
-            stream_chunk<D>(base, b1, hd.r0, hd.s0, hd.smask, sub_run, run_start, Xs, n, a0, x,
-                            thr, acc, any_acc, src, len, ps, pc, pm);
-        if (acc) add_fixed<D>(hacc, n, tl.r, ps, pc, pm);
     }
 }
 
@@ -1480,33 +1890,40 @@ static inline int queue_blocks(const Geo &g) {
     return (int)std::max<long long>(1, std::min<long long>(cap, (tiles_max + waves - 1) / waves));
 }
 
+template <int D, bool MM>
+static void launch_tiles(const Geo &g, GridBufs &b, int *rdbg, int qb, int qt, DevState *st,
+                         hipStream_t s) {
+    if constexpr (MM)
+        k_update_dense<D><<<qb, qt, 0, s>>>(b, rdbg, g, st);
+    else
+        k_update_tile<D><<<qb, qt, 0, s>>>(
+            b.Xs, b.cell_start, b.cell_g, b.Ts, b.Tc, b.ob, b.oe, b.run_start, b.cell_run,
+            b.grp_cell, b.point_cell, b.utile_off, b.cell_sub, b.sub_start, b.smin, b.smax,
+            b.sub_run, b.TsS, b.TcS, b.rres, rdbg, b.hacc, b.hdesc, b.dtiles, b.rdbg, g, st);
+    if (!b.hacc) return;
+    k_update_heavy<D, MM><<<qb, qt, 0, s>>>(b.Xs, b.cell_g, b.run_start, b.cell_run, b.grp_cell,
+                                            b.point_cell, b.utile_off, b.sub_run, b.hdesc, b.hacc,
+                                            g, st);
+    k_update_finish<D><<<qb, qt, 0, s>>>(b.Xs, b.cell_start, b.cell_g, b.run_start, b.cell_run,
+                                         b.grp_cell, b.point_cell, b.utile_off, b.dtiles, b.rdbg,
+                                         b.hacc, b.rres, rdbg, g, st);
+}
+
 void launch_update_egg(const Geo &g, GridBufs &b, DevState *st, const DebugOut *dbg,
                        hipStream_t s) {
     DebugOut d = dbg ? *dbg : DebugOut{nullptr, nullptr, nullptr, nullptr};
     const int qb = queue_blocks(g), qt = queue_threads(g);
     int *rdbg = (d.N || d.half || d.border || d.synced) ? b.rdbg : nullptr;
-#define UPD_CASE(DD)                                                                          \
-    case DD:                                                                                  \
-        k_update_tile<DD><<<qb, qt, 0, s>>>(b.Xs, b.cell_start, b.cell_g, b.Ts, b.Tc,     \
-                                            b.ob, b.oe, b.run_start, b.cell_run,              \
-                                            b.grp_cell, b.point_cell, b.utile_off,            \
-                                            b.cell_sub, b.sub_start, b.smin, b.smax,          \
-                                            b.sub_run, b.TsS, b.TcS, b.rres, rdbg, b.hacc,    \
-                                            b.hdesc,                                          \
-                                            b.dtiles, b.rdbg, g, st);                         \
-        if (b.hacc) {                                                                         \
-            k_update_heavy<DD><<<qb, qt, 0, s>>>(b.Xs, b.cell_g, b.run_start, b.cell_run,     \
-                                                 b.grp_cell, b.point_cell, b.utile_off,       \
-                                                 b.sub_run, b.hdesc, b.hacc, g, st);          \
-            k_update_finish<DD><<<qb, qt, 0, s>>>(b.Xs, b.cell_start, b.cell_g, b.run_start,  \
-                                                  b.cell_run, b.grp_cell, b.point_cell,       \
-                                                  b.utile_off, b.dtiles, b.rdbg, b.hacc,      \
-                                                  b.rres, rdbg, g, st);                       \
-        }                                                                                     \
-        launch_update_pairs(g, b, rdbg, st, s);                                               \
-        k_scatter_runs<DD><<<grid_for(g.n), kBlock, 0, s>>>(b.point_run, b.rres, rdbg,       \
-                                                            b.perm_s, b.X, b.perm, g.n, st,   \
-                                                            d);                               \
+#define UPD_CASE(DD)                                                                      \
+    case DD:                                                                              \
+        if (DD <= kStreamMaxD && g.n < (1 << 24))                                         \
+            launch_tiles<DD, (DD <= kStreamMaxD)>(g, b, rdbg, qb, qt, st, s);             \
+        else                                                                              \
+            launch_tiles<DD, false>(g, b, rdbg, qb, qt, st, s);                           \
+        launch_update_pairs(g, b, rdbg, st, s);                                           \
+        k_scatter_runs<DD><<<grid_for(g.n), kBlock, 0, s>>>(b.point_run, b.rres, rdbg,    \
+                                                            b.perm_s, b.X, b.perm, g.n,   \
+                                                            st, d);                       \
         break;
     switch (g.d) {
         EGG_EACH_D(UPD_CASE)

@@ -545,3 +545,33 @@ def test_grid_tables_on_both_sides_of_the_wide_tiles(S, O):
         assert a["C"] == b["C"]
         for k in ("order", "cell_of", "cell_start", "cell_g", "ob", "oe"):
             assert np.array_equal(a[k], b[k]), (n, k)
+
+
+@pytest.mark.parametrize("d", [1, 2, 3, 4, 5])
+def test_dense_update_on_the_boundaries(S, O, d):
+    """The dense update where its matrix-core test cannot decide and the reference's formula must: a
+    lattice of spacing eps / 4, so that many pairs lie at eps and eps / 2 up to rounding, beside
+    dense random cells (segments of every remainder, more than 64 runs a tile), clamped points
+    (coordinate 1), points on cell faces and runs of several points.  Bit for bit in the counts and
+    flags, within 1e-6 in the positions, as in test_iteration_bit_exact."""
+    rng = np.random.default_rng(110 + d)
+    for eps in (0.05, 0.15 * np.sqrt(d)):
+        k = int(round(1500 ** (1.0 / d)))
+        step = np.float32(eps / 4)
+        lattice = np.stack(np.meshgrid(*[np.arange(k)] * d), -1).reshape(-1, d).astype(f32) * step
+        lattice = lattice[(lattice <= 1).all(1)]
+        cs = S.nat.geometry(4000, d, eps)["cs"]
+        dense = (0.4 + 1.5 * cs * rng.random((1200, d))).astype(f32)
+        X = np.concatenate([lattice, dense, rng.random((300, d)).astype(f32)])
+        X[-300:-250] = X[-300]
+        X[-250:-200, 0] = np.float32(3 * cs) if 3 * cs <= 1 else f32(0.5)
+        X[-200:-150] = 1.0 - X[-200:-150] * f32(0.02)
+        X[-1] = 1.0
+        X = X[rng.permutation(len(X))]
+        _say("dense update", X.shape, eps)
+        a = S.iteration(X, eps)
+        b = O.egg_iteration(X, eps)
+        for key in ("order", "N", "half", "border", "synced"):
+            assert np.array_equal(a[key], b[key]), (eps, key)
+        assert (a["flag_local"], a["flag_final"]) == (b["flag_local"], b["flag_final"])
+        assert np.abs(a["X_next"] - b["X_next"]).max() <= 1e-6, eps
