@@ -177,3 +177,38 @@ def test_gradients_of_a_batch_beyond_the_partial_tiles(L):
     lr, gr = M.loss_and_grad(net.state(), F.cpu().numpy(), T.cpu().numpy(), 8, 64, 2)
     assert abs(loss - lr) <= 1e-5 * max(1.0, abs(lr))
     assert np.abs(g.cpu().numpy() - gr).max() <= 2e-4 * np.abs(gr).max()
+
+
+@pytest.mark.parametrize("d", [1, 2, 3, 5, 20])
+def test_features_at_row_edges(L, O, d):
+    """Rows of the features at the remainders of a wavefront's 64, into memory aligned to 16 bytes
+    and not: positions as given, means within 1e-6 of FP64 sums over the oracle's cells (totals
+    compensated to a few 2^-24 of values up to 1), displacements as their FP32 formula."""
+    nat, eps = L.nat, 0.3
+    rng = np.random.default_rng(200 + d)
+    for n in (1, 63, 64, 65, 1000):
+        X = rng.random((n, d)).astype(np.float32)
+        prev = rng.random((n, d)).astype(np.float32)
+        cell = np.empty(n, np.int64)
+        g = O.build_grid(X, eps)
+        cell[g["order"]] = g["cell_of"]
+        cnt = np.bincount(cell, minlength=g["C"])[:, None]
+        mean = [np.stack([np.bincount(cell, f(X[:, l].astype(np.float64)), g["C"])
+                          for l in range(d)], 1) / cnt for f in (np.sin, np.cos)]
+        inv = np.float32(1.0) / np.float32(eps)
+        Xd, Pd = torch.from_numpy(X).cuda(), torch.from_numpy(prev).cuda()
+        for shift in (0, 1):
+            for p in (Pd, None):
+                _say("features", n, d, shift, p is not None)
+                buf = torch.full((n * 4 * d + 2,), -7.0, device="cuda")
+                rc = nat.lib().egg_sync_features_device(nat.ptr(Xd), nat.ptr(p), n, d, eps,
+                                                        nat.ptr(buf[shift:]), None)
+                nat.check(rc, "egg_sync_features_device")
+                out = buf.cpu().numpy()
+                assert np.all(out[:shift] == -7.0) and np.all(out[shift + n * 4 * d:] == -7.0)
+                F = out[shift:shift + n * 4 * d].reshape(n, 4, d)
+                assert np.array_equal(F[:, 0], X)
+                assert np.abs(F[:, 1] - mean[0][cell]).max() <= 1e-6
+                assert np.abs(F[:, 2] - mean[1][cell]).max() <= 1e-6
+                want = (X - prev) * inv if p is not None else np.zeros_like(X)
+                assert np.array_equal(F[:, 3], want)
