@@ -1821,10 +1821,91 @@ __attribute__((amdgpu_waves_per_eu(D <= 8 ? 8 : 4))) void k_update_sync(
     }
 }
 
-// Block partial sums of the points' r_p / N, combined in a fixed order by
-// k_rc_finish, so r_c is deterministic.
 constexpr int kRcBlocks = 1024;
 
+// The same pass with a lane per target, each adding its neighbours one after the
+// other: k_update_sync spreads a target's candidates over a wavefront and so fills
+// the chip from a few thousand points on, but has a serial chain of additions for
+// each target with few lanes to share; once there are targets enough for every lane
+// of the chip, a lane's own chain hides behind the others'.
+template <int D, bool WRITE>
+__global__ __launch_bounds__(kBlock) void k_update_sync_lane(
+    const float *__restrict__ Xs, float *__restrict__ Xout, const int *__restrict__ perm_s,
+    int *__restrict__ perm_out, const int *__restrict__ point_cell,
+    const int *__restrict__ cell_start, const int *__restrict__ cell_g,
+    const int *__restrict__ ob, const int *__restrict__ oe, Geo g, const DevState *st,
+    double *__restrict__ ratio) {
+    if (WRITE && st->done) return;
+    const int n = g.n, od = g.od, R = g.R + 1;
+    const int *cg_od = cell_g + (long long)od * n;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        float x[D], sum[D];
+        int g0[D];
+        const int c0 = point_cell[i];
+#pragma unroll
+        for (int l = 0; l < D; l++) {
+            x[l] = Xs[(long long)l * n + i];
+            g0[l] = cell_g[(long long)l * n + c0];
+            sum[l] = 0.f;
+        }
+        const int g0od = select_dim<D>(g0, od);
+        int N = 0;
+        double r = 0.0;
+        Odo<D> odo;
+        odo.init(od, R);
+        while (!odo.finished) {
+            const int o = odo.outer(g0, g);
+            if (o >= 0) {
+                int cb = ob[o];
+                const int ce = oe[o];
+                if (od < D) cb = column_lower(cg_od, cb, ce, g0od - R);
+                for (int c = cb; c < ce; c++) {
+                    int gc[D];
+#pragma unroll
+                    for (int l = 0; l < D; l++) gc[l] = cell_g[(long long)l * n + c];
+                    if (od < D && select_dim<D>(gc, od) > g0od + R) break;
+                    bool skip = false;
+#pragma unroll
+                    for (int l = 0; l < D; l++)
+                        if (l > od && (gc[l] - g0[l] > R || g0[l] - gc[l] > R)) skip = true;
+                    if (skip) continue;
+                    for (int j = cell_start[c]; j < cell_start[c + 1]; j++) {
+                        float xq[D];
+                        const float s = dist2_to<D>(x, Xs, n, j, xq);
+                        if (s <= g.thr_eps) {
+                            if (WRITE) {
+#pragma unroll
+                                for (int l = 0; l < D; l++) sum[l] += sinf(xq[l] - x[l]);
+                            }
+                            N++;
+                            r += (double)expf(-fabsf(sqrtf(s)));
+                        }
+                    }
+                }
+            }
+            odo.next(od, R);
+        }
+        if (WRITE) {
+#pragma unroll
+            for (int l = 0; l < D; l++) {
+                const float t = sum[l] / (float)N;
+                Xout[(long long)l * n + i] = x[l] + t;
+            }
+            perm_out[i] = perm_s[i];
+        }
+        ratio[i] = N > 0 ? r / (double)N : 1.0;
+    }
+}
+
+// From this many points on the SynC pass takes k_update_sync_lane.  Wavefront /
+// lane form, ms a pass on blobs as given and, second, converged: n = 65,536 at d = 2
+// 3.1 / 7.6 and 3.5 / 4.2, at d = 3 1.8 / 5.7 and 3.6 / 7.0; n = 131,072 10.9 / 12.3
+// and 11.8 / 8.0, 6.4 / 9.9 and 13.4 / 8.1; n = 200,000 18 / 13 and 27 / 17, 16 / 31
+// and 29 / 11; n = 1,000,000, d = 3, converged 702 / 197.
+constexpr int kSyncLaneMin = 1 << 17;
+
+// Block partial sums of the points' r_p / N, combined in a fixed order by
+// k_rc_finish, so r_c is deterministic.
 __global__ __launch_bounds__(kBlock) void k_rc_sum(const double *__restrict__ ratio, int n,
                                                    const DevState *st, bool guard,
                                                    double *__restrict__ rc_part) {
@@ -1953,13 +2034,19 @@ void launch_update_sync(const Geo &g, GridBufs &b, DevState *st, double *rc_part
                         hipStream_t s) {
     double *ratio = (double *)b.rdbg;  // [n] of its 4n ints, unused by this pass
 #define SY_LAUNCH(DD, W, X, P)                                                                    \
-    k_update_sync<DD, W><<<(g.n + SyncShape<DD, W>::T - 1) / SyncShape<DD, W>::T,                 \
+    if (g.n >= kSyncLaneMin)                                                                      \
+        k_update_sync_lane<DD, W><<<kRcBlocks, kBlock, 0, s>>>(                                   \
+            b.Xs, X, b.perm_s, P, b.point_cell, b.cell_start, b.cell_g, b.ob, b.oe, g, st, ratio); \
+    else k_update_sync<DD, W><<<(g.n + SyncShape<DD, W>::T - 1) / SyncShape<DD, W>::T,                 \
                            SyncShape<DD, W>::kThreads, 0, s>>>(                                   \
         b.Xs, X, b.perm_s, P, b.point_cell, b.cell_start, b.cell_g, b.ob, b.oe, g, st, ratio)
 #define SY_CASE(DD)                                       \
     case DD:                                              \
-        if (write_pos) SY_LAUNCH(DD, true, b.X, b.perm);  \
-        else SY_LAUNCH(DD, false, nullptr, nullptr);      \
+        if (write_pos) {                                  \
+            SY_LAUNCH(DD, true, b.X, b.perm);             \
+        } else {                                          \
+            SY_LAUNCH(DD, false, nullptr, nullptr);       \
+        }                                                 \
         break;
     switch (g.d) {
         EGG_EACH_D(SY_CASE)

@@ -575,3 +575,25 @@ def test_dense_update_on_the_boundaries(S, O, d):
             assert np.array_equal(a[key], b[key]), (eps, key)
         assert (a["flag_local"], a["flag_final"]) == (b["flag_local"], b["flag_final"])
         assert np.abs(a["X_next"] - b["X_next"]).max() <= 1e-6, eps
+
+
+@pytest.mark.parametrize("d", [2, 3])
+def test_sync_pass_on_both_sides_of_the_lane_form(S, d):
+    """The SynC pass below and from 2^17 points on takes another form.  The same points twice over,
+    far apart in one coordinate, make two copies of one problem: at 2^16 points a copy the pass
+    over one copy and over both give each point the same neighbours and so the same bits."""
+    nat = S.nat
+    rng = np.random.default_rng(130 + d)
+    n = 1 << 16
+    X = rng.random((n, d)).astype(f32)
+    X[:, 0] = f32(0.25) * X[:, 0]  # the copy: + 0.5, exact in its grid of 2^-26
+    X[:, 0] = np.round(X[:, 0] * 2.0 ** 23).astype(f32) * f32(2.0 ** -23)
+    Y = X.copy()
+    Y[:, 0] += f32(0.5)
+    Z = np.concatenate([X, Y])
+    eps = 0.01 if d == 2 else 0.03
+    _say("sync pass forms", Z.shape)
+    one = S.solve(X, eps, stop_rule=nat.STOP_RC, lam=1.5, max_iter=1)
+    two = S.solve(Z, eps, stop_rule=nat.STOP_RC, lam=1.5, max_iter=1)
+    assert np.abs(two["X"][:n] - one["X"]).max() <= 1e-6
+    assert abs(two["stats"]["rc"] - one["stats"]["rc"]) <= 1e-7
