@@ -43,9 +43,9 @@ ITERS_PER_SYNC = 4
 # pass's MFMA instructions too; those alone are UPDATE_MFMA_INSTS_N1M).
 # Measured for this workload only, so reported only when n is 1,000,000.
 UPDATE_PROFILE = "profiles/update_pass_config1_n1M_counters.md"
-UPDATE_TRAFFIC_BYTES_N1M = 826.7e6
-UPDATE_VALU_INSTS_N1M = 4.15e9
-UPDATE_MFMA_INSTS_N1M = 2.75e8
+UPDATE_TRAFFIC_BYTES_N1M = 89.9e6
+UPDATE_VALU_INSTS_N1M = 2.92e9
+UPDATE_MFMA_INSTS_N1M = 4.78e8
 
 
 def cpu_baseline(X, eps, target_seconds=12.0):
@@ -370,7 +370,7 @@ def main():
                      "frac": achieved / HBM_PEAK_GBS,
                      "traffic": UPDATE_TRAFFIC_BYTES_N1M if full_size else None,
                      "traffic_source": UPDATE_PROFILE if full_size else None,
-                     "kernel": "update pass: k_update_tile<3> + k_update_heavy<3> + "
+                     "kernel": "update pass: k_update_dense<3> + k_update_heavy<3> + "
                                "k_update_finish<3> + k_run_boxes<3> + k_super_boxes<3> + "
                                "k_update_pairs<3> + k_scatter_runs<3>",
                      "launches": launches,
