@@ -458,6 +458,15 @@ struct SumGroups {
     float *partial;                   // [slots][6 d], kept for the second pass
 };
 
+// A sub-cell's box from the keys of its points' bounds.  A point that is not a
+// number sorts beyond the infinities; its box then reaches to infinity, so that no
+// test takes the sub-cell as a whole.
+__device__ __forceinline__ void store_box(const SumGroups &q, long long at, unsigned kmin,
+                                          unsigned kmax) {
+    q.mnk[at] = max(kmin, 0x007FFFFFu);  // ord_key(-inf)
+    q.mxk[at] = min(kmax, 0xFF800000u);  // ord_key(inf)
+}
+
 // Per dim: S_sin = sum(sinf(x) - sinf(g*cs)), S_cos likewise (EGG_SynC.cu:362-363),
 // Kahan-compensated per lane, combined across lanes by compensated butterflies,
 // then T_sin = sinf(g*cs)*cnt + S_sin (the bracket of EGG_SynC.cu:651-654).  A
@@ -507,10 +516,7 @@ __device__ __forceinline__ void sum_chunk(const float *__restrict__ Xs, int n,
                 const float t2 = ca * cnt;
                 q.Ts[(long long)l * n + grp] = t1 + (s1 + e1);
                 q.Tc[(long long)l * n + grp] = t2 + (s2 + e2);
-                if (q.mnk) {
-                    q.mnk[(long long)l * n + grp] = kmin;
-                    q.mxk[(long long)l * n + grp] = kmax;
-                }
+                if (q.mnk) store_box(q, (long long)l * n + grp, kmin, kmax);
             } else {
                 float *pp = &q.partial[((long long)summary_slot(c0, (j0 - c0) / kSumChunk) * D + l) * 6];
                 pp[0] = s1; pp[1] = e1; pp[2] = s2; pp[3] = e2;
@@ -610,10 +616,7 @@ __global__ __launch_bounds__(kBlock) void k_summary(const float *__restrict__ Xs
                     const float t2 = ca * c;
                     q.Ts[(long long)l * n + grp[k]] = t1 + (s1 + e1);
                     q.Tc[(long long)l * n + grp[k]] = t2 + (s2 + e2);
-                    if (k) {
-                        q.mnk[(long long)l * n + grp[k]] = kmin;
-                        q.mxk[(long long)l * n + grp[k]] = kmax;
-                    }
+                    if (k) store_box(q, (long long)l * n + grp[k], kmin, kmax);
                 }
             }
         }
@@ -652,10 +655,7 @@ __device__ __forceinline__ void sum_partials(int n, const SumGroups &q, int grp,
             const float t2 = cosf(a) * cnt;
             q.Ts[(long long)l * n + grp] = t1 + (s1 + e1);
             q.Tc[(long long)l * n + grp] = t2 + (s2 + e2);
-            if (q.mnk) {
-                q.mnk[(long long)l * n + grp] = kmin;
-                q.mxk[(long long)l * n + grp] = kmax;
-            }
+            if (q.mnk) store_box(q, (long long)l * n + grp, kmin, kmax);
         }
     }
 }

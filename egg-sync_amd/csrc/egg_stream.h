@@ -169,7 +169,8 @@ struct Stream {
         for (int l = 0; l < D; l++) {
             a0[l] = tile_anchor(g0[l], l, g);
             ctr[l] = cell_mid(g0[l], g.cs);
-            const float u = active ? x[l] - ctr[l] : 0.f;
+            // a target that is not a number is within eps of nothing and tests nothing
+            const float u = active && x[l] == x[l] ? x[l] - ctr[l] : 0.f;
             u2 += u * u;
             X[l] = 2.0f * u * inv_m;
         }
@@ -217,18 +218,23 @@ struct Stream {
                     e_n = run_start[rr_n + 1];
                 }
             }
-            const bool on = rr >= 0;
+            float u[D], uu = 0.f;
+#pragma unroll
+            for (int l = 0; l < D; l++) {
+                u[l] = rr >= 0 ? xq[l] - ctr[l] : 0.f;
+                uu += u[l] * u[l];
+            }
+            // a source that is infinite or not a number is within eps of no target
+            // and takes no slot: its column times 0 would not be 0
+            const bool on = rr >= 0 && uu < INFINITY;
             const float w = on ? (float)(e - j) : 0.f;  // exact: < 2^24
-            float uu = 0.f;
 #pragma unroll
             for (int l = 0; l < D; l++) {
                 float sv, cv;
                 sincosm1_small(on ? xq[l] - a0[l] : 0.f, sv, cv);
                 s.col[l][lane] = w * sv;
                 s.col[D + 1 + l][lane] = w * cv;
-                const float u = on ? xq[l] - ctr[l] : 0.f;
-                s.u[l][lane] = u;
-                uu += u * u;
+                s.u[l][lane] = on ? u[l] : 0.f;
             }
             s.col[D][lane] = w;
             s.u[D][lane] = on ? -(uu * inv_m) : kNever;

@@ -210,7 +210,10 @@ int egg_sync_build_grid_device(const float *d_D, int64_t n, int32_t d, float eps
  * order) visited in order d_order_in (NULL = identity): writes d_next (n x d,
  * point-id order), d_order_out[n] and, per sorted position, d_N, d_half,
  * d_border, d_synced (each may be NULL); *flag_local / *flag_final (host) as
- * the reference's r_local before / after the extra check. */
+ * the reference's r_local before / after the extra check.  The positions are
+ * taken as they are: a point outside [0,1] belongs to the grid's nearest cell (a
+ * NaN to cell 0), one that is not finite or far outside is within eps of nothing,
+ * and other points move as without it, except that its cell's totals hold it. */
 int egg_sync_iteration_device(const float *d_D, int64_t n, int32_t d, float eps,
                               const int32_t *d_order_in, float *d_next, int32_t *d_order_out,
                               int32_t *d_N, int32_t *d_half, int32_t *d_border,

@@ -597,3 +597,49 @@ def test_sync_pass_on_both_sides_of_the_lane_form(S, d):
     two = S.solve(Z, eps, stop_rule=nat.STOP_RC, lam=1.5, max_iter=1)
     assert np.abs(two["X"][:n] - one["X"]).max() <= 1e-6
     assert abs(two["stats"]["rc"] - one["stats"]["rc"]) <= 1e-7
+
+
+BAD = (np.nan, np.inf, -np.inf, 1e20, -1e20, 1e6, -3e5, 2e4)
+
+
+def _equal_where_finite(a, b, X):
+    """The pass a against the oracle's b: the order, N, half and synced of every point, border and the
+    positions of the points that are finite and in the grid, with non-numbers at the same places."""
+    good = ((X >= 0) & (X <= 1)).all(1)
+    at = good[b["order"]]
+    assert np.array_equal(a["order"], b["order"])
+    for k in ("N", "half", "synced"):
+        assert np.array_equal(a[k][at], b[k][at]), k
+    assert np.array_equal(a["border"][at], b["border"][at])
+    assert a["flag_local"] == b["flag_local"]
+    x, y = a["X_next"][good], b["X_next"][good]
+    assert np.array_equal(np.isfinite(x), np.isfinite(y))
+    ok = np.isfinite(x) & np.isfinite(y)
+    assert np.abs(x[ok] - y[ok]).max() <= 1e-6
+    return good
+
+
+@pytest.mark.parametrize("d", [1, 2, 3, 4, 5])
+def test_dense_update_keeps_bad_coordinates_to_their_points(S, O, d):
+    """A single pass takes its input as it is.  Points with a coordinate that is no number, infinite or
+    far out of the grid are neighbours of nothing: every other point moves as the oracle's does
+    (1e-6, as in test_iteration_bit_exact).  A dense grid whose occupied cells include those that
+    bad coordinates fall in (0 and the last): a full cell's totals hold the bad point, as in the reference, but no point that
+    tests its neighbours one by one takes anything from it.  The largest cells of d = 1 and 2 hold heavy
+    ranges (more than 4,096 runs)."""
+    eps = 0.1 * np.sqrt(d)
+    rng = np.random.default_rng(150 + d)
+    for n, width in {1: ((4000, 0.3), (60000, 0.12)), 2: ((4000, 0.3), (60000, 0.12)),
+                     3: ((4000, 0.3), (20000, 0.3)), 4: ((6000, 0.2), (20000, 0.25)),
+                     5: ((20000, 0.2),)}[d]:
+        X = (width * rng.random((n, d))).astype(f32)
+        X[n // 2:] = f32(1) - X[n // 2:]
+        for k, v in enumerate(BAD):
+            for l in range(d):
+                X[97 * k + l, l] = f32(v)
+                X[n // 2 + 97 * k + l, l] = f32(v)
+        X = X[rng.permutation(n)]
+        _say("dense update, bad coordinates", d, n)
+        b = O.egg_iteration(X, eps)
+        good = _equal_where_finite(S.iteration(X, eps), b, X)
+        assert np.isfinite(b["X_next"][good]).any()
