@@ -93,13 +93,17 @@ size_t pair_scratch_bytes(size_t n, size_t d) {
 }
 
 // The runs' rows, the cells' totals (at their first runs) and the blocks' boxes;
-// one wavefront per four blocks.
+// one wavefront per four blocks.  A coordinate that is not a number, or farther out
+// than PairBounds::far, becomes `far` in its row: the pair loop evaluates rows of
+// runs that its target does not count, with weight 0, which is nothing only of a
+// finite term.
 template <int D>
 __global__ __launch_bounds__(kBlock) void k_run_boxes(
     const float *__restrict__ Xs, const int *__restrict__ run_start,
     const int *__restrict__ point_cell, const int *__restrict__ cell_run,
     const int *__restrict__ cell_start, const int *__restrict__ cell_g,
-    const float *__restrict__ Ts, const float *__restrict__ Tc, Geo g, DevState *st, PairData p) {
+    const float *__restrict__ Ts, const float *__restrict__ Tc, Geo g, DevState *st, PairData p,
+    float far) {
     if (st->done || st->sparse_count == 0) return;
     constexpr int NC = (2 * D + 3) / 4;
     const int n = g.n, runs = st->runs, lane = __lane_id();
@@ -120,7 +124,7 @@ __global__ __launch_bounds__(kBlock) void k_run_boxes(
                 const float x = Xs[(long long)l * n + i];
                 lo[l] = hi[l] = x;
                 clamped |= x / g.cs >= wf;  // cell_coord's clamp of w to w-1
-                row[l] = x;
+                row[l] = fabsf(x) <= far ? x : far;
                 row[D + l] = ((float)cell_g[(long long)l * n + c] + 0.5f) * g.cs;
             }
             f = (cell_run[c] == r ? 1 : 0) | (clamped ? 2 : 0);
@@ -234,6 +238,7 @@ struct PairBounds {
     float thr_filter, thr_clamp;  // squared filter radii, of clamped sources
     float r, rounding;            // larger filter radius; relative error of the MFMA distance
     float lo, hi;                 // face distances less D h^2 surely <= / > thr_eps
+    float far;                    // points with a coordinate beyond it are near no other
 };
 
 constexpr int kPairTargets = 16;  // targets of a tile, four lanes each
@@ -364,15 +369,19 @@ __attribute__((amdgpu_waves_per_eu(D <= 3 ? 4 : (D <= 8 ? 3 : 1)))) void k_updat
         const int own = cell_start[c0 + 1] - cell_start[c0];
         // full cells' totals and partial cells' terms, on each of the four lanes
         float x[D], sum[D], sml[D];
-        bool border = false;
+        bool border = false, near = active;  // near: not a target that counts nothing
         float rho = 0.f;
 #pragma unroll
         for (int l = 0; l < D; l++) {
             x[l] = Xs[(long long)l * n + i];
             sum[l] = sml[l] = 0.f;
             border |= on_border(x[l], g.cs);
-            float tlo = active ? x[l] : __builtin_inff();
-            float thi = active ? x[l] : -__builtin_inff();
+            near = near && fabsf(x[l]) <= pb.far;
+        }
+#pragma unroll
+        for (int l = 0; l < D; l++) {
+            float tlo = near ? x[l] : __builtin_inff();
+            float thi = near ? x[l] : -__builtin_inff();
             for (int o = kWave / 2; o > 2; o >>= 1) {
                 tlo = fminf(tlo, __shfl_xor(tlo, o, kWave));
                 thi = fmaxf(thi, __shfl_xor(thi, o, kWave));
@@ -411,7 +420,7 @@ __attribute__((amdgpu_waves_per_eu(D <= 3 ? 4 : (D <= 8 ? 3 : 1)))) void k_updat
                     bf[l / 4] = -2.f * u;
                 }
             }
-            const bool on = t * kPairTargets + j16 < count;
+            const bool on = __shfl(near, 4 * j16, kWave);
             if (kq == 0) b1 = on ? u2 - pb.thr_filter - slack : 1e30f;
         }
         const float one_last = 4 * (KD - 1) + kq < D ? 1.f : 0.f;
@@ -650,6 +659,9 @@ static PairBounds pair_bounds(const Geo &g) {
     const double r = (double)g.eps + std::sqrt((double)g.d) * gap;
     p.thr_clamp = std::max(p.thr_filter, (float)(r * r * (1.0 + 0x1p-10)));
     p.r = (float)(std::sqrt((double)p.thr_clamp) * (1.0 + 0x1p-20));
+    // what a target counts lies in the grid, or within the filter radius of a target
+    // within eps of it
+    p.far = 2.0f + 2.0f * (g.eps + p.r);
     p.rounding = (float)((4 * g.d + 32) * 0x1p-24);
     const double m = 0x1p-24 * (16.0 * std::sqrt((double)g.d) / (double)g.eps + 12.0 * g.d + 64.0);
     const double dh2 = 0.25 * g.d * (double)g.cs * (double)g.cs;
@@ -677,7 +689,7 @@ void launch_update_pairs(const Geo &g, GridBufs &b, int *rdbg, DevState *st, hip
     case DD:                                                                                   \
         k_run_boxes<DD><<<pb, kBlock, 0, s>>>(b.Xs, b.run_start, b.point_cell, b.cell_run,     \
                                               b.cell_start, b.cell_g, b.Ts, b.Tc, g, st,       \
-                                              data);                                           \
+                                              data, bounds.far);                               \
         k_super_boxes<DD><<<sb, kBlock, 0, s>>>(g, st, data);                                  \
         if (pair_small) PAIR_LAUNCH(DD, true);                                                 \
         else PAIR_LAUNCH(DD, false);                                                           \

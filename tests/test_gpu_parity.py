@@ -643,3 +643,22 @@ def test_dense_update_keeps_bad_coordinates_to_their_points(S, O, d):
         b = O.egg_iteration(X, eps)
         good = _equal_where_finite(S.iteration(X, eps), b, X)
         assert np.isfinite(b["X_next"][good]).any()
+
+
+@pytest.mark.parametrize("d", [2, 3, 6, 8, 14])
+def test_pair_update_keeps_bad_coordinates_to_their_points(S, O, d):
+    """As above in a sparse grid, also where a bad point is in the same tile of targets or batch of
+    sources as others; none shares a cell with them."""
+    eps = {2: 0.02, 3: 0.05, 6: 0.15, 8: 0.2, 14: 0.25}[d]
+    rng = np.random.default_rng(140 + d)
+    X = (0.35 + 0.3 * rng.random((3000, d))).astype(f32)
+    for k, v in enumerate(BAD):
+        for l in range(d):
+            X[100 * k + l, l] = f32(v)   # in every dimension, the others a point's
+        X[100 * k + 50, :] = f32(v)
+    X[900, 0], X[900, d - 1] = np.nan, np.inf
+    X = X[rng.permutation(len(X))]
+    _say("pair update, bad coordinates", d)
+    b = O.egg_iteration(X, eps)
+    good = _equal_where_finite(S.iteration(X, eps), b, X)
+    assert np.isfinite(b["X_next"][good]).all() and b["N"].max() > 8
