@@ -104,9 +104,13 @@ struct Candidates {
         return true;
     }
 
-    // Point f of the loaded ranges (f < total): the last range whose offset is
-    // <= f (empty ranges share their successor's offset).
-    __device__ __forceinline__ int point(int f) const {
+    // Point f of the loaded ranges (f < total), of the 64 from a uniform f0 on the
+    // lane's (the last lanes may share one): the last range whose offset is <= f
+    // (empty ranges share their successor's offset).  In dense cells all 64 are in one.
+    __device__ __forceinline__ int point(int f, int f0) const {
+        const int k0 = __popcll(__ballot(rp <= f0)) - 1;
+        if (k0 == kWave - 1 || __builtin_amdgcn_readlane(rp, k0 + 1) >= min(f0 + kWave, total))
+            return __builtin_amdgcn_readlane(rj, k0) + f;
         int k = 0;
 #pragma unroll
         for (int s = kWave / 2; s > 0; s >>= 1)

@@ -86,7 +86,7 @@ __global__ __launch_bounds__(kBlock) void k_lonely(
     bool found = false;
     while (!found && cand.more()) {
         const int f = cand.f0 + lane;
-        const int j = cand.point(min(f, cand.total - 1));
+        const int j = cand.point(min(f, cand.total - 1), cand.f0);
         cand.f0 += kWave;
         found = __any(f < cand.total && j != i && point_dist2<D>(x, Xs, n, j) <= g.thr_eps);
     }
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(kLabBlock) void k_labels_sync(
         while (cand.more()) {
             for (int f0 = t - __lane_id(); f0 < cand.total; f0 += kLabBlock) {
                 const int f = f0 + __lane_id();
-                const int j = cand.point(min(f, cand.total - 1));
+                const int j = cand.point(min(f, cand.total - 1), f0);
                 if (f < cand.total && j != si && point_dist2<D>(x, Xs, n, j) <= g.thr_eps) {
                     labels[perm_s[j]] = cl;
                     any = true;

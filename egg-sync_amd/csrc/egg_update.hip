@@ -1699,7 +1699,11 @@ __global__ __launch_bounds__(kBlock) void k_extra_mbr(
 // SynC pass over the grid (SynC.cpp:16-56): every point within FP32 distance
 // eps (candidates: Chebyshev radius R+1 in the outer dimensions, which contains
 // every such point) contributes sinf(x_j - x) to the update and
-// expf(-|x_j - x|) to r_p, in ascending sorted position.
+// expf(-|x_j - x|) to r_p, in ascending sorted position.  Targets are the runs of
+// equal positions, whose points have the same sums; k_sync_points hands the results to
+// the points.  A target per point took 6 to 20 times as long on final positions, with
+// tens to hundreds of points to a run: r_c at n = 100,000, d = 3, eps = 0.02: 7.7 ms,
+// here 0.9; n = 400,000 31.9 and 3.0.
 //
 // A workgroup takes T consecutive targets, a wavefront each.  In a round every
 // wavefront tests its target's next S candidates, one per lane, packs the
@@ -1711,56 +1715,77 @@ __global__ __launch_bounds__(kBlock) void k_extra_mbr(
 // coordinate) once per 64 accepted pairs, ~40 instructions per 64 tested ones.
 // One thread per target ran the terms for every candidate any of 64 lanes
 // accepted, and 8,000 targets filled 125 of 1,024 SIMDs: n = 8,000, d = 2,
-// eps = 0.05: 3,760 us a pass, here 167.
+// eps = 0.05: 3,760 us a pass, here 154.
+//
+// Which form (kLaneMin): k_update_sync_lane gives each target a lane, which adds its
+// neighbours by itself.  It tests a candidate in fewer instructions, but its
+// wavefronts run the terms of every candidate any lane accepts, and end with their
+// longest list.  Wavefront / lane form, ms of a pass with its grid build, blobs as
+// given, eps = 0.002 to 0.1:
+//   n        d = 1      2        3        4        6
+//   65,536   1.3/2.7  4.1/10   2.4/6.4  5.8/52   3.7/18
+//   131,072  2.6/3.3  14/20    7.7/12   20/56    11/48
+//   200,000  4.9/4.7  22/22    19/32    43/86    24/76
+//   400,000  18/13    79/56    67/63    173/246  78/177
+// and of r_c alone at d = 1 0.73/1.5, 1.25/1.33 (n = 100,000), 1.74/1.79, 3.4/2.2.
+// From d = 3 on the line could lie higher; it is where d = 1 and 2 are even.
 template <int D, bool WRITE>
 struct SyncShape {
     static constexpr int NC = WRITE ? D + 1 : 1;             // terms per pair
     static constexpr int T = NC <= 17 ? 16 : 8;              // targets, and wavefronts
     static constexpr int S = NC <= 4 ? 128 : 64;             // candidates per round
     static constexpr int kThreads = T * kWave;
+    // from this many targets on a lane each (k_update_sync_lane)
+    static constexpr int kLaneMin = D == 1 && !WRITE ? 3 << 15 : 1 << 17;
+    static constexpr int P = S + 4;                          // row of a target's terms: 4 banks
+                                                             // apart for the adding lanes
     static constexpr int kAdders = (D * T + kWave - 1) / kWave;
-    static_assert(2 * T * S * NC * 4 <= 144 * 1024, "LDS");
+    static_assert(2 * T * (P * NC + 1) * 4 <= 160 * 1024, "LDS");
     static_assert(!WRITE || kAdders < T, "the last wavefront adds r_p");
+    // workgroups of at most n targets, fewer than kLaneMin
+    static int blocks(int n) { return (std::min(n, kLaneMin - 1) + T - 1) / T; }
 };
 
 template <int D, bool WRITE>
 __global__ __launch_bounds__((SyncShape<D, WRITE>::kThreads))
 __attribute__((amdgpu_waves_per_eu(D <= 8 ? 8 : 4))) void k_update_sync(
-    const float *__restrict__ Xs, float *__restrict__ Xout, const int *__restrict__ perm_s,
-    int *__restrict__ perm_out, const int *__restrict__ point_cell,
-    const int *__restrict__ cell_start, const int *__restrict__ cell_g,
-    const int *__restrict__ ob, const int *__restrict__ oe, Geo g, const DevState *st,
-    double *__restrict__ ratio) {
+    const float *__restrict__ Xs, const int *__restrict__ run_start,
+    const int *__restrict__ point_cell, const int *__restrict__ cell_start,
+    const int *__restrict__ cell_g, const int *__restrict__ ob, const int *__restrict__ oe, Geo g,
+    const DevState *st, float *__restrict__ rres, double *__restrict__ ratio) {
     if (WRITE && st->done) return;
     using Sh = SyncShape<D, WRITE>;
-    constexpr int T = Sh::T, S = Sh::S, NC = Sh::NC;
-    __shared__ float s_term[2][NC][T * S];
+    constexpr int T = Sh::T, S = Sh::S, P = Sh::P, NC = Sh::NC;
+    const int runs = st->runs;
+    if ((int)blockIdx.x * T >= runs || runs >= Sh::kLaneMin) return;
+    __shared__ __align__(16) float s_term[2][NC][T * P];
     __shared__ int s_cnt[2][T];
     const int n = g.n, lane = __lane_id();
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int i = blockIdx.x * T + w;  // this wavefront's target
+    const int target = blockIdx.x * T + w;  // this wavefront's run
+    const int i = run_start[min(target, runs - 1)];
     float x[D];
     Candidates<D> cand;
 #pragma unroll
-    for (int l = 0; l < D; l++) x[l] = Xs[(long long)l * n + min(i, n - 1)];
-    cand.init(g, cell_g, cell_start, ob, oe, point_cell[min(i, n - 1)], g.R + 1);
+    for (int l = 0; l < D; l++) x[l] = Xs[(long long)l * n + i];
+    cand.init(g, cell_g, cell_start, ob, oe, point_cell[i], g.R + 1);
     // the adding lanes' target and coordinate; the last wavefront adds r_p
     const int at = lane % T, ac = w * (kWave / T) + lane / T;
     const bool adds = WRITE && w < Sh::kAdders && ac < D, adds_r = w == T - 1 && lane < T;
     float sum = 0.f;
     double r = 0.0;
     int N = 0;
-    bool left = i < n;
+    bool left = target < runs;
     for (int k = 0;; k++) {
         int cnt = 0;
         if (left) {
-            float(*term)[T * S] = s_term[k & 1];
+            float(*term)[T * P] = s_term[k & 1];
             for (int step = 0; step < S / kWave; step++) {
                 left = cand.more();
                 if (!left) break;
                 const int f = cand.f0 + lane;
                 const bool in_range = f < cand.total;
-                const int j = cand.point(min(f, cand.total - 1));
+                const int j = cand.point(min(f, cand.total - 1), cand.f0);
                 cand.f0 += kWave;
                 float df[D], s = 0.f;
 #pragma unroll
@@ -1771,7 +1796,7 @@ __attribute__((amdgpu_waves_per_eu(D <= 8 ? 8 : 4))) void k_update_sync(
                 const bool in = in_range && s <= g.thr_eps;
                 const unsigned long long m = __ballot(in);
                 if (in) {
-                    const int e = w * S + cnt + __popcll(m & lanemask_lt());
+                    const int e = w * P + cnt + __popcll(m & lanemask_lt());
                     if (WRITE) {
 #pragma unroll
                         for (int l = 0; l < D; l++) term[l][e] = df[l];
@@ -1782,7 +1807,7 @@ __attribute__((amdgpu_waves_per_eu(D <= 8 ? 8 : 4))) void k_update_sync(
             }
             wave_sync();
             for (int q = lane; q < cnt; q += kWave) {
-                const int e = w * S + q;
+                const int e = w * P + q;
                 if (WRITE) {
 #pragma unroll
                     for (int l = 0; l < D; l++) term[l][e] = sinf(term[l][e]);
@@ -1793,7 +1818,7 @@ __attribute__((amdgpu_waves_per_eu(D <= 8 ? 8 : 4))) void k_update_sync(
         if (lane == 0) s_cnt[k & 1][w] = cnt;
         if (k > 0 && (adds || adds_r)) {
             const int b = (k - 1) & 1, c = s_cnt[b][at];
-            const float *t = s_term[b][adds ? ac : NC - 1] + at * S;
+            const float *t = s_term[b][adds ? ac : NC - 1] + at * P;
             N += c;
             for (int q0 = 0; q0 < c; q0 += 8) {
                 float v[8];
@@ -1813,32 +1838,28 @@ __attribute__((amdgpu_waves_per_eu(D <= 8 ? 8 : 4))) void k_update_sync(
         // one more round than the longest candidate list, to add its last terms
         if (!__syncthreads_or(left || cnt > 0)) break;
     }
-    const int ia = blockIdx.x * T + at;
-    if (adds && ia < n) Xout[(long long)ac * n + ia] = Xs[(long long)ac * n + ia] + sum / (float)N;
-    if (adds_r && ia < n) {
-        ratio[ia] = N > 0 ? r / (double)N : 1.0;
-        if (WRITE) perm_out[ia] = perm_s[ia];
-    }
+    const int ra = blockIdx.x * T + at;
+    if (adds && ra < runs)
+        rres[(long long)ac * n + ra] = Xs[(long long)ac * n + run_start[ra]] + sum / (float)N;
+    if (adds_r && ra < runs) ratio[ra] = N > 0 ? r / (double)N : 1.0;
 }
 
 constexpr int kRcBlocks = 1024;
 
 // The same pass with a lane per target, each adding its neighbours one after the
-// other: k_update_sync spreads a target's candidates over a wavefront and so fills
-// the chip from a few thousand points on, but has a serial chain of additions for
-// each target with few lanes to share; once there are targets enough for every lane
-// of the chip, a lane's own chain hides behind the others'.
+// other (SyncShape::kLaneMin).
 template <int D, bool WRITE>
 __global__ __launch_bounds__(kBlock) void k_update_sync_lane(
-    const float *__restrict__ Xs, float *__restrict__ Xout, const int *__restrict__ perm_s,
-    int *__restrict__ perm_out, const int *__restrict__ point_cell,
-    const int *__restrict__ cell_start, const int *__restrict__ cell_g,
-    const int *__restrict__ ob, const int *__restrict__ oe, Geo g, const DevState *st,
-    double *__restrict__ ratio) {
+    const float *__restrict__ Xs, const int *__restrict__ run_start,
+    const int *__restrict__ point_cell, const int *__restrict__ cell_start,
+    const int *__restrict__ cell_g, const int *__restrict__ ob, const int *__restrict__ oe, Geo g,
+    const DevState *st, float *__restrict__ rres, double *__restrict__ ratio) {
     if (WRITE && st->done) return;
-    const int n = g.n, od = g.od, R = g.R + 1;
+    const int n = g.n, od = g.od, R = g.R + 1, runs = st->runs;
+    if (runs < SyncShape<D, WRITE>::kLaneMin) return;
     const int *cg_od = cell_g + (long long)od * n;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < runs; t += gridDim.x * blockDim.x) {
+        const int i = run_start[t];
         float x[D], sum[D];
         int g0[D];
         const int c0 = point_cell[i];
@@ -1888,31 +1909,35 @@ __global__ __launch_bounds__(kBlock) void k_update_sync_lane(
         if (WRITE) {
 #pragma unroll
             for (int l = 0; l < D; l++) {
-                const float t = sum[l] / (float)N;
-                Xout[(long long)l * n + i] = x[l] + t;
+                const float mean = sum[l] / (float)N;
+                rres[(long long)l * n + t] = x[l] + mean;
             }
-            perm_out[i] = perm_s[i];
         }
-        ratio[i] = N > 0 ? r / (double)N : 1.0;
+        ratio[t] = N > 0 ? r / (double)N : 1.0;
     }
 }
 
-// From this many points on the SynC pass takes k_update_sync_lane.  Wavefront /
-// lane form, ms a pass on blobs as given and, second, converged: n = 65,536 at d = 2
-// 3.1 / 7.6 and 3.5 / 4.2, at d = 3 1.8 / 5.7 and 3.6 / 7.0; n = 131,072 10.9 / 12.3
-// and 11.8 / 8.0, 6.4 / 9.9 and 13.4 / 8.1; n = 200,000 18 / 13 and 27 / 17, 16 / 31
-// and 29 / 11; n = 1,000,000, d = 3, converged 702 / 197.
-constexpr int kSyncLaneMin = 1 << 17;
-
-// Block partial sums of the points' r_p / N, combined in a fixed order by
-// k_rc_finish, so r_c is deterministic.
-__global__ __launch_bounds__(kBlock) void k_rc_sum(const double *__restrict__ ratio, int n,
-                                                   const DevState *st, bool guard,
-                                                   double *__restrict__ rc_part) {
-    if (guard && st->done) return;
+// A run's results to its points: with `write` the new positions (and the point ids,
+// for the next grid build's order), and block partial sums of the points' r_p / N,
+// combined in a fixed order by k_rc_finish, so r_c is deterministic.
+__global__ __launch_bounds__(kBlock) void k_sync_points(const int *__restrict__ point_run,
+                                                        const double *__restrict__ ratio,
+                                                        const float *__restrict__ rres,
+                                                        const int *__restrict__ perm_s, int n,
+                                                        int d, bool write, const DevState *st,
+                                                        float *__restrict__ Xout,
+                                                        int *__restrict__ perm_out,
+                                                        double *__restrict__ rc_part) {
+    if (write && st->done) return;
     double racc = 0.0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        racc += ratio[i];
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const int r = point_run[i];
+        racc += ratio[r];
+        if (write) {
+            for (int l = 0; l < d; l++) Xout[(long long)l * n + i] = rres[(long long)l * n + r];
+            perm_out[i] = perm_s[i];
+        }
+    }
     __shared__ double s_r[kBlock / kWave];
 #pragma unroll
     for (int o = kWave / 2; o > 0; o >>= 1) racc += __shfl_xor(racc, o, kWave);
@@ -2033,27 +2058,30 @@ int rc_partials(int n) { return kRcBlocks; }
 void launch_update_sync(const Geo &g, GridBufs &b, DevState *st, double *rc_part, bool write_pos,
                         hipStream_t s) {
     double *ratio = (double *)b.rdbg;  // [n] of its 4n ints, unused by this pass
-#define SY_LAUNCH(DD, W, X, P)                                                                    \
-    if (g.n >= kSyncLaneMin)                                                                      \
-        k_update_sync_lane<DD, W><<<kRcBlocks, kBlock, 0, s>>>(                                   \
-            b.Xs, X, b.perm_s, P, b.point_cell, b.cell_start, b.cell_g, b.ob, b.oe, g, st, ratio); \
-    else k_update_sync<DD, W><<<(g.n + SyncShape<DD, W>::T - 1) / SyncShape<DD, W>::T,                 \
-                           SyncShape<DD, W>::kThreads, 0, s>>>(                                   \
-        b.Xs, X, b.perm_s, P, b.point_cell, b.cell_start, b.cell_g, b.ob, b.oe, g, st, ratio)
-#define SY_CASE(DD)                                       \
-    case DD:                                              \
-        if (write_pos) {                                  \
-            SY_LAUNCH(DD, true, b.X, b.perm);             \
-        } else {                                          \
-            SY_LAUNCH(DD, false, nullptr, nullptr);       \
-        }                                                 \
+    // the number of targets is on the device: each form returns at the other's numbers
+#define SY_ARGS                                                                                   \
+    b.Xs, b.run_start, b.point_cell, b.cell_start, b.cell_g, b.ob, b.oe, g, st, b.rres, ratio
+#define SY_LAUNCH(DD, W)                                                                          \
+    k_update_sync<DD, W><<<SyncShape<DD, W>::blocks(g.n), SyncShape<DD, W>::kThreads, 0, s>>>(     \
+        SY_ARGS);                                                                                 \
+    if (g.n >= SyncShape<DD, W>::kLaneMin)                                                        \
+        k_update_sync_lane<DD, W><<<kRcBlocks, kBlock, 0, s>>>(SY_ARGS)
+#define SY_CASE(DD)                     \
+    case DD:                            \
+        if (write_pos) {                \
+            SY_LAUNCH(DD, true);        \
+        } else {                        \
+            SY_LAUNCH(DD, false);       \
+        }                               \
         break;
     switch (g.d) {
         EGG_EACH_D(SY_CASE)
     }
 #undef SY_CASE
 #undef SY_LAUNCH
-    k_rc_sum<<<kRcBlocks, kBlock, 0, s>>>(ratio, g.n, st, write_pos, rc_part);
+#undef SY_ARGS
+    k_sync_points<<<kRcBlocks, kBlock, 0, s>>>(b.point_run, ratio, b.rres, b.perm_s, g.n, g.d,
+                                               write_pos, st, b.X, b.perm, rc_part);
     k_rc_finish<<<1, kBlock, 0, s>>>(rc_part, kRcBlocks, g.n, st, write_pos);
 }
 

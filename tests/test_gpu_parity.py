@@ -662,3 +662,60 @@ def test_pair_update_keeps_bad_coordinates_to_their_points(S, O, d):
     b = O.egg_iteration(X, eps)
     good = _equal_where_finite(S.iteration(X, eps), b, X)
     assert np.isfinite(b["X_next"][good]).all() and b["N"].max() > 8
+
+
+@pytest.mark.parametrize("d,eps", [(1, 0.002), (2, 0.02), (4, 0.1), (6, 0.2)])
+def test_sync_forms_give_the_same_bits(S, d, eps):
+    """The SynC pass with a wavefront per target and with a lane per target (from 2^17 targets on): 2^16
+    points alone and beside a copy far away, on grids of the same outer dimensions, so that every
+    point of the first copy meets the same neighbours in the same order.  The second copy's cells lie
+    otherwise and its FP32 sums are in another order (1e-6, as in test_iteration_bit_exact); r_c is a
+    mean of 64-bit sums of the same terms."""
+    nat = S.nat
+    rng = np.random.default_rng(160 + d)
+    n = 1 << 16
+    X = rng.random((n, d)).astype(f32)
+    # no two alike; + 0.5 is exact, and so are the differences of the copy
+    X[:, 0] = rng.permutation(1 << 21)[:n].astype(f32) * f32(2.0 ** -23)
+    Y = X.copy()
+    Y[:, 0] += f32(0.5)
+    Z = np.concatenate([X, Y])
+    assert nat.geometry(n, d, eps)["od"] == nat.geometry(2 * n, d, eps)["od"]
+    _say("sync forms", Z.shape)
+    one = S.solve(X, eps, stop_rule=nat.STOP_RC, label_rule=nat.LABELS_CELLS, lam=1.5, max_iter=1)
+    two = S.solve(Z, eps, stop_rule=nat.STOP_RC, label_rule=nat.LABELS_CELLS, lam=1.5, max_iter=1)
+    assert np.array_equal(two["X"][:n], one["X"])
+    Y1 = one["X"].copy()
+    Y1[:, 0] += f32(0.5)
+    assert np.abs(two["X"][n:] - Y1).max() <= 1e-6
+    assert abs(two["stats"]["rc"] - one["stats"]["rc"]) <= 1e-12
+    assert abs(S.rc(Z, eps) - S.rc(X, eps)) <= 1e-12
+
+
+@pytest.mark.parametrize("d,times", [(1, 3), (2, 63), (2, 64), (3, 5), (5, 70)])
+def test_sync_pass_of_repeated_points(S, d, times):
+    """Targets of the SynC pass are runs of equal positions, below and above 2^17 points.  Repeating
+    every point leaves the means as they are; a sum of N terms of at most eps in FP32 is within
+    N * 2^-24 of the terms' bound per term of its mean, and r_c's terms within 4 * 2^-24."""
+    nat = S.nat
+    rng = np.random.default_rng(170 + d)
+    eps = {1: 0.01, 2: 0.05, 3: 0.1, 5: 0.25}[d]
+    P = rng.random((2048, d)).astype(f32)
+    X = np.repeat(P, times, axis=0)[rng.permutation(2048 * times)]
+    s = np.zeros((2048, 2048), f32)
+    for l in range(d):
+        df = P[:, None, l] - P[None, :, l]
+        s = s + df * df
+    near = np.sqrt(s) <= f32(eps)
+    N = near.sum(1)
+    want = np.stack([P[:, l] + (np.sin(P[None, :, l].astype(np.float64) - P[:, None, l]) * near)
+                     .sum(1) / N for l in range(d)], 1)
+    rc = ((np.exp(-np.sqrt(s.astype(np.float64))) * near).sum(1) / N).mean()
+    _say("sync pass, repeated points", d, times)
+    got = S.solve(X, eps, stop_rule=nat.STOP_RC, label_rule=nat.LABELS_CELLS, lam=1.5, max_iter=1)
+    key = {p.tobytes(): k for k, p in enumerate(P)}
+    at = np.array([key[x.tobytes()] for x in X])
+    tol = (N * times * eps + 1) * 2.0 ** -24
+    assert (np.abs(got["X"] - want[at]) <= tol[at][:, None]).all()
+    assert abs(got["stats"]["rc"] - rc) <= 2.0 ** -22
+    assert abs(S.rc(X, eps) - rc) <= 2.0 ** -22
