@@ -418,7 +418,7 @@ __device__ __forceinline__ void stream_chunk(int base, int total, int r0, int s0
             }
             if (sq <= thr) {
                 const int lk = len[k];
-                const float w = (float)lk;  // exact: lk < 2^24
+                const float w = (float)lk;  // of 2^24 points on within 2^-24; the count is exact
 #pragma unroll
                 for (int l = 0; l < D; l++) {
                     const float a = w * qq.sv[l];
@@ -507,6 +507,7 @@ __device__ __forceinline__ bool finish_run(const float (&x)[D], const float (&su
 
 // The matrix path (egg_stream.h) serves up to kStreamMaxD dimensions and n < 2^24.
 constexpr int kStreamMaxD = 5;
+static_assert(kStreamMaxD <= kHeavyMaxD, "k_update_dense defers heavy ranges at every d");
 
 // A wavefront's LDS in k_update_heavy: sources of the scalar paths, or the matrix
 // path's chunk.

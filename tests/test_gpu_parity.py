@@ -719,3 +719,105 @@ def test_sync_pass_of_repeated_points(S, d, times):
     assert (np.abs(got["X"] - want[at]) <= tol[at][:, None]).all()
     assert abs(got["stats"]["rc"] - rc) <= 2.0 ** -22
     assert abs(S.rc(X, eps) - rc) <= 2.0 ** -22
+
+
+def _pass_rows(S, P, w, eps, rows):
+    """N, half, border, synced and the next position (64-bit sums) of the points `rows` in one pass over
+    the distinct points P, point k w[k] times: EGG_SynC.cu:583-709 from the source, with the points
+    of a cell visited together."""
+    n, d = int(w.sum()), P.shape[1]
+    g = S.nat.geometry(n, d, eps)
+    e, cs = f32(eps), f32(g["cs"])
+    gc = np.minimum(np.trunc(P / cs).astype(np.int64), g["w"] - 1)
+    key = gc @ (g["w"] ** np.arange(d))
+    _, first, of = np.unique(key, return_index=True, return_inverse=True)
+    cells = gc[first]
+    count = np.bincount(of, weights=w).astype(np.int64)
+    by_cell = np.argsort(of, kind="stable")
+    start = np.concatenate([[0], np.cumsum(np.bincount(of))])
+    out = []
+    for t in rows:
+        x, c0 = P[t], of[t]
+        near = (np.abs(cells[:, :g["od"]] - gc[t, :g["od"]]) <= g["R"]).all(1)
+        lo, hi = cells.astype(f32) * cs - x, (cells + 1).astype(f32) * cs - x
+        small = large = np.zeros(len(cells), f32)
+        for l in range(d):
+            u, v = lo[:, l] * lo[:, l], hi[:, l] * hi[:, l]
+            small, large = small + np.minimum(u, v), large + np.maximum(u, v)
+        full = near & (np.sqrt(large) <= e)
+        part = near & (np.sqrt(small) <= e) & ~full
+        xd, at = x.astype(np.float64), np.trunc(x / cs)
+        border = bool(((np.trunc((xd - 0.00001) / float(cs)) != at) |
+                       (np.trunc((xd + 0.00001) / float(cs)) != at)).any())
+        N = half = 0
+        move = np.zeros(d)
+        for c in np.nonzero(full | part)[0]:
+            j = by_cell[start[c]:start[c + 1]]
+            s = np.zeros(len(j), f32)
+            for l in range(d):
+                s = s + (x[l] - P[j, l]) * (x[l] - P[j, l])
+            if border and full[c]:
+                half += int(count[c] if c == c0 else w[j[np.sqrt(s).astype(float) <= float(e) / 2]].sum())
+            if part[c]:
+                j = j[np.sqrt(s) <= e]
+            N += int(w[j].sum())
+            move += (w[j, None] * np.sin(P[j].astype(np.float64) - xd)).sum(0)
+        out.append((N, half if border else -1, int(border), int(N == (half if border else count[c0])),
+                    xd + move / N))
+    return out
+
+
+def _check_pass_rows(S, P, w, eps, X, rng, k=150):
+    """A pass over the points X, of which the first are P: k random ones of these, and as many of those
+    in the band of the on-border test.  Counts and flags bit for bit, positions within 1e-6, as in
+    test_iteration_bit_exact."""
+    cs = S.nat.geometry(len(X), P.shape[1], eps)["cs"]
+    band = np.nonzero((np.abs(P / cs - np.round(P / cs)) * cs < 0.9e-5).any(1))[0]
+    rows = np.concatenate([rng.choice(len(P), k), rng.permutation(band)[:k]])
+    a = S.iteration(X, eps)
+    pos = np.empty(len(X), np.int64)
+    pos[a["order"]] = np.arange(len(X))
+    want = _pass_rows(S, P, w, eps, rows)
+    for t, (N, half, border, synced, x) in zip(rows, want):
+        q = pos[t]
+        assert (a["N"][q], a["border"][q], a["synced"][q]) == (N, border, synced), t
+        assert half < 0 or a["half"][q] == half, t
+        assert np.abs(a["X_next"][t] - x).max() <= 1e-6, t
+    assert max(half for _, half, *_ in want) > 0
+
+
+@pytest.mark.parametrize("d,m", [(1, 60_000), (2, 60_000), (3, 120_000), (4, 300_000),
+                                 (5, 700_000)])
+def test_update_from_2_24_points_on(S, d, m):
+    """From 2^24 points on the update sums on the vector ALUs, with counts that a float does not hold:
+    cells of about 9,000 distinct points (heavy ranges), each dozens of times."""
+    rng = np.random.default_rng(180 + d)
+    P = np.unique((0.12 * rng.random((m, d))).astype(f32), axis=0)
+    P = P[rng.permutation(len(P))]
+    times = (1 << 24) // len(P) + 1
+    _say("pass of", times, "times", P.shape)
+    _check_pass_rows(S, P, np.full(len(P), times), 0.1 * np.sqrt(d),
+                     torch.from_numpy(P).cuda().repeat(times, 1), rng, 150 if d < 4 else 30)
+
+
+def test_update_beside_a_run_of_more_than_2_24_points(S):
+    rng = np.random.default_rng(186)
+    P = (0.3 * rng.random((3000, 2))).astype(f32)
+    w = np.ones(len(P), np.int64)
+    w[0] += 1 << 24
+    D = torch.from_numpy(P).cuda()
+    _say("pass beside a run of", w[0])
+    _check_pass_rows(S, P, w, 0.15, torch.cat([D, D[:1].repeat(1 << 24, 1)]), rng)
+
+
+@pytest.mark.parametrize("n,eps", [(2_400_000, 0.02), (1 << 24, 0.004)])
+def test_update_with_the_heavy_queue_full(S, n, eps):
+    """More heavy ranges than the queue of 65,536 takes, in both forms of the update: each of n / 64 tiles
+    has two cells that hold neighbours in part, half a cell of more than 4,096 runs of each, and
+    border points count such ranges within eps / 2."""
+    rng = np.random.default_rng(190)
+    P = rng.permutation(1 << 24)[:n, None].astype(f32) * f32(2.0 ** -24)
+    w = S.nat.geometry(n, 1, eps)["w"]
+    assert 2 * (w - 4) / w * n / 64 > 65536 and n / (2 * w) > 4096
+    _say("pass of", n, "distinct points")
+    _check_pass_rows(S, P, np.ones(n, np.int64), eps, torch.from_numpy(P).cuda(), rng, 60)
