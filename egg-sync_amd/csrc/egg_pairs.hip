@@ -84,12 +84,7 @@ static PairData pair_data(const Geo &g, const GridBufs &b) {
 size_t pair_scratch_bytes(size_t n, size_t d) {
     const size_t nb = n / kBlkRuns + 1, ns = n / ((size_t)kBlkRuns * kSupBlks) + 1;
     auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
-    const size_t used = al(8 * d * n) + 2 * al(4 * d * nb) + 2 * al(4 * nb) + 2 * al(4 * d * ns) +
-                        al(4 * ns);
-    // not below what earlier layouts held, so that the workspace keeps its size
-    return std::max(used, al(4 * n) * 3 + al(4 * d * n) * 2 + al(4 * d * (n / 64 + 1)) * 2 +
-                              al(4 * (n / 64 + 1)) * 2 + al(4 * d * (n / 4096 + 1)) * 2 +
-                              al(4 * (n / 4096 + 1)));
+    return al(8 * d * n) + 2 * al(4 * d * nb) + 2 * al(4 * nb) + 2 * al(4 * d * ns) + al(4 * ns);
 }
 
 // The runs' rows, the cells' totals (at their first runs) and the blocks' boxes;

@@ -196,11 +196,6 @@ Layout carve(void *base, const Geo &g) {
     L.rc_trace = c.take<double>(kTraceCap);
     L.cells_trace = c.take<int>(kTraceCap);
     L.err = c.take<int>(1);
-    // room the solve does not use, so that the size of a workspace, and with it the
-    // largest n the fixed scratch array holds, stays what callers have sized for
-    const size_t wide = (std::max(n, hist) + kScanTile - 1) / kScanTile + 1;
-    c.off += 10 * align_up(4 * n) + align_up(4) + align_up(4 * (8 * wide + 20)) -
-             align_up(4 * (scan_tmp_ints((int)std::max(n, hist)) + 16));
     L.bytes = c.off;
     return L;
 }
@@ -235,6 +230,21 @@ static int check_scans(const Layout &L, hipStream_t s) {
 constexpr size_t kScratchBytes = (size_t)64 << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 void *g_scratch_ptr[64];
+
+// Whether a workload fits the scratch array.  Its callers have sized their data by an
+// earlier layout, with ten more ints a point, scans of wide tiles only and a pair
+// update of 64-run blocks; what that one refused stays refused.
+bool scratch_holds(const Geo &g, const Layout &L) {
+    const size_t n = (size_t)g.n, d = (size_t)g.d, m = std::max(n, sort_tmp_ints(g.n));
+    const size_t wide = (m + kScanTile - 1) / kScanTile + 1;
+    const size_t had = 10 * align_up(4 * n) + align_up(4) + align_up(4 * (8 * wide + 20)) +
+                       3 * align_up(4 * n) + 2 * align_up(4 * d * n) +
+                       2 * align_up(4 * d * (n / 64 + 1)) + 2 * align_up(4 * (n / 64 + 1)) +
+                       2 * align_up(4 * d * (n / 4096 + 1)) + align_up(4 * (n / 4096 + 1));
+    const size_t has = align_up(4 * (scan_tmp_ints((int)m) + 16)) +
+                       align_up(pair_scratch_bytes(n, d));
+    return L.bytes <= kScratchBytes && L.bytes + had <= kScratchBytes + has;
+}
 
 int scratch_base(void **out) {
     int dev = 0;
@@ -526,7 +536,7 @@ int solve_device_impl(const float *d_D, int64_t n64, int d, float eps,
         void *base = nullptr;
         rc = scratch_base(&base);
         if (rc) return rc;
-        if (carve(nullptr, g).bytes > kScratchBytes) return EGG_SYNC_E_TOO_BIG;
+        if (!scratch_holds(g, carve(nullptr, g))) return EGG_SYNC_E_TOO_BIG;
         L = carve(base, g);
     } else {
         rc = acquire(g, L, ws);

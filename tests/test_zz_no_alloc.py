@@ -72,3 +72,16 @@ def test_noalloc_rejects_too_large(nat):
     rc_b, lab_b, fin_b, _ = _call(nat, nat.lib().egg_sync_solve_device_noalloc, D2, eps2)
     assert rc_a == rc_b == 0
     assert np.array_equal(lab_a, lab_b) and np.array_equal(fin_a, fin_b)
+
+
+@pytest.mark.parametrize("d,eps,most", [(1, 0.01, 223_936), (3, 0.02, 138_524),
+                                        (8, 0.1, 84_834), (20, 0.3, 39_088)])
+def test_noalloc_limit_is_a_rule_of_its_own(nat, d, eps, most):
+    """The largest number of points it takes, fixed by an earlier layout, and one more.  The workspace
+    itself is smaller: it holds nothing that the solve does not use."""
+    X = (torch.randint(1, 10, (most + 1, 1)) / 10.0).repeat(1, d).cuda()
+    for n, code in ((most, 0), (most + 1, nat.E_TOO_BIG)):
+        _say("noalloc limit", n, d)
+        rc, _, _, st = _call(nat, nat.lib().egg_sync_solve_device_noalloc, X[:n], eps)
+        assert rc == code
+        assert code or st.workspace_bytes + 40 * n <= 64 << 20
