@@ -1738,10 +1738,12 @@ struct SyncShape {
     static constexpr int kThreads = T * kWave;
     // from this many targets on a lane each (k_update_sync_lane)
     static constexpr int kLaneMin = D == 1 && !WRITE ? 3 << 15 : 1 << 17;
-    static constexpr int P = S + 4;                          // row of a target's terms: 4 banks
-                                                             // apart for the adding lanes
+    // row of a target's terms: 4 banks apart for the adding lanes, 2 where 4 would cost
+    // the second workgroup of a CU its LDS (d = 18)
+    static constexpr int kLds = 160 * 1024, kRows = 8 * T * NC;
+    static constexpr int P = kLds / (kRows * (S + 4)) == kLds / (kRows * S) ? S + 4 : S + 2;
     static constexpr int kAdders = (D * T + kWave - 1) / kWave;
-    static_assert(2 * T * (P * NC + 1) * 4 <= 160 * 1024, "LDS");
+    static_assert(kRows * P + 8 * T <= kLds, "LDS");
     static_assert(!WRITE || kAdders < T, "the last wavefront adds r_p");
     // workgroups of at most n targets, fewer than kLaneMin
     static int blocks(int n) { return (std::min(n, kLaneMin - 1) + T - 1) / T; }
