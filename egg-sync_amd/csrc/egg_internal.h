@@ -13,7 +13,7 @@ void scan_exclusive(const int *in, int *out, int n, int *tmp, int *total, hipStr
 // kMaxScanCh channels, in scan_tmp_ints(n) ints of their own.  It must be zero
 // before the first of them (scan_tmp_reset, not for graph capture); each scan
 // leaves it ready for the next on the same stream.
-constexpr int kMaxScanCh = 4;
+constexpr int kMaxScanCh = 3;
 int scan_tmp_reset(int *tmp, int n, hipStream_t s);
 // Nonzero if a scan using tmp gave up waiting (an internal error).
 int scan_tmp_error(const int *tmp, hipStream_t s, int *err);
@@ -29,8 +29,9 @@ void rank_sort(const uint64_t *keys, int *sidx, int n, int kw, const int *run_st
 // 8 bits per pass.  keys_a/keys_b: [kw][n] u64; vals_a/vals_b: [n] int32.
 // On entry keys are in keys_a and vals are implicit (0..m-1), m = *n_dev
 // (<= n); *hist_n_dev must hold 256 * max(1, ceil(m / kSortTile)) (the
-// histogram entries of the tiles that hold elements).  Returns 0 if the sorted result is in the *_a buffers, 1 if
-// in *_b, -1 if no pass was needed (identity order).
+// histogram entries of the tiles that hold elements).  Returns 0 if the sorted
+// result is in the *_a buffers, 1 if in *_b, -1 if no pass was needed (identity
+// order).
 size_t sort_tmp_ints(int n);
 int radix_sort(uint64_t *keys_a, uint64_t *keys_b, int *vals_a, int *vals_b, int n, int kw,
                int key_bits, int *hist, int *scan_tmp, const DevState *st, hipStream_t s,
@@ -131,7 +132,6 @@ void launch_update_sync(const Geo &g, GridBufs &b, DevState *st, double *rc_part
                         hipStream_t s);
 int rc_partials(int n);
 void launch_set_flag(DevState *st, hipStream_t s);
-void launch_finish(DevState *st, hipStream_t s);
 
 // Labels (egg_labels.hip).
 void launch_labels_egg(const Geo &g, GridBufs &b, int *labels, DevState *st, hipStream_t s);

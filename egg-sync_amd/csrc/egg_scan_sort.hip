@@ -129,17 +129,17 @@ __device__ __forceinline__ int digit_of(const uint64_t *keys, int n, int e, int 
 }
 
 // Keys are stored with stride n ([kw][n]); the first m = min(n, *n_dev) of
-// them (all n without n_dev) are sorted.
+// them are sorted.
 __global__ __launch_bounds__(kBlock) void k_rs_hist(const uint64_t *__restrict__ keys, int n,
                                                     const int *n_dev, int shift,
-                                                    int *__restrict__ hist, int ntiles,
+                                                    int *__restrict__ hist,
                                                     const DevState *st) {
     if (st && st->done) return;
     __shared__ int h[256];
-    const int m = n_dev ? min(n, *n_dev) : n;
+    const int m = min(n, *n_dev);
     // tiles holding elements: the histogram's stride (its scan covers 256
     // of them per digit)
-    const int nt = n_dev ? max(1, (m + kSortTile - 1) / kSortTile) : ntiles;
+    const int nt = max(1, (m + kSortTile - 1) / kSortTile);
     if ((int)blockIdx.x >= nt) return;
     h[threadIdx.x] = 0;
     __syncthreads();
@@ -160,10 +160,10 @@ __global__ __launch_bounds__(kBlock) void k_rs_scatter(const uint64_t *__restric
                                                        int *__restrict__ vout, int n,
                                                        const int *n_dev, int shift,
                                                        const int *__restrict__ hist_scan,
-                                                       int ntiles, const DevState *st) {
+                                                       const DevState *st) {
     if (st && st->done) return;
-    const int m = n_dev ? min(n, *n_dev) : n;
-    const int nt = n_dev ? max(1, (m + kSortTile - 1) / kSortTile) : ntiles;
+    const int m = min(n, *n_dev);
+    const int nt = max(1, (m + kSortTile - 1) / kSortTile);
     if ((int)blockIdx.x >= nt) return;
     __shared__ int s_off[256];
     __shared__ int s_wc[kBlock / kWave][256];
@@ -365,12 +365,12 @@ int radix_sort(uint64_t *keys_a, uint64_t *keys_b, int *vals_a, int *vals_b, int
     int where = 0;
     for (int p = 0; p < passes; p++) {
         const int shift = p * 8;
-        k_rs_hist<<<ntiles, kBlock, 0, s>>>(kin, n, n_dev, shift, hist, ntiles, st);
+        k_rs_hist<<<ntiles, kBlock, 0, s>>>(kin, n, n_dev, shift, hist, st);
         launch_scan<1>(HistScan{hist, hist_n_dev}, 256 * ntiles, scan_tmp, st, s);
 #define RS_CASE(KW)                                                                          \
     case KW:                                                                                 \
         k_rs_scatter<KW><<<ntiles, kBlock, 0, s>>>(kin, vin, kout, vout, n, n_dev, shift,    \
-                                                   hist, ntiles, st);                        \
+                                                   hist, st);                                \
         break;
         switch (kw) {
             RS_CASE(1) RS_CASE(2) RS_CASE(3) RS_CASE(4)

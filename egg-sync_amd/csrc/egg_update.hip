@@ -1975,11 +1975,6 @@ __global__ void k_set_flag(DevState *st) {
     reset_pass_state(st);
 }
 
-__global__ void k_finish(DevState *st) {
-    if (st->done) return;
-    finish_iteration(st);
-}
-
 static inline int grid_for(long long n) {
     long long b = (n + kBlock - 1) / kBlock;
     if (b < 1) b = 1;
@@ -2089,7 +2084,5 @@ void launch_update_sync(const Geo &g, GridBufs &b, DevState *st, double *rc_part
 }
 
 void launch_set_flag(DevState *st, hipStream_t s) { k_set_flag<<<1, 1, 0, s>>>(st); }
-
-void launch_finish(DevState *st, hipStream_t s) { k_finish<<<1, 1, 0, s>>>(st); }
 
 }  // namespace egg
