@@ -60,12 +60,12 @@ struct BruteState {
 // SIMDs: n = 8,000, d = 3, eps = 0.05: 4,150 us a pass, here 140.
 template <int D>
 struct BruteShape {
-    // up to 64 KiB of LDS for d <= 7, so that two workgroups share a CU
+    // up to 68 KiB of LDS for d <= 7, so that two workgroups share a CU
     static constexpr int T = D <= 16 ? 16 : 8;        // targets, and wavefronts
     static constexpr int S = D <= 3 ? 128 : 64;       // sources per round
     static constexpr int kThreads = T * kWave;
     static constexpr int kAdders = ((D + 1) * T + kWave - 1) / kWave;  // adding wavefronts
-    static_assert(2 * T * S * (D + 1) * 4 <= 144 * 1024 && kAdders <= T, "LDS, adders");
+    static_assert(8 * (T * S * (D + 1) + T + D * S) <= 160 * 1024 && kAdders <= T, "LDS, adders");
 };
 
 template <int D>

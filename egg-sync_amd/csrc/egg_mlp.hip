@@ -522,7 +522,7 @@ struct AdamStep {
 };
 
 // The workgroups' gradients added in order, the Adam step on them, and the
-// loss.  64 parameters per workgroup (289 for the jump network, so that the
+// loss.  64 parameters per workgroup (291 for the jump network, so that the
 // whole chip reads the partials' 19 MB): its four wavefronts bring the
 // partials to LDS, the first adds them one after another.
 __global__ __launch_bounds__(kThreads) void k_train_finish(

@@ -232,7 +232,11 @@ __global__ __launch_bounds__(kBlock) void k_scan(IO io, int *lb, const DevState 
 // thread.  Wide tiles mean fewer steps of look-back, narrow ones more CUs at work:
 // the radix sort's 12,500 histogram values at n = 100,000 take 5.7 us narrow and
 // 7.2 wide, its 125,000 at n = 1,000,000 12.4 and 8.6; k_tables<3> takes 20 us
-// narrow and 38 wide at n = 100,000, 11 and 26 at n = 2,000.
+// narrow and 38 wide at n = 100,000, 11 and 26 at n = 2,000.  The tables' line
+// (kTablesNarrowMax) lies where the forms are even: a features call at d = 3, which has
+// two such scans, takes 240 us narrow and 262 wide at n = 131,072, 288 and 289 at
+// 262,144, 351 and 320 at 400,000, 676 and 498 at 1,000,000; d = 2 and 5 cross between
+// 200,000 and 262,144 too.
 static inline int scan_blocks(int n, bool wide) {
     const int tile = kBlock * (wide ? kScanItems : kScanNarrow);
     return n > 0 ? (n + tile - 1) / tile : 1;

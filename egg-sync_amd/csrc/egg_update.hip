@@ -846,13 +846,16 @@ struct DenseLds {
 //   Streamed ranges are noted and summed together on the matrix cores (Stream), from
 // one place in the code: the loop over the cells returns to its head for it.
 // Bound by the VALU: per cell some 250 instructions of tests, per 8 sources 37 beside
-// the matrix instructions.  Held to three wavefronts a SIMD (162 registers): with four
-// the spills cost more than the fourth hides (100 ms against 81 in one state of it).
+// the matrix instructions.  Up to d = 3 held to three wavefronts a SIMD (165 registers
+// at d = 3, and 171 spilled scalar ones): with four the spills cost more than the
+// fourth hides (100 ms against 81 in one state of it).  At d = 4 and 5 a workgroup's
+// 60 and 74 KB of LDS leave a CU two of them, two wavefronts a SIMD (193 and 207
+// registers).
 // Against k_update_tile (which had the sums alone on the matrix cores), whole solve,
 // n = 1,000,000, d = 3, eps = 0.02: 88 -> 70 ms; one pass of n = 100,003, d = 3: 4.0 ->
 // 3.4 ms; n = 100,000, d = 2: 5.1 -> 3.9; d = 5 passes of a batch 116 -> 75 us.
 template <int D>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(D <= 3 ? 3 : 3)))
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(D <= 3 ? 3 : 2)))
 void k_update_dense(GridBufs b, int *__restrict__ rdbg, Geo g, DevState *st) {
     if (st->done) return;
     __shared__ DenseLds<D> s_lds[kBlock / kWave];
