@@ -43,8 +43,8 @@ ITERS_PER_SYNC = 4
 # pass's MFMA instructions too; those alone are UPDATE_MFMA_INSTS_N1M).
 # Measured for this workload only, so reported only when n is 1,000,000.
 UPDATE_PROFILE = "profiles/update_pass_config1_n1M_counters.md"
-UPDATE_TRAFFIC_BYTES_N1M = 89.9e6
-UPDATE_VALU_INSTS_N1M = 2.92e9
+UPDATE_TRAFFIC_BYTES_N1M = 89.4e6
+UPDATE_VALU_INSTS_N1M = 2.93e9
 UPDATE_MFMA_INSTS_N1M = 4.78e8
 
 

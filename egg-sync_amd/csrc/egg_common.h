@@ -157,7 +157,7 @@ struct DevState {
     float lam;
     int pair_count;    // extra check: (p, q) pairs found this iteration
     int T;             // tiles of every cell group (<= 64 runs of one group each): extra check
-    int TU;            // tiles of the groups k_update_tile updates (sparse groups excluded)
+    int TU;            // tiles of the groups updated by tiles (sparse groups excluded)
     int tile_next;     // work-queue head of the update kernel
     int xtile_next;    // work-queue head of the extra check
     int runs;          // runs of equal positions in the sorted order

@@ -661,7 +661,7 @@ __device__ __forceinline__ void sum_partials(int n, const SumGroups &q, int grp,
 }
 
 // Per cell group: its tiles of 64 runs (every group: the extra check's table),
-// the same for the groups k_update_tile updates (none for sparse groups), and
+// the same for the groups updated by tiles (none for sparse groups), and
 // the runs of sparse groups (k_update_pairs), listed at the offsets of their
 // scan.  cell_groups: every cell is its own group.
 struct GroupScan {

@@ -84,7 +84,7 @@ struct GridBufs {
     // cells); a tile holds <= 64 runs of one group
     int *grp_cell;       // [n+1] first cell of each group, grp_cell[G] = C
     int *tile_off;       // [n] first tile of each group (every group: extra check)
-    int *utile_off;      // [n] the same for the groups of k_update_tile (not sparse)
+    int *utile_off;      // [n] the same for the groups updated by tiles (not sparse)
     float *rres;         // [d][n] new position of each run
     int *sparse_runs;    // [n]   runs of sparse cell groups
     // pair update (egg_pairs.hip): memory of its own (pair_scratch_bytes); it

@@ -730,7 +730,8 @@ int setup_single(const float *d_D, int64_t n64, int d, float eps, const int32_t 
 // iterations of all streams are captured once, forked from and joined to one
 // origin stream, and the graph is replayed.
 
-// Kernel nodes of one captured loop iteration (an upper bound) and the
+// Kernel nodes a captured loop iteration is counted as (15 where the sort compares
+// every pair, 16 and three per 8 key bits with the radix sort: 64 at 128 bits) and the
 // largest batched graph that is captured.
 constexpr int kGraphNodesPerIter = 64;
 constexpr long long kMaxBatchGraphNodes = 65536;
