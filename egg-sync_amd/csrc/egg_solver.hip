@@ -730,11 +730,17 @@ int setup_single(const float *d_D, int64_t n64, int d, float eps, const int32_t 
 // iterations of all streams are captured once, forked from and joined to one
 // origin stream, and the graph is replayed.
 
-// Kernel nodes a captured loop iteration is counted as (15 where the sort compares
-// every pair, 16 and three per 8 key bits with the radix sort: 64 at 128 bits) and the
-// largest batched graph that is captured.
+// Kernel nodes a captured loop iteration is counted as, never fewer than it has, and the
+// largest batched graph that is captured.  An iteration has 15 where the sort compares
+// every pair and three more per 8 key bits with the radix sort: 63 at 128 bits, 111 at
+// 256.  Up to 128 bits all count as kGraphNodesPerIter.
 constexpr int kGraphNodesPerIter = 64;
 constexpr long long kMaxBatchGraphNodes = 65536;
+
+int graph_nodes_per_iter(const Geo &g) {
+    if (g.n <= kRankSortMax) return kGraphNodesPerIter;
+    return std::max(kGraphNodesPerIter, 15 + 3 * ((g.sort_bits + 7) / 8));
+}
 
 struct BatchWs {
     void *base = nullptr;
@@ -947,7 +953,10 @@ int solve_batch_impl(const float *d_D, const egg_sync_instance *inst, int n_inst
     int graph_live = 0;
     auto ensure_graph = [&](int n_live) -> int {
         if (!opt.use_graph) return 0;
-        if ((long long)n_live * K * kGraphNodesPerIter > kMaxBatchGraphNodes) {
+        long long nodes = 0;
+        for (int k : active)
+            if (live[k]) nodes += (long long)K * graph_nodes_per_iter(G[k]);
+        if (nodes > kMaxBatchGraphNodes) {
             drop_graph(bw.gexec, bw.gkey);
             graph_live = 0;
             return 0;

@@ -144,6 +144,24 @@ def _passes_match_oracle_along_gpu_trajectory(S, O, X, e, iters):
         prev = cur
 
 
+def test_batch_graph_with_wide_keys(S):
+    """64 instances x 16 iterations whose radix sorts take 22 passes (175 key
+    bits): counted as 81 kernels an iteration, 82,944 in all, past the largest
+    batched graph, so it launches plainly and gives what one instance gives."""
+    rng = np.random.default_rng(5)
+    n, d, eps = 24577, 20, 0.1
+    X = rng.random((n // 2 + 1, d))
+    X = np.repeat(X, 2, axis=0)[:n] + 0.002 * rng.random((n, d))
+    X = np.clip(X, 0, 1).astype(np.float32)
+    one = S.solve(X, eps, max_iter=3)
+    D, specs = S.pack_instances([X], [[eps] * 64])
+    r = S.solve_batch(D, specs, streams=4, use_graph=True, iters_per_sync=16, max_iter=3)
+    for k in range(64):
+        assert r["results"][k]["iterations"] == one["stats"]["iterations"], k
+        assert np.array_equal(r["labels"][k], one["labels"]), k
+        assert np.array_equal(r["X"][k].view(np.uint32), one["X"].view(np.uint32)), k
+
+
 def test_batch_config3_sample_against_oracle(S, O):
     """Iterations and partitions equal the oracle's.  Final positions agree to
     1e-5 unless the trajectory is sensitive to last-bit differences: a pair at
